@@ -51,7 +51,7 @@ __device__ __forceinline__ int64_t csr_find(const uint32_t* idx, int64_t a, int6
 template <bool SPARSE>
 __global__ __launch_bounds__(kRankThreads) void wta_hash_kernel(
     const uint32_t* __restrict__ windows, int k, int L, int ws, int bits,
-    const float* __restrict__ x, int64_t ldx, const int64_t* __restrict__ xoff,
+    const float* __restrict__ x, int64_t ldx, const int64_t* __restrict__ xoff, int xstep,
     const uint32_t* __restrict__ xidx, const float* __restrict__ xval, int64_t batch,
     uint32_t* __restrict__ codes) {
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kRankThreads) void wta_hash_kernel(
     int best = 0;
     float bv = -INFINITY;
     for (int p = 0; p < ws; ++p) {
-      const float v = SPARSE ? csr_value(xidx, xval, xoff[row], xoff[row + 1], win[p])
+      const float v = SPARSE ? csr_value(xidx, xval, xoff[row * xstep], xoff[row * xstep + 1], win[p])
                              : x[row * ldx + win[p]];
       if (v > bv) {
         bv = v;
@@ -79,13 +79,13 @@ __global__ __launch_bounds__(kRankThreads) void wta_hash_kernel(
 // DWTA over CSR rows (dwta.rs:108-166).
 __global__ __launch_bounds__(kRankThreads) void dwta_sparse_kernel(
     const uint32_t* __restrict__ windows, const uint32_t* __restrict__ fallback, int k, int L,
-    int ws, int bits, const int64_t* __restrict__ xoff, const uint32_t* __restrict__ xidx,
+    int ws, int bits, const int64_t* __restrict__ xoff, int xstep, const uint32_t* __restrict__ xidx,
     const float* __restrict__ xval, int64_t batch, uint32_t* __restrict__ codes) {
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (q >= batch * L) return;
   const int64_t row = q / L;
   const int t = static_cast<int>(q % L);
-  const int64_t a = xoff[row], b = xoff[row + 1];
+  const int64_t a = xoff[row * xstep], b = xoff[row * xstep + 1];
   uint64_t h = 0;
   for (int f = 0; f < k; ++f) {
     const uint32_t* win = windows + (static_cast<size_t>(t) * k + f) * ws;
@@ -118,7 +118,7 @@ constexpr int64_t kMhMaxRows = 1 << 22;  // rows (blocks) per launch
 template <bool SPARSE>
 __global__ __launch_bounds__(kMhThreads) void minhash_rows_kernel(
     const uint32_t* __restrict__ perms, int dim, int k, int L, const float* __restrict__ x,
-    int64_t ldx, const int64_t* __restrict__ xoff, const uint32_t* __restrict__ xidx,
+    int64_t ldx, const int64_t* __restrict__ xoff, int xstep, const uint32_t* __restrict__ xidx,
     uint32_t* __restrict__ codes) {
   extern __shared__ uint32_t nzd[];  // dense: the row's nonzero dimensions (any order)
   __shared__ uint32_t wmin[kMhWaves][kMaxMinHashBins];
@@ -128,9 +128,9 @@ __global__ __launch_bounds__(kMhThreads) void minhash_rows_kernel(
   const uint32_t* list;
   int64_t nnz;
   if constexpr (SPARSE) {
-    const int64_t a = xoff[row];
+    const int64_t a = xoff[row * xstep];
     list = xidx + a;
-    nnz = xoff[row + 1] - a;
+    nnz = xoff[row * xstep + 1] - a;
   } else {
     if (threadIdx.x == 0) nnz_s = 0;
     __syncthreads();
@@ -258,7 +258,7 @@ int rank_hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx,
     for (int64_t b0 = 0; b0 < batch; b0 += kMhMaxRows) {
       hipLaunchKernelGGL(minhash_rows_kernel<false>, dim3(static_cast<unsigned>(std::min(batch - b0, kMhMaxRows))),
                          dim3(kMhThreads), sizeof(uint32_t) * h->dim, st, h->perms_dev, h->dim, h->k, h->L,
-                         x + b0 * ldx, ldx, nullptr, nullptr, codes + b0 * h->L);
+                         x + b0 * ldx, ldx, nullptr, 1, nullptr, codes + b0 * h->L);
       KH_LAUNCHED();
     }
     return KH_OK;
@@ -267,31 +267,31 @@ int rank_hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx,
                        h->k, h->L, x, ldx, batch, codes);
   else  // WTA and DWTA hash dense rows alike (dwta.rs:143-152)
     hipLaunchKernelGGL(wta_hash_kernel<false>, dim3(blocks), dim3(kRankThreads), 0, st,
-                       h->windows_dev, h->k, h->L, h->ws, h->bits, x, ldx, nullptr, nullptr, nullptr,
+                       h->windows_dev, h->k, h->L, h->ws, h->bits, x, ldx, nullptr, 1, nullptr, nullptr,
                        batch, codes);
   KH_LAUNCHED();
   return KH_OK;
 }
 
 int rank_hash_sparse_launch(const kh_hash_family* h, const int64_t* xoff, const uint32_t* xidx,
-                            const float* xval, int64_t batch, uint32_t* codes, hipStream_t st) {
+                            const float* xval, int64_t batch, uint32_t* codes, hipStream_t st, int xstep) {
   if (batch == 0) return KH_OK;
   const int64_t n = batch * h->L;
   const unsigned blocks = static_cast<unsigned>((n + kRankThreads - 1) / kRankThreads);
   if (h->kind == KH_FAMILY_MINHASH) {
     for (int64_t b0 = 0; b0 < batch; b0 += kMhMaxRows) {
       hipLaunchKernelGGL(minhash_rows_kernel<true>, dim3(static_cast<unsigned>(std::min(batch - b0, kMhMaxRows))),
-                         dim3(kMhThreads), 0, st, h->perms_dev, h->dim, h->k, h->L, nullptr, 0, xoff + b0,
-                         xidx, codes + b0 * h->L);
+                         dim3(kMhThreads), 0, st, h->perms_dev, h->dim, h->k, h->L, nullptr, 0, xoff + b0 * xstep,
+                         xstep, xidx, codes + b0 * h->L);
       KH_LAUNCHED();
     }
     return KH_OK;
   } else if (h->kind == KH_FAMILY_DWTA)
     hipLaunchKernelGGL(dwta_sparse_kernel, dim3(blocks), dim3(kRankThreads), 0, st, h->windows_dev,
-                       h->fallback_dev, h->k, h->L, h->ws, h->bits, xoff, xidx, xval, batch, codes);
+                       h->fallback_dev, h->k, h->L, h->ws, h->bits, xoff, xstep, xidx, xval, batch, codes);
   else
     hipLaunchKernelGGL(wta_hash_kernel<true>, dim3(blocks), dim3(kRankThreads), 0, st, h->windows_dev,
-                       h->k, h->L, h->ws, h->bits, nullptr, 0, xoff, xidx, xval, batch, codes);
+                       h->k, h->L, h->ws, h->bits, nullptr, 0, xoff, xstep, xidx, xval, batch, codes);
   KH_LAUNCHED();
   return KH_OK;
 }

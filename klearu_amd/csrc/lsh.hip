@@ -458,13 +458,13 @@ __global__ __launch_bounds__(256) void hash_dense_mfma_kernel(
 constexpr int kHashSparseBatch = 16;
 __global__ __launch_bounds__(kHashThreads) void hash_sparse_kernel(
     const int8_t* __restrict__ planes, int k, int L, int dim, const int64_t* __restrict__ xoff,
-    const uint32_t* __restrict__ xidx, const float* __restrict__ xval,
+    int xstep, const uint32_t* __restrict__ xidx, const float* __restrict__ xval,
     uint32_t* __restrict__ codes) {
   __shared__ uint32_t cw[kHashThreads];
   const int64_t row = blockIdx.x;
   const int tpb = kHashThreads / k;           // tables per block
   const int t0 = blockIdx.y * tpb, t1 = min(L, t0 + tpb);
-  const int64_t a = xoff[row], b = xoff[row + 1];
+  const int64_t a = xoff[row * xstep], b = xoff[row * xstep + 1];
   for (int t = threadIdx.x; t < t1 - t0; t += blockDim.x) cw[t] = 0u;
   __syncthreads();
   const int p = t0 * k + threadIdx.x;
@@ -1014,13 +1014,14 @@ int hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx, int6
 }
 
 int hash_sparse_launch(const kh_hash_family* h, const int64_t* xoff, const uint32_t* xidx,
-                       const float* xval, int64_t batch, uint32_t* codes, hipStream_t st) {
+                       const float* xval, int64_t batch, uint32_t* codes, hipStream_t st, int xstep) {
   if (batch == 0) return KH_OK;
-  if (h->kind != KH_FAMILY_TERNARY) return rank_hash_sparse_launch(h, xoff, xidx, xval, batch, codes, st);
+  if (h->kind != KH_FAMILY_TERNARY)
+    return rank_hash_sparse_launch(h, xoff, xidx, xval, batch, codes, st, xstep);
   KH_CHECK_ARG(h->L <= 256, "hash_sparse supports at most 256 tables");
   const int tpb = kHashThreads / h->k;
   hipLaunchKernelGGL(hash_sparse_kernel, dim3((unsigned)batch, ceil_div(h->L, tpb)), dim3(kHashThreads),
-                     0, st, h->planes_dev, h->k, h->L, h->dim, xoff, xidx, xval, codes);
+                     0, st, h->planes_dev, h->k, h->L, h->dim, xoff, xstep, xidx, xval, codes);
   KH_LAUNCHED();
   return KH_OK;
 }

@@ -63,8 +63,10 @@ namespace kh {
 
 int hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx, int64_t batch,
                       uint32_t* codes, hipStream_t st);
+// Row r holds entries xoff[r * xstep] .. xoff[r * xstep + 1]: CSR offsets with
+// xstep 1, one (start, end) pair per row with xstep 2.
 int hash_sparse_launch(const kh_hash_family* h, const int64_t* xoff, const uint32_t* xidx,
-                       const float* xval, int64_t batch, uint32_t* codes, hipStream_t st);
+                       const float* xval, int64_t batch, uint32_t* codes, hipStream_t st, int xstep = 1);
 // Per-row unique ids (ascending) and hit counts into [batch][stride] buffers.
 int query_launch(const kh_lsh_index* idx, const uint32_t* qcodes, int64_t batch, uint32_t* qids,
                  uint32_t* qcnt, int stride, int32_t* ulen, hipStream_t st);
@@ -73,7 +75,7 @@ int query_stride(const kh_lsh_index* idx);
 int rank_hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx, int64_t batch,
                            uint32_t* codes, hipStream_t st);
 int rank_hash_sparse_launch(const kh_hash_family* h, const int64_t* xoff, const uint32_t* xidx,
-                            const float* xval, int64_t batch, uint32_t* codes, hipStream_t st);
+                            const float* xval, int64_t batch, uint32_t* codes, hipStream_t st, int xstep);
 // Row lengths -> CSR offsets, copies of up to four per-row arrays, then a
 // synchronising capacity check.
 int csr_finish(const uint32_t* qids, const uint32_t* qcnt, const float* f1, const float* f2,
