@@ -7,29 +7,33 @@
 // (crates/klearu-dejavu/src/attention.rs:18-74).
 //
 // Every output is bit-identical to the reference: each one is a sequential f32
-// sum of rounded products in the reference's order, owned by one thread.
-//   Linear rows     one thread per (token, output row): -0.0 + w[r][0]*x[0] + ...
-//                   then + bias[r].  Weights are stored transposed, WT[in][out],
-//                   so the threads of a wave read adjacent floats of one WT row
-//                   at every step while the input value is shared.
-//   SparseMlp       gate and up chains of a selected neuron in one thread,
-//                   h = silu(g) * u; then one thread per (token, output j) adds
-//                   WT_down[sel[a]][j] * h[a] for every selected a with h != 0,
-//                   in selection order from +0.0, then the bias.
-//   SparseAttention q/k/v rows of the selected heads scattered into zeroed
-//                   [heads*head_dim] vectors, one thread per (token, selected
-//                   head) for the sigmoid score and the scaled v, then o_proj
-//                   over the whole (zero-filled) vector like Linear::forward.
+// sum of rounded products in the reference's order, added by one lane.
+//   Linear rows     per (token, output row): -0.0 + w[r][0]*x[0] + ... then
+//                   + bias[r].
+//   SparseMlp       gate and up rows of a selected neuron, h = silu(g) * u; then
+//                   per (token, output j) W_down[j][sel[a]] * h[a] added for every
+//                   selected a with h != 0, in selection order from +0.0, then the
+//                   bias.
+//   SparseAttention q/k/v rows of the selected heads into [heads*head_dim]
+//                   vectors, a wave per (token, head) for the sigmoid score and
+//                   the scaled v (zero for other heads), then o_proj over the
+//                   whole (zero-filled) vector like Linear::forward.
+// A handle keeps its weights twice: row-major [out][in], which the selected rows
+// of a gather read in whole pieces, and transposed [in][out], which the columns
+// of SparseMlp's down projection and the wide form below read.
 // Index lists arrive from the host (the reference's &[usize]), are checked
 // there (an out-of-range index is the reference's panic) and are uploaded to
 // the handle's scratch; the upload is waited for, so the caller's list may be
 // freed on return and the kernels stay queued behind it.
+#include <algorithm>
 #include <vector>
 
-#include "common.hpp"
+#include "chain_add.hpp"
+#include "gather.hpp"
 
 struct kh_dejavu_linear {
   int in_f = 0, out_f = 0;
+  float* w = nullptr;     // [out_f][in_f]
   float* wt = nullptr;    // [in_f][out_f]
   float* bias = nullptr;  // [out_f]
   mutable kh::StreamWs ws;  // forward_sparse row list, per stream
@@ -49,76 +53,284 @@ namespace kh {
 
 constexpr int kDlThreads = 256;
 
-__global__ __launch_bounds__(kDlThreads) void dl_rows_kernel(
-    const float* __restrict__ wt, int in_f, int out_f, const float* __restrict__ bias,
-    const float* __restrict__ x, int64_t ldx, int64_t batch, const int64_t* __restrict__ rows,
-    int64_t nrows, float* __restrict__ y, int64_t ldy, int scatter) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= batch * nrows) return;
-  const int64_t b = gid / nrows, a = gid - b * nrows;
-  const int64_t r = rows ? rows[a] : a;
-  const float* xb = x + b * ldx;
-  float s = -0.0f;
-  for (int j = 0; j < in_f; ++j) s = __fadd_rn(s, __fmul_rn(wt[(int64_t)j * out_f + r], xb[j]));
-  y[b * ldy + (scatter ? r : a)] = __fadd_rn(s, bias[r]);
-}
+// Few outputs: a chain of in_f dependent adds per output bounds the call (about
+// 6 cycles a step), so a block gives all else to other waves.  It owns 16 rows
+// x TB tokens, one chain per lane of wave 0 (the consumer); waves 1..8 hold the
+// weights of the next kDcAhead chunks of kDcStep steps in registers and form a
+// chunk's products in LDS while wave 0 adds the chunk before, four per read.
+// Products past the end are -0.0, which leaves every sum unchanged.  A thread per
+// output with one load in flight per add took 107 us for a 1024-square Linear of
+// 1 to 128 tokens and 212 us at 2048 (both launch-bound here up to 16 tokens, about
+// 11 us a call); SparseMlp 1024 / 2752, 30% of the neurons, 16 tokens: 668 -> 37 us,
+// 1024 tokens: 11.8 -> 1.1 ms.
+constexpr int kDcRows = 16;                    // output rows (or columns) per block
+constexpr int kDcStep = 128;                   // steps per chunk
+constexpr int kDcAhead = 4;                    // chunks in flight per producer
+constexpr int kDcProd = kDcStep / 4 * kDcRows; // producer threads: one float4 of one row each
+constexpr int kDcThreads = 64 + kDcProd;
+constexpr int kDcQuads = kDcStep / 4;
+// Quads of one chunk [step / 4][chain], each quad row padded by one float4 so
+// that the down kernel's 4-byte writes fall in distinct banks.
+template <int TB>
+struct DcLds {
+  static constexpr int kStride = kDcRows * TB + 1;
+  float4 q[2][kDcQuads * kStride];
+};
 
-__global__ __launch_bounds__(kDlThreads) void dl_gateup_kernel(
-    const float* __restrict__ wg, const float* __restrict__ bg, const float* __restrict__ wu,
-    const float* __restrict__ bu, int hidden, int inter, const float* __restrict__ x,
-    int64_t batch, const int64_t* __restrict__ sel, int64_t n, float* __restrict__ h) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= batch * n) return;
-  const int64_t b = gid / n, a = gid - b * n;
-  const int64_t r = sel[a];
-  const float* xb = x + b * hidden;
-  float g = -0.0f, u = -0.0f;
-  for (int j = 0; j < hidden; ++j) {
-    const float xj = xb[j];
-    g = __fadd_rn(g, __fmul_rn(wg[(int64_t)j * inter + r], xj));
-    u = __fadd_rn(u, __fmul_rn(wu[(int64_t)j * inter + r], xj));
+struct DcMat {
+  const float* w;     // rows kernel: [out][in]; down kernel: transposed [in][out]
+  const float* bias;
+  float* y;
+};
+struct DcRows {
+  DcMat m[3];         // blockIdx.z picks one; gate/up: m[0] gate, m[1] up
+  int in_f;
+  const float* x;     // [batch][ldx]
+  int64_t ldx, batch;
+  const int64_t* rows;  // null: every row
+  int64_t nrows, ldy;
+  int scatter;        // outputs at y[row] instead of y[position in the list]
+};
+
+// Eight producer waves and the consumer step through nch chunks: make(c, u) puts
+// chunk c's products (register slot u = c % kDcAhead) into LDS buffer c & 1 and
+// requests chunk c + kDcAhead.  The loop has no branch around a load (chunks past
+// the end are clamped, formed and not added): behind a branch the compiler waits
+// for every load in flight.
+template <int TB, typename Make>
+__device__ __forceinline__ float dc_run(DcLds<TB>& lds, int nch, float s0, Make make) {
+  const int lane = threadIdx.x & 63;
+  float s = s0;
+  if (threadIdx.x >= 64) {
+    for (int c0 = 0; c0 < nch; c0 += kDcAhead) {
+#pragma unroll
+      for (int u = 0; u < kDcAhead; ++u) {
+        make(c0 + u, u);
+        lds_barrier();
+      }
+    }
+  } else {
+    const int last = (nch + kDcAhead - 1) / kDcAhead * kDcAhead;
+    for (int c = 0; c < last; ++c) {
+      lds_barrier();
+      if (c < nch) s = chain_add_static<kDcQuads, DcLds<TB>::kStride>(&lds.q[c & 1][min(lane, kDcRows * TB - 1)], s);
+    }
   }
-  g = __fadd_rn(g, bg[r]);
-  u = __fadd_rn(u, bu[r]);
-  h[gid] = __fmul_rn(silu_ref(g), u);
+  return s;
 }
 
-__global__ __launch_bounds__(kDlThreads) void dl_down_kernel(
+// Four consecutive floats at p[k..k+3], k + i < n (others read p[n - 1]).
+template <bool VEC>
+__device__ __forceinline__ float4 dc_load4(const float* __restrict__ p, int k, int n) {
+  if constexpr (VEC) return *reinterpret_cast<const float4*>(p + min(k, n - 4));
+  return make_float4(p[min(k, n - 1)], p[min(k + 1, n - 1)], p[min(k + 2, n - 1)], p[min(k + 3, n - 1)]);
+}
+
+// GATEUP: rows 0..7 of the block are gate rows, 8..15 the same neurons' up rows.
+// VEC: in_f and ldx multiples of 4, x 16-byte aligned.
+template <bool GATEUP, int TB, bool VEC>
+__global__ __launch_bounds__(kDcThreads) void dl_chain_rows_kernel(const DcRows a) {
+  __shared__ DcLds<TB> lds;
+  constexpr int kOwn = GATEUP ? kDcRows / 2 : kDcRows;   // list entries per block
+  const int64_t a0 = (int64_t)blockIdx.x * kOwn, b0 = (int64_t)blockIdx.y * TB;
+  const int n = a.in_f, nch = (n + kDcStep - 1) / kDcStep;
+  const bool prod = threadIdx.x >= 64;
+  const int pt = (int)threadIdx.x - 64;
+  // lanes of a producer wave: 16 rows x 4 quads, so a quad row's 16 products are
+  // written as one contiguous piece per token
+  const int i = prod ? pt & (kDcRows - 1) : (int)threadIdx.x & (kDcRows - 1);
+  const int k4 = pt >> 4;
+  const DcMat& mat = a.m[GATEUP ? i / kOwn : (int)blockIdx.z];
+  const int64_t at = min(a0 + (GATEUP ? i % kOwn : i), a.nrows - 1);
+  const int64_t r = a.rows ? a.rows[at] : at;
+  const float* __restrict__ wr = mat.w + r * n;
+  const float* __restrict__ xr[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) xr[t] = a.x + min(b0 + t, a.batch - 1) * a.ldx;
+  float4 w[kDcAhead], x[kDcAhead][TB];
+  auto fetch = [&](int c, int u) {
+    const int k = c * kDcStep + 4 * k4;
+    w[u] = dc_load4<VEC>(wr, k, n);
+#pragma unroll
+    for (int t = 0; t < TB; ++t) x[u][t] = dc_load4<VEC>(xr[t], k, n);
+  };
+  if (prod) {
+#pragma unroll
+    for (int u = 0; u < kDcAhead; ++u) fetch(u, u);
+  }
+  float s = dc_run<TB>(lds, nch, -0.0f, [&](int c, int u) {
+    const int k = c * kDcStep + 4 * k4;
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+      float4 p;
+      p.x = k < n ? w[u].x * x[u][t].x : -0.0f;
+      p.y = k + 1 < n ? w[u].y * x[u][t].y : -0.0f;
+      p.z = k + 2 < n ? w[u].z * x[u][t].z : -0.0f;
+      p.w = k + 3 < n ? w[u].w * x[u][t].w : -0.0f;
+      lds.q[c & 1][k4 * DcLds<TB>::kStride + t * kDcRows + i] = p;
+    }
+    fetch(c + kDcAhead, u);
+  });
+  if (threadIdx.x >= 64) return;
+  const int64_t b = b0 + ((int)threadIdx.x >> 4);
+  const bool live = (int)threadIdx.x < kDcRows * TB && b < a.batch;
+  s = __fadd_rn(s, mat.bias[r]);
+  if constexpr (GATEUP) {
+    const float up = __shfl(s, (int)threadIdx.x + kOwn);
+    if (live && i < kOwn && a0 + i < a.nrows) a.m[0].y[b * a.ldy + at] = __fmul_rn(silu_ref(s), up);
+  } else {
+    if (live && a0 + i < a.nrows) mat.y[b * a.ldy + (a.scatter ? r : at)] = s;
+  }
+}
+
+// SparseMlp's down projection: chains over the selected neurons; a block owns 16
+// output columns.  A producer thread takes one neuron's float4 of columns.
+// VEC: hidden a multiple of 4.
+template <int TB, bool VEC>
+__global__ __launch_bounds__(kDcThreads) void dl_chain_down_kernel(
     const float* __restrict__ wdt, const float* __restrict__ bd, int hidden,
-    const float* __restrict__ h, int64_t batch, const int64_t* __restrict__ sel, int64_t n,
+    const float* __restrict__ h, int64_t batch, const int64_t* __restrict__ sel, int n,
     float* __restrict__ y) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= batch * hidden) return;
-  const int64_t b = gid / hidden;
-  const int j = (int)(gid - b * hidden);
-  const float* hb = h + b * n;
-  float s = 0.0f;
-  for (int64_t a = 0; a < n; ++a) {
-    const float v = hb[a];
-    if (v != 0.0f) s = __fadd_rn(s, __fmul_rn(wdt[sel[a] * hidden + j], v));
+  __shared__ DcLds<TB> lds;
+  const int j0 = blockIdx.x * kDcRows;
+  const int64_t b0 = (int64_t)blockIdx.y * TB;
+  const int nch = (n + kDcStep - 1) / kDcStep;
+  const bool prod = threadIdx.x >= 64;
+  const int pt = (int)threadIdx.x - 64;
+  const int q = pt & 3, e = pt >> 2;          // column quad, step within the chunk
+  const float* __restrict__ hr[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) hr[t] = h + min(b0 + t, batch - 1) * n;
+  int id[kDcAhead];                           // neuron of the chunk kDcAhead past the slot's
+  float4 w[kDcAhead];
+  float v[kDcAhead][TB];
+  auto ids = [&](int c, int u) { id[u] = (int)sel[min(c * kDcStep + e, n - 1)]; };
+  auto fetch = [&](int c, int u) {
+    w[u] = dc_load4<VEC>(wdt + (size_t)id[u] * hidden, j0 + 4 * q, hidden);
+#pragma unroll
+    for (int t = 0; t < TB; ++t) v[u][t] = hr[t][min(c * kDcStep + e, n - 1)];
+  };
+  if (prod && nch > 0) {
+#pragma unroll
+    for (int u = 0; u < kDcAhead; ++u) ids(u, u);
+#pragma unroll
+    for (int u = 0; u < kDcAhead; ++u) fetch(u, u);
+#pragma unroll
+    for (int u = 0; u < kDcAhead; ++u) ids(u + kDcAhead, u);
   }
-  y[gid] = __fadd_rn(s, bd[j]);
+  float s = dc_run<TB>(lds, nch, 0.0f, [&](int c, int u) {
+    float* dst = reinterpret_cast<float*>(&lds.q[c & 1][(e >> 2) * DcLds<TB>::kStride]) + (e & 3);
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+      // a zero activation adds nothing, whatever the weight
+      const bool on = c * kDcStep + e < n && v[u][t] != 0.0f;
+      float* d = dst + 4 * (t * kDcRows + 4 * q);
+      d[0] = on ? w[u].x * v[u][t] : -0.0f;
+      d[4] = on ? w[u].y * v[u][t] : -0.0f;
+      d[8] = on ? w[u].z * v[u][t] : -0.0f;
+      d[12] = on ? w[u].w * v[u][t] : -0.0f;
+    }
+    fetch(c + kDcAhead, u);
+    ids(c + 2 * kDcAhead, u);
+  });
+  const int lane = threadIdx.x;
+  if (lane >= kDcRows * TB) return;
+  const int j = j0 + (lane & (kDcRows - 1));
+  const int64_t b = b0 + (lane >> 4);
+  if (b < batch && j < hidden) y[b * hidden + j] = __fadd_rn(s, bd[j]);
 }
 
-__global__ void dl_fill_kernel(float* __restrict__ p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0f;
+// Many outputs (kDlWide of them or more): one thread per output row and TB
+// tokens.  A group of kDlAhead coalesced loads of the transposed weights is in
+// flight while the group before is added; the tokens' inputs are the same for
+// every lane (scalar loads).  No LDS traffic is spent on products, and the TB
+// chains of a thread hide each other's adds.
+constexpr int kDlAhead = 16;
+template <int TB>
+__global__ __launch_bounds__(64) void dl_wide_rows_kernel(const DcRows a, int out_f) {
+  const int64_t at = min((int64_t)blockIdx.x * 64 + threadIdx.x, a.nrows - 1);
+  const int64_t r = a.rows ? a.rows[at] : at;
+  const int64_t b0 = (int64_t)blockIdx.y * TB;
+  const DcMat& mat = a.m[blockIdx.z];
+  const float* __restrict__ wt = mat.w + r;
+  const float* __restrict__ xr[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) xr[t] = a.x + min(b0 + t, a.batch - 1) * a.ldx;
+  float s[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) s[t] = -0.0f;
+  const int n = a.in_f, full = n / kDlAhead * kDlAhead;
+  float w0[kDlAhead], w1[kDlAhead];
+  auto load = [&](float (&w)[kDlAhead], int j) {
+#pragma unroll
+    for (int u = 0; u < kDlAhead; ++u) w[u] = wt[(int64_t)min(j + u, n - 1) * out_f];
+  };
+  auto add = [&](const float (&w)[kDlAhead], int j) {
+#pragma unroll
+    for (int u = 0; u < kDlAhead; ++u)
+#pragma unroll
+      for (int t = 0; t < TB; ++t) s[t] = __fadd_rn(s[t], __fmul_rn(w[u], xr[t][j + u]));
+  };
+  load(w0, 0);
+  int j = 0;
+  for (; j + 2 * kDlAhead <= full; j += 2 * kDlAhead) {
+    load(w1, j + kDlAhead);
+    __builtin_amdgcn_sched_barrier(0);
+    add(w0, j);
+    load(w0, j + 2 * kDlAhead);
+    __builtin_amdgcn_sched_barrier(0);
+    add(w1, j + kDlAhead);
+  }
+  if (j < full) {
+    add(w0, j);
+    j += kDlAhead;
+  }
+  for (; j < n; ++j) {
+    const float w = wt[(int64_t)j * out_f];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) s[t] = __fadd_rn(s[t], __fmul_rn(w, xr[t][j]));
+  }
+  if ((int64_t)blockIdx.x * 64 + threadIdx.x >= a.nrows) return;
+  const float bi = mat.bias[r];
+#pragma unroll
+  for (int t = 0; t < TB; ++t)
+    if (b0 + t < a.batch) mat.y[(b0 + t) * a.ldy + (a.scatter ? r : at)] = __fadd_rn(s[t], bi);
 }
 
-// q, k, v, att: [batch][qd]; one thread per (token, selected head).
-__global__ __launch_bounds__(kDlThreads) void dl_head_score_kernel(
+// One wave per (head, token): the score's products in LDS, added by one lane in
+// order, then the scaled v; zeros for a head that is not selected (att rows are
+// whole).  q, k, v, att: [batch][qd].
+constexpr int kDlHeadTile = 64;
+__global__ __launch_bounds__(64) void dl_head_score_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    float* __restrict__ att, int64_t qd, int head_dim, int64_t batch,
-    const int64_t* __restrict__ heads, int64_t n_heads, float scale) {
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= batch * n_heads) return;
-  const int64_t b = gid / n_heads, a = gid - b * n_heads;
-  const int64_t st = b * qd + heads[a] * head_dim;
+    float* __restrict__ att, int64_t qd, int head_dim, const int64_t* __restrict__ heads,
+    int64_t n_heads, float scale) {
+  __shared__ float4 p4[kDlHeadTile / 4];
+  float* p = reinterpret_cast<float*>(p4);
+  const int lane = threadIdx.x;
+  const int64_t head = blockIdx.x;
+  const int64_t st = (int64_t)blockIdx.y * qd + head * head_dim;
+  bool on = false;
+  for (int64_t i = lane; i < n_heads; i += 64) on = on || heads[i] == head;
+  if (__ballot(on) == 0ull) {
+    for (int d = lane; d < head_dim; d += 64) att[st + d] = 0.0f;
+    return;
+  }
   float s = -0.0f;
-  for (int d = 0; d < head_dim; ++d) s = __fadd_rn(s, __fmul_rn(q[st + d], k[st + d]));
-  s = __fdiv_rn(s, scale);
-  const float sc = sigmoid_ref(s);
-  for (int d = 0; d < head_dim; ++d) att[st + d] = __fmul_rn(v[st + d], sc);
+  for (int d0 = 0; d0 < head_dim; d0 += kDlHeadTile) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kDlHeadTile / 64; ++u) {
+      const int d = d0 + u * 64 + lane;
+      const int64_t at = st + min(d, head_dim - 1);
+      const float pr = __fmul_rn(q[at], k[at]);
+      p[u * 64 + lane] = d < head_dim ? pr : -0.0f;
+    }
+    __syncthreads();
+    s = chain_add_static<kDlHeadTile / 4, 1>(p4, s);   // every lane: the same sum
+  }
+  const float sc = sigmoid_ref(__fdiv_rn(s, scale));
+  for (int d = lane; d < head_dim; d += 64) att[st + d] = __fmul_rn(v[st + d], sc);
 }
 
 static unsigned grid_for(int64_t threads) {
@@ -143,22 +355,98 @@ static int upload_indices(WsSet* w, const int64_t* idx_host, int64_t n, int64_t 
   return KH_OK;
 }
 
-static int rows_launch(const kh_dejavu_linear* l, const float* x, int64_t ldx, int64_t batch,
-                       const int64_t* rows, int64_t nrows, float* y, int64_t ldy, int scatter,
-                       hipStream_t st) {
-  if (batch * nrows == 0) return KH_OK;
-  hipLaunchKernelGGL(dl_rows_kernel, dim3(grid_for(batch * nrows)), dim3(kDlThreads), 0, st,
-                     l->wt, l->in_f, l->out_f, l->bias, x, ldx, batch, rows, nrows, y, ldy,
-                     scatter);
-  KH_LAUNCHED();
+// Outputs from which the thread-per-output form is taken.  A square Linear of
+// 1024 (chain kernel, wide form; us per call): 64 tokens 28.2, 30.1; 128 tokens
+// 54.9, 30.3; of 2048: 32 tokens 45, 57; 64 tokens 89, 57.
+constexpr int64_t kDlWide = 3 << 15;
+// Waves of one token each below which a thread takes two tokens rather than four
+// (1024: 256 tokens 35.4 with two, 38.2 with four; 1024 tokens 96.9, 69.5).
+constexpr int64_t kDlWideSplit = 6144;
+
+template <bool GATEUP, int TB>
+static void chain_rows_go(const DcRows& a, bool vec, int mats, hipStream_t st) {
+  const int own = GATEUP ? kDcRows / 2 : kDcRows;
+  const dim3 g((unsigned)ceil_div(a.nrows, own), (unsigned)ceil_div(a.batch, TB), (unsigned)mats);
+  if (vec)
+    hipLaunchKernelGGL((dl_chain_rows_kernel<GATEUP, TB, true>), g, dim3(kDcThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((dl_chain_rows_kernel<GATEUP, TB, false>), g, dim3(kDcThreads), 0, st, a);
+}
+
+// Tokens per block: no more than the batch needs (a token's chains cost LDS).
+template <bool GATEUP>
+static int chain_rows(DcRows a, int mats, hipStream_t st) {
+  const bool vec = a.in_f % 4 == 0 && a.ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
+  constexpr int64_t kMaxTokens = 65535;   // grid.y blocks of at least one token
+  const float* x = a.x;
+  const int64_t batch = a.batch;
+  float* y[3] = {a.m[0].y, a.m[1].y, a.m[2].y};
+  for (int64_t b0 = 0; b0 < batch; b0 += kMaxTokens) {
+    a.batch = std::min(batch - b0, kMaxTokens);
+    a.x = x + b0 * a.ldx;
+    for (int i = 0; i < 3; ++i) a.m[i].y = y[i] ? y[i] + b0 * a.ldy : nullptr;
+    if (a.batch == 1) chain_rows_go<GATEUP, 1>(a, vec, mats, st);
+    else if (a.batch == 2) chain_rows_go<GATEUP, 2>(a, vec, mats, st);
+    else chain_rows_go<GATEUP, 4>(a, vec, mats, st);
+    KH_LAUNCHED();
+  }
   return KH_OK;
 }
 
-static int fill_zero(float* p, int64_t n, hipStream_t st) {
-  if (n == 0) return KH_OK;
-  hipLaunchKernelGGL(dl_fill_kernel, dim3(grid_for(n)), dim3(kDlThreads), 0, st, p, n);
-  KH_LAUNCHED();
+static int wide_rows(DcRows a, int out_f, int mats, hipStream_t st) {
+  constexpr int64_t kMaxTokens = 65535 * 4;
+  const float* x = a.x;
+  const int64_t batch = a.batch;
+  float* y[3] = {a.m[0].y, a.m[1].y, a.m[2].y};
+  for (int64_t b0 = 0; b0 < batch; b0 += kMaxTokens) {
+    a.batch = std::min(batch - b0, kMaxTokens);
+    a.x = x + b0 * a.ldx;
+    for (int i = 0; i < 3; ++i) a.m[i].y = y[i] ? y[i] + b0 * a.ldy : nullptr;
+    const unsigned gx = (unsigned)ceil_div(a.nrows, 64);
+    if (a.batch == 1)
+      hipLaunchKernelGGL(dl_wide_rows_kernel<1>, dim3(gx, 1, (unsigned)mats), dim3(64), 0, st, a, out_f);
+    else if (a.batch < 4 || (int64_t)gx * a.batch * mats < kDlWideSplit)
+      hipLaunchKernelGGL(dl_wide_rows_kernel<2>, dim3(gx, (unsigned)ceil_div(a.batch, 2), (unsigned)mats), dim3(64), 0,
+                         st, a, out_f);
+    else
+      hipLaunchKernelGGL(dl_wide_rows_kernel<4>, dim3(gx, (unsigned)ceil_div(a.batch, 4), (unsigned)mats), dim3(64), 0,
+                         st, a, out_f);
+    KH_LAUNCHED();
+  }
   return KH_OK;
+}
+
+// `mats` projections of one shape (bias, outputs y[i]) of the same inputs.
+static int rows_launch(const kh_dejavu_linear* const* l, int mats, const float* x, int64_t ldx,
+                       int64_t batch, const int64_t* rows, int64_t nrows, float* const* y,
+                       int64_t ldy, int scatter, hipStream_t st) {
+  if (batch * nrows == 0) return KH_OK;
+  const bool wide = batch * nrows >= kDlWide;
+  DcRows a{};
+  for (int i = 0; i < mats; ++i) a.m[i] = {wide ? l[i]->wt : l[i]->w, l[i]->bias, y[i]};
+  a.in_f = l[0]->in_f;
+  a.x = x;
+  a.ldx = ldx;
+  a.batch = batch;
+  a.rows = rows;
+  a.nrows = nrows;
+  a.ldy = ldy;
+  a.scatter = scatter;
+  if (wide) return wide_rows(a, l[0]->out_f, mats, st);
+  return chain_rows<false>(a, mats, st);
+}
+
+template <int TB>
+static void chain_down_go(const kh_dejavu_linear* d, const float* h, int64_t batch, const int64_t* sel,
+                          int n, float* y, hipStream_t st) {
+  const int H = d->out_f;
+  const dim3 g((unsigned)ceil_div(H, kDcRows), (unsigned)ceil_div(batch, TB));
+  if (H % 4 == 0)
+    hipLaunchKernelGGL((dl_chain_down_kernel<TB, true>), g, dim3(kDcThreads), 0, st, d->wt, d->bias, H, h, batch,
+                       sel, n, y);
+  else
+    hipLaunchKernelGGL((dl_chain_down_kernel<TB, false>), g, dim3(kDcThreads), 0, st, d->wt, d->bias, H, h, batch,
+                       sel, n, y);
 }
 
 }  // namespace kh
@@ -172,29 +460,28 @@ extern "C" int kh_dejavu_linear_create(int in_features, int out_features, const 
                out_features);
   *out = nullptr;
   const size_t n = (size_t)in_features * (size_t)out_features;
-  std::vector<float> wt(n);
-  for (int r = 0; r < out_features; ++r)
-    for (int j = 0; j < in_features; ++j)
-      wt[(size_t)j * out_features + r] = w_host[(size_t)r * in_features + j];
   auto* l = new kh_dejavu_linear;
   l->in_f = in_features;
   l->out_f = out_features;
+  l->w = static_cast<float*>(dev_alloc(n * sizeof(float)));
   l->wt = static_cast<float*>(dev_alloc(n * sizeof(float)));
   l->bias = static_cast<float*>(dev_alloc((size_t)out_features * sizeof(float)));
-  if (!l->wt || !l->bias) {
-    dev_free(l->wt);
-    dev_free(l->bias);
-    delete l;
+  if (!l->w || !l->wt || !l->bias) {
+    kh_dejavu_linear_destroy(l);
     return KH_ERR_ALLOC;
   }
-  hipError_t e = hipMemcpy(l->wt, wt.data(), n * sizeof(float), hipMemcpyHostToDevice);
+  hipError_t e = hipMemcpy(l->w, w_host, n * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(l->bias, b_host, (size_t)out_features * sizeof(float), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(transpose_kernel<float>, dim3(ceil_div(in_features, 32), ceil_div(out_features, 32)),
+                       dim3(256), 0, 0, l->w, out_features, in_features, l->wt);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+  }
   if (e != hipSuccess) {
-    set_error("hipMemcpy failed: %s", hipGetErrorString(e));
-    dev_free(l->wt);
-    dev_free(l->bias);
-    delete l;
+    set_error("linear upload failed: %s", hipGetErrorString(e));
+    kh_dejavu_linear_destroy(l);
     return KH_ERR_HIP;
   }
   *out = l;
@@ -203,6 +490,7 @@ extern "C" int kh_dejavu_linear_create(int in_features, int out_features, const 
 
 extern "C" int kh_dejavu_linear_destroy(kh_dejavu_linear* l) {
   if (!l) return KH_OK;
+  dev_free(l->w);
   dev_free(l->wt);
   dev_free(l->bias);
   delete l;
@@ -213,7 +501,7 @@ extern "C" int kh_dejavu_linear_forward(const kh_dejavu_linear* l, const float* 
                                         int64_t batch, float* y_dev, void* stream) {
   KH_CHECK_ARG(l && x_dev && y_dev, "null argument");
   KH_CHECK_ARG(batch >= 0, "bad batch");
-  return rows_launch(l, x_dev, l->in_f, batch, nullptr, l->out_f, y_dev, l->out_f, 0,
+  return rows_launch(&l, 1, x_dev, l->in_f, batch, nullptr, l->out_f, &y_dev, l->out_f, 0,
                      as_stream(stream));
 }
 
@@ -227,7 +515,7 @@ extern "C" int kh_dejavu_linear_forward_sparse(const kh_dejavu_linear* l, const 
   const int64_t* rows = nullptr;
   int rc = upload_indices(l->ws.get(st), idx_host, n_idx, l->out_f, "row", st, &rows);
   if (rc != KH_OK) return rc;
-  return rows_launch(l, x_dev, l->in_f, batch, rows, n_idx, y_dev, n_idx, 0, st);
+  return rows_launch(&l, 1, x_dev, l->in_f, batch, rows, n_idx, &y_dev, n_idx, 0, st);
 }
 
 extern "C" int kh_dejavu_sparse_mlp_create(int hidden, int inter, kh_dejavu_sparse_mlp** out) {
@@ -265,13 +553,28 @@ extern "C" int kh_dejavu_sparse_mlp_forward(const kh_dejavu_sparse_mlp* m, const
   float* h = static_cast<float*>(m->ws.get(st)->get(1, sizeof(float) * (size_t)(batch * n_sel + 1)));
   if (!h) return KH_ERR_ALLOC;
   if (batch * n_sel > 0) {
-    hipLaunchKernelGGL(dl_gateup_kernel, dim3(grid_for(batch * n_sel)), dim3(kDlThreads), 0, st,
-                       gate->wt, gate->bias, up->wt, up->bias, H, I, x_dev, batch, sel, n_sel, h);
+    DcRows g{};
+    g.m[0] = {gate->w, gate->bias, h};
+    g.m[1] = {up->w, up->bias, nullptr};
+    g.in_f = H;
+    g.x = x_dev;
+    g.ldx = H;
+    g.batch = batch;
+    g.rows = sel;
+    g.nrows = n_sel;
+    g.ldy = n_sel;
+    rc = chain_rows<true>(g, 1, st);
+    if (rc != KH_OK) return rc;
+  }
+  for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
+    const int64_t nb = std::min<int64_t>(batch - b0, 65535);
+    const float* hb = h + b0 * n_sel;
+    float* yb = y_dev + b0 * H;
+    if (nb == 1) chain_down_go<1>(down, hb, nb, sel, (int)n_sel, yb, st);
+    else if (nb == 2) chain_down_go<2>(down, hb, nb, sel, (int)n_sel, yb, st);
+    else chain_down_go<4>(down, hb, nb, sel, (int)n_sel, yb, st);
     KH_LAUNCHED();
   }
-  hipLaunchKernelGGL(dl_down_kernel, dim3(grid_for(batch * H)), dim3(kDlThreads), 0, st, down->wt,
-                     down->bias, H, h, batch, sel, n_sel, y_dev);
-  KH_LAUNCHED();
   return KH_OK;
 }
 
@@ -321,16 +624,15 @@ extern "C" int kh_dejavu_sparse_attention_forward(
   float* buf = static_cast<float*>(a->ws.get(st)->get(1, sizeof(float) * (size_t)(4 * batch * qd)));
   if (!buf) return KH_ERR_ALLOC;
   float *qv = buf, *kv = buf + batch * qd, *vv = buf + 2 * batch * qd, *att = buf + 3 * batch * qd;
-  if ((rc = fill_zero(buf, 4 * batch * qd, st)) != KH_OK) return rc;
   const int64_t* rows = dl + n_heads;
-  const int64_t nrows = n_heads * hd;
-  if ((rc = rows_launch(q, x_dev, H, batch, rows, nrows, qv, qd, 1, st)) != KH_OK) return rc;
-  if ((rc = rows_launch(k, x_dev, H, batch, rows, nrows, kv, qd, 1, st)) != KH_OK) return rc;
-  if ((rc = rows_launch(v, x_dev, H, batch, rows, nrows, vv, qd, 1, st)) != KH_OK) return rc;
-  if (batch * n_heads > 0) {
-    hipLaunchKernelGGL(dl_head_score_kernel, dim3(grid_for(batch * n_heads)), dim3(kDlThreads), 0,
-                       st, qv, kv, vv, att, qd, hd, batch, dl, n_heads, sqrtf((float)hd));
+  const kh_dejavu_linear* qkv[3] = {q, k, v};
+  float* outs[3] = {qv, kv, vv};
+  if ((rc = rows_launch(qkv, 3, x_dev, H, batch, rows, n_heads * hd, outs, qd, 1, st)) != KH_OK) return rc;
+  for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
+    const int64_t o0 = b0 * qd;
+    hipLaunchKernelGGL(dl_head_score_kernel, dim3((unsigned)a->num_heads, (unsigned)std::min<int64_t>(batch - b0, 65535)),
+                       dim3(64), 0, st, qv + o0, kv + o0, vv + o0, att + o0, qd, hd, dl, n_heads, sqrtf((float)hd));
     KH_LAUNCHED();
   }
-  return rows_launch(o, att, qd, batch, nullptr, H, y_dev, H, 0, st);
+  return rows_launch(&o, 1, att, qd, batch, nullptr, H, &y_dev, H, 0, st);
 }

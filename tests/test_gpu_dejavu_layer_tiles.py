@@ -1,0 +1,65 @@
+"""GPU parity: the klearu-dejavu layer's kernels at the edges of their tiles (16 rows and
+4 tokens per block, 128 steps per chunk, four chunks in flight; the thread-per-output
+form from 98304 outputs), vs the oracle.  Bar: bit-exact."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_dejavu_layer import bits, xavier
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("in_f,out_f,batch", [
+    (1, 1, 1), (3, 17, 2), (4, 15, 5), (127, 16, 3), (128, 33, 4), (129, 31, 6), (512, 20, 1), (516, 18, 2),
+    (640, 48, 7), (20, 1024, 96), (37, 1100, 90), (16, 6200, 64), (33, 99000, 1), (48, 33000, 3)])
+def test_linear_tile_edges(kh, orc, in_f, out_f, batch):
+    from klearu_amd.dejavu_transformer import Linear
+    rng = np.random.default_rng(in_f * 7 + out_f + batch)
+    w, b = xavier(rng, out_f, in_f), rng.normal(0, 0.1, out_f).astype(np.float32)
+    x = rng.standard_normal((batch, in_f)).astype(np.float32)
+    x[0, ::3] = 0.0
+    # a base 4 bytes past a 16-byte boundary: no vector loads of the inputs
+    pad = torch.zeros(batch * in_f + 1, device="cuda")
+    pad[1:] = torch.from_numpy(x).reshape(-1)
+    lin = Linear(w, b)
+    idx = rng.integers(0, out_f, 19)
+    for xd in (torch.from_numpy(x).cuda(), pad[1:].view(batch, in_f)):
+        y, ys = lin.forward(xd).cpu().numpy(), lin.forward_sparse(xd, idx).cpu().numpy()
+        for r in sorted({0, batch // 2, batch - 1}):
+            ref = orc.dejavu_linear_forward(w, b, x[r])
+            np.testing.assert_array_equal(bits(y[r]), bits(ref))
+            np.testing.assert_array_equal(bits(ys[r]), bits(ref[idx]))
+
+
+@pytest.mark.parametrize("H,I,n,batch", [(1, 1, 1, 1), (17, 40, 9, 3), (64, 300, 129, 5), (130, 90, 8, 2), (20, 700, 640, 4)])
+def test_sparse_mlp_tile_edges(kh, orc, H, I, n, batch):
+    """Non-finite weights of a neuron whose activation is zero add nothing."""
+    from klearu_amd.dejavu_transformer import Linear, SparseMlp
+    rng = np.random.default_rng(H + I + n)
+    wg, wu, wd = xavier(rng, I, H), xavier(rng, I, H), xavier(rng, H, I)
+    bg, bu, bd = (rng.normal(0, 0.05, m).astype(np.float32) for m in (I, I, H))
+    wu[0], bu[0] = 0.0, 0.0
+    wd[:, 0] = np.inf
+    x = rng.standard_normal((batch, H)).astype(np.float32)
+    sel = rng.choice(I, n, replace=False)
+    sel[0] = 0
+    y = SparseMlp(H, I).forward(torch.from_numpy(x).cuda(), Linear(wg, bg), Linear(wu, bu), Linear(wd, bd), sel)
+    for r in range(batch):
+        ref = orc.dejavu_sparse_mlp_forward(wg, bg, wu, bu, wd, bd, x[r], sel)
+        np.testing.assert_array_equal(bits(y[r].cpu().numpy()), bits(ref))
+
+
+@pytest.mark.parametrize("H,nh,hd,batch", [(24, 3, 1, 2), (40, 2, 63, 1), (32, 2, 65, 5), (16, 1, 200, 3)])
+def test_sparse_attention_head_dims(kh, orc, H, nh, hd, batch):
+    from klearu_amd.dejavu_transformer import Linear, SparseAttention
+    rng = np.random.default_rng(H + hd)
+    ws = [xavier(rng, nh * hd, H) for _ in range(3)] + [xavier(rng, H, nh * hd)]
+    bs = [rng.normal(0, 0.05, w.shape[0]).astype(np.float32) for w in ws]
+    x = rng.standard_normal((batch, H)).astype(np.float32)
+    heads = [nh - 1]
+    y = SparseAttention(H, nh, hd).forward(torch.from_numpy(x).cuda(), *(Linear(w, b) for w, b in zip(ws, bs)), heads)
+    args = [a for pair in zip(ws, bs) for a in pair]
+    for r in range(batch):
+        ref = orc.dejavu_sparse_attention_forward(*args, nh, hd, x[r], heads)
+        np.testing.assert_array_equal(bits(y[r].cpu().numpy()), bits(ref))
