@@ -530,8 +530,9 @@ int kh_dejavu_mlp_block_batch(const kh_predictor* p, const kh_sparse_ffn* f, flo
 /* klearu-dejavu transformer layer: f32 Linear with bias, SparseMlp,        */
 /* SparseAttention (crates/klearu-dejavu/src/{transformer/mod.rs,mlp.rs,     */
 /* attention.rs}).  Outputs are bit-identical to the reference.  Index lists */
-/* are host arrays (the reference's &[usize]); these calls wait until the   */
-/* list is uploaded, then leave the kernels queued on `stream`.             */
+/* are host arrays (the reference's &[usize]), free to go on return; lists   */
+/* of up to 960 indices travel in a launch, for longer ones the call waits   */
+/* until the list is uploaded.  The kernels stay queued on `stream`.         */
 /* ======================================================================== */
 
 typedef struct kh_dejavu_linear kh_dejavu_linear;

@@ -22,11 +22,10 @@
 // of a gather read in whole pieces, and transposed [in][out], which the columns
 // of SparseMlp's down projection and the wide form below read.
 // Index lists arrive from the host (the reference's &[usize]), are checked
-// there (an out-of-range index is the reference's panic) and are uploaded to
-// the handle's scratch; the upload is waited for, so the caller's list may be
-// freed on return and the kernels stay queued behind it.
+// there (an out-of-range index is the reference's panic) and go to the handle's
+// scratch: short ones inside a launch, longer ones by a copy that is waited for;
+// either way the caller's list may be freed on return.
 #include <algorithm>
-#include <vector>
 
 #include "chain_add.hpp"
 #include "gather.hpp"
@@ -89,8 +88,17 @@ struct DcRows {
   int64_t ldx, batch;
   const int64_t* rows;  // null: every row
   int64_t nrows, ldy;
+  int head_dim;       // 0: rows lists rows; else it lists heads of head_dim rows each
   int scatter;        // outputs at y[row] instead of y[position in the list]
 };
+
+// Output row of position `at` of the call's list.
+__device__ __forceinline__ int64_t dc_row(const DcRows& a, int64_t at) {
+  if (!a.rows) return at;
+  if (a.head_dim == 0) return a.rows[at];
+  const int64_t h = at / a.head_dim;
+  return a.rows[h] * a.head_dim + (at - h * a.head_dim);
+}
 
 // Eight producer waves and the consumer step through nch chunks: make(c, u) puts
 // chunk c's products (register slot u = c % kDcAhead) into LDS buffer c & 1 and
@@ -142,7 +150,7 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_rows_kernel(const DcRows 
   const int k4 = pt >> 4;
   const DcMat& mat = a.m[GATEUP ? i / kOwn : (int)blockIdx.z];
   const int64_t at = min(a0 + (GATEUP ? i % kOwn : i), a.nrows - 1);
-  const int64_t r = a.rows ? a.rows[at] : at;
+  const int64_t r = dc_row(a, at);
   const float* __restrict__ wr = mat.w + r * n;
   const float* __restrict__ xr[TB];
 #pragma unroll
@@ -249,7 +257,7 @@ constexpr int kDlAhead = 16;
 template <int TB>
 __global__ __launch_bounds__(64) void dl_wide_rows_kernel(const DcRows a, int out_f) {
   const int64_t at = min((int64_t)blockIdx.x * 64 + threadIdx.x, a.nrows - 1);
-  const int64_t r = a.rows ? a.rows[at] : at;
+  const int64_t r = dc_row(a, at);
   const int64_t b0 = (int64_t)blockIdx.y * TB;
   const DcMat& mat = a.m[blockIdx.z];
   const float* __restrict__ wt = mat.w + r;
@@ -337,7 +345,19 @@ static unsigned grid_for(int64_t threads) {
   return (unsigned)((threads + kDlThreads - 1) / kDlThreads);
 }
 
-// Checks idx_host[0..n) against [0, bound) and uploads it to slot 0 of the
+// Lists of up to kDlArgList indices travel in the launch itself: the caller's
+// list may be freed on return and nothing waits, where a copy from pageable host
+// memory made every call wait for its stream (f32 layer of 822 neurons and 6
+// heads, 3 tokens: see kh_dejavu_sparse_mlp_forward).  Longer lists are copied.
+constexpr int kDlArgList = 960;
+struct DlList {
+  int32_t v[kDlArgList];
+};
+__global__ __launch_bounds__(kDlThreads) void dl_list_kernel(const DlList l, int n, int64_t* __restrict__ out) {
+  for (int i = threadIdx.x; i < n; i += kDlThreads) out[i] = l.v[i];
+}
+
+// Checks idx_host[0..n) against [0, bound) and puts it into slot 0 of the
 // stream's workspace w.
 static int upload_indices(WsSet* w, const int64_t* idx_host, int64_t n, int64_t bound,
                           const char* what, hipStream_t st, const int64_t** out) {
@@ -347,7 +367,12 @@ static int upload_indices(WsSet* w, const int64_t* idx_host, int64_t n, int64_t 
                  (long long)bound);
   int64_t* d = static_cast<int64_t*>(w->get(0, sizeof(int64_t) * (size_t)(n > 0 ? n : 1)));
   if (!d) return KH_ERR_ALLOC;
-  if (n > 0) {
+  if (n > 0 && n <= kDlArgList) {
+    DlList l;
+    for (int64_t a = 0; a < n; ++a) l.v[a] = static_cast<int32_t>(idx_host[a]);   // bound is an int
+    hipLaunchKernelGGL(dl_list_kernel, dim3(1), dim3(kDlThreads), 0, st, l, (int)n, d);
+    KH_LAUNCHED();
+  } else if (n > 0) {
     KH_HIP(hipMemcpyAsync(d, idx_host, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, st));
     KH_HIP(hipStreamSynchronize(st));
   }
@@ -419,7 +444,7 @@ static int wide_rows(DcRows a, int out_f, int mats, hipStream_t st) {
 // `mats` projections of one shape (bias, outputs y[i]) of the same inputs.
 static int rows_launch(const kh_dejavu_linear* const* l, int mats, const float* x, int64_t ldx,
                        int64_t batch, const int64_t* rows, int64_t nrows, float* const* y,
-                       int64_t ldy, int scatter, hipStream_t st) {
+                       int64_t ldy, int scatter, int head_dim, hipStream_t st) {
   if (batch * nrows == 0) return KH_OK;
   const bool wide = batch * nrows >= kDlWide;
   DcRows a{};
@@ -432,6 +457,7 @@ static int rows_launch(const kh_dejavu_linear* const* l, int mats, const float* 
   a.nrows = nrows;
   a.ldy = ldy;
   a.scatter = scatter;
+  a.head_dim = head_dim;
   if (wide) return wide_rows(a, l[0]->out_f, mats, st);
   return chain_rows<false>(a, mats, st);
 }
@@ -501,7 +527,7 @@ extern "C" int kh_dejavu_linear_forward(const kh_dejavu_linear* l, const float* 
                                         int64_t batch, float* y_dev, void* stream) {
   KH_CHECK_ARG(l && x_dev && y_dev, "null argument");
   KH_CHECK_ARG(batch >= 0, "bad batch");
-  return rows_launch(&l, 1, x_dev, l->in_f, batch, nullptr, l->out_f, &y_dev, l->out_f, 0,
+  return rows_launch(&l, 1, x_dev, l->in_f, batch, nullptr, l->out_f, &y_dev, l->out_f, 0, 0,
                      as_stream(stream));
 }
 
@@ -515,7 +541,7 @@ extern "C" int kh_dejavu_linear_forward_sparse(const kh_dejavu_linear* l, const 
   const int64_t* rows = nullptr;
   int rc = upload_indices(l->ws.get(st), idx_host, n_idx, l->out_f, "row", st, &rows);
   if (rc != KH_OK) return rc;
-  return rows_launch(&l, 1, x_dev, l->in_f, batch, rows, n_idx, &y_dev, n_idx, 0, st);
+  return rows_launch(&l, 1, x_dev, l->in_f, batch, rows, n_idx, &y_dev, n_idx, 0, 0, st);
 }
 
 extern "C" int kh_dejavu_sparse_mlp_create(int hidden, int inter, kh_dejavu_sparse_mlp** out) {
@@ -609,30 +635,20 @@ extern "C" int kh_dejavu_sparse_attention_forward(
                "projection shapes do not match hidden %d / %d heads x %d", H, a->num_heads, hd);
   if (batch == 0) return KH_OK;
   hipStream_t st = as_stream(stream);
-  for (int64_t i = 0; i < n_heads; ++i)
-    KH_CHECK_ARG(heads_host[i] >= 0 && heads_host[i] < a->num_heads,
-                 "head index %lld out of range (%d)", (long long)heads_host[i], a->num_heads);
-  // index list: the selected heads, then the q/k/v rows of each selected head
-  std::vector<int64_t> lists((size_t)(n_heads + n_heads * hd));
-  for (int64_t i = 0; i < n_heads; ++i) {
-    lists[(size_t)i] = heads_host[i];
-    for (int d = 0; d < hd; ++d) lists[(size_t)(n_heads + i * hd + d)] = heads_host[i] * hd + d;
-  }
   const int64_t* dl = nullptr;
-  int rc = upload_indices(a->ws.get(st), lists.data(), (int64_t)lists.size(), qd, "row", st, &dl);
+  int rc = upload_indices(a->ws.get(st), heads_host, n_heads, a->num_heads, "head", st, &dl);
   if (rc != KH_OK) return rc;
   float* buf = static_cast<float*>(a->ws.get(st)->get(1, sizeof(float) * (size_t)(4 * batch * qd)));
   if (!buf) return KH_ERR_ALLOC;
   float *qv = buf, *kv = buf + batch * qd, *vv = buf + 2 * batch * qd, *att = buf + 3 * batch * qd;
-  const int64_t* rows = dl + n_heads;
   const kh_dejavu_linear* qkv[3] = {q, k, v};
   float* outs[3] = {qv, kv, vv};
-  if ((rc = rows_launch(qkv, 3, x_dev, H, batch, rows, n_heads * hd, outs, qd, 1, st)) != KH_OK) return rc;
+  if ((rc = rows_launch(qkv, 3, x_dev, H, batch, dl, n_heads * hd, outs, qd, 1, hd, st)) != KH_OK) return rc;
   for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
     const int64_t o0 = b0 * qd;
     hipLaunchKernelGGL(dl_head_score_kernel, dim3((unsigned)a->num_heads, (unsigned)std::min<int64_t>(batch - b0, 65535)),
                        dim3(64), 0, st, qv + o0, kv + o0, vv + o0, att + o0, qd, hd, dl, n_heads, sqrtf((float)hd));
     KH_LAUNCHED();
   }
-  return rows_launch(&o, 1, att, qd, batch, nullptr, H, &y_dev, H, 0, st);
+  return rows_launch(&o, 1, att, qd, batch, nullptr, H, &y_dev, H, 0, 0, st);
 }

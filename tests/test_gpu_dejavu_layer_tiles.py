@@ -63,3 +63,14 @@ def test_sparse_attention_head_dims(kh, orc, H, nh, hd, batch):
     for r in range(batch):
         ref = orc.dejavu_sparse_attention_forward(*args, nh, hd, x[r], heads)
         np.testing.assert_array_equal(bits(y[r].cpu().numpy()), bits(ref))
+
+
+@pytest.mark.parametrize("n", [960, 961])
+def test_index_list_in_the_launch_and_copied(kh, orc, n):
+    from klearu_amd.dejavu_transformer import Linear
+    rng = np.random.default_rng(n)
+    w, b = xavier(rng, 500, 12), rng.normal(0, 0.1, 500).astype(np.float32)
+    x = rng.standard_normal(12).astype(np.float32)
+    idx = rng.integers(0, 500, n)
+    y = Linear(w, b).forward_sparse(x, idx).cpu().numpy()
+    np.testing.assert_array_equal(bits(y), bits(orc.dejavu_linear_forward(w, b, x)[idx]))
