@@ -9,7 +9,7 @@
 // then a scalar tail.  Here each of those accumulator lanes is a GPU lane
 // running the same FMA chain, so the results are bit-identical.  The BF16
 // dots are sequential sums and run as one chain per row.
-#include "common.hpp"
+#include "chain_add.hpp"
 
 namespace kh {
 
@@ -19,7 +19,11 @@ __device__ __forceinline__ float hsum8_tree(const float v[8]) {
   return (s0 + s1) + (s2 + s3);
 }
 
-// One 16-lane group per row; 4 rows per wave.
+// One 16-lane group per row; 4 rows per wave.  A lane's chain is n / 16 FMAs, so
+// what counts is the rows' bytes in flight: kDdAhead chunks are requested while
+// the kDdAhead before them are added.  11008 x 4096 (180 MB): 33 us, 5.4 TB/s
+// (85 us with one chunk at a time).
+constexpr int kDdAhead = 16;
 __global__ __launch_bounds__(256) void dense_dot_kernel(const float* __restrict__ a, int64_t rows,
                                                         int64_t lda, const float* __restrict__ b,
                                                         int64_t n, float* __restrict__ out) {
@@ -27,14 +31,39 @@ __global__ __launch_bounds__(256) void dense_dot_kernel(const float* __restrict_
   const int64_t row = gid >> 4;
   const int l = threadIdx.x & 15;
   const bool ok = row < rows;
-  const float* ar = a + (ok ? row : 0) * lda;
-  const int64_t chunks = n / 16;
+  const float* __restrict__ ar = a + (ok ? row : 0) * lda;
+  const int64_t chunks = n / 16, full = chunks / kDdAhead * kDdAhead;
   float acc = 0.0f;
-  if (ok)
-    for (int64_t c = 0; c < chunks; ++c) acc = fmaf(ar[c * 16 + l], b[c * 16 + l], acc);
+  float a0[kDdAhead], a1[kDdAhead], b0[kDdAhead], b1[kDdAhead];
+  // the last group's request past the end repeats the group before it
+  auto load = [&](float (&av)[kDdAhead], float (&bv)[kDdAhead], int64_t c) {
+    const int64_t c1 = min(c, full - kDdAhead);
+#pragma unroll
+    for (int u = 0; u < kDdAhead; ++u) av[u] = ar[(c1 + u) * 16 + l];
+#pragma unroll
+    for (int u = 0; u < kDdAhead; ++u) bv[u] = b[(c1 + u) * 16 + l];
+  };
+  auto add = [&](const float (&av)[kDdAhead], const float (&bv)[kDdAhead]) {
+#pragma unroll
+    for (int u = 0; u < kDdAhead; ++u) acc = fmaf(av[u], bv[u], acc);
+  };
+  int64_t c = 0;
+  if (full > 0) {
+    load(a0, b0, 0);
+    for (; c + kDdAhead < full; c += 2 * kDdAhead) {
+      load(a1, b1, c + kDdAhead);
+      __builtin_amdgcn_sched_barrier(0);
+      add(a0, b0);
+      load(a0, b0, c + 2 * kDdAhead);
+      __builtin_amdgcn_sched_barrier(0);
+      add(a1, b1);
+    }
+    if (c < full) add(a0, b0);
+  }
+  for (c = full; c < chunks; ++c) acc = fmaf(ar[c * 16 + l], b[c * 16 + l], acc);
   const int64_t rs = chunks * 16;
   const bool extra = rs + 8 <= n;
-  if (ok && extra && l < 8) acc = fmaf(ar[rs + l], b[rs + l], acc);
+  if (extra && l < 8) acc = fmaf(ar[rs + l], b[rs + l], acc);
   // lane l < 8 holds acc0[l], lane l+8 holds acc1[l]
   const float other = __shfl_down(acc, 8, 16);
   float v[8];
@@ -46,91 +75,269 @@ __global__ __launch_bounds__(256) void dense_dot_kernel(const float* __restrict_
   out[row] = sum;
 }
 
-__global__ __launch_bounds__(64) void sparse_dot_kernel(const uint32_t* __restrict__ idx,
-                                                        const float* __restrict__ val, int64_t nnz,
-                                                        const float* __restrict__ dense,
-                                                        float* __restrict__ out) {
+// The whole block gathers a tile of (value, dense value) pairs into LDS, then
+// lanes 0..7 run the reference's eight FMA lanes over it, so a call waits for two
+// dependent loads per tile and not per 8 entries (75 entries: 8.1 -> 4.9 us).
+constexpr int kSdTile = 2048;
+__global__ __launch_bounds__(256) void sparse_dot_kernel(const uint32_t* __restrict__ idx,
+                                                         const float* __restrict__ val, int64_t nnz,
+                                                         const float* __restrict__ dense,
+                                                         float* __restrict__ out) {
+  __shared__ float sv[kSdTile], sd[kSdTile];
+  constexpr int kPer = kSdTile / 256;
   const int l = threadIdx.x;
   const int64_t chunks = nnz / 8;
-  float acc = 0.0f;
-  if (l < 8)
-    for (int64_t c = 0; c < chunks; ++c) acc = fmaf(val[c * 8 + l], dense[idx[c * 8 + l]], acc);
-  float v[8];
+  float acc = 0.0f, sum = 0.0f;
+  for (int64_t e0 = 0; e0 < nnz; e0 += kSdTile) {
+    uint32_t id[kPer];
+    float v[kPer], d[kPer];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = __shfl(acc, i, 64);
-  if (l != 0) return;
-  float sum = hsum8_tree(v);
-  for (int64_t i = chunks * 8; i < nnz; ++i) sum = __fadd_rn(sum, __fmul_rn(val[i], dense[idx[i]]));
-  *out = sum;
+    for (int u = 0; u < kPer; ++u) {
+      const int64_t e = min(e0 + u * 256 + l, nnz - 1);
+      id[u] = idx[e];
+      v[u] = val[e];
+    }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) d[u] = dense[id[u]];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      sv[u * 256 + l] = v[u];
+      sd[u * 256 + l] = d[u];
+    }
+    __syncthreads();
+    const int64_t left = chunks * 8 - e0;
+    const int m = (int)(left < 0 ? 0 : left < kSdTile ? left : kSdTile);
+    if (l < 8)
+      for (int e = l; e < m; e += 8) acc = fmaf(sv[e], sd[e], acc);
+    if (e0 + kSdTile >= nnz && l < 64) {   // last tile: the lanes' sum, then the scalar tail
+      float t[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t[i] = __shfl(acc, i, 64);
+      sum = hsum8_tree(t);
+      const int end = (int)(nnz - e0);
+      for (int e = m; e < end; ++e) sum = __fadd_rn(sum, __fmul_rn(sv[e], sd[e]));
+    }
+  }
+  if (l == 0) *out = sum;
 }
 
-// Deterministic scatter-add: chunks of 1024 entries in order; within a chunk
-// the first occurrence of each index applies all of that index's updates in
-// entry order, one rounded add at a time (as scatter_add_avx2's scalar stores).
+// Deterministic scatter-add: chunks of 1024 entries in order; within a chunk the
+// first occurrence of each index applies all of that index's updates in entry
+// order, one rounded add at a time (as scatter_add_avx2's scalar stores).  An LDS
+// hash table of entry positions finds each index's first entry and its count, so
+// only an index that repeats looks through the chunk (75 entries: 11.6 -> 4.5 us
+// against a look through all earlier and later entries by every thread).
+constexpr int kSaSlots = 2048;
 __global__ __launch_bounds__(1024) void scatter_add_kernel(const uint32_t* __restrict__ idx,
                                                            const float* __restrict__ val,
                                                            int64_t n, float* __restrict__ dense,
                                                            float scale) {
   __shared__ uint32_t sidx[1024];
   __shared__ float sval[1024];
+  __shared__ int rep[kSaSlots];    // 1 + position of an entry with the slot's index; 0: free
+  __shared__ int first[kSaSlots], count[kSaSlots];
+  const int t = threadIdx.x;
   for (int64_t c0 = 0; c0 < n; c0 += 1024) {
     const int m = (int)min<int64_t>(1024, n - c0);
-    const int t = threadIdx.x;
+    const uint32_t me = idx[c0 + min(t, m - 1)];
+    const float v = __fmul_rn(val[c0 + min(t, m - 1)], scale);
+    sidx[t] = me;
+    sval[t] = v;
+    for (int s = t; s < kSaSlots; s += 1024) {
+      rep[s] = 0;
+      first[s] = 1024;
+      count[s] = 0;
+    }
+    const float d0 = dense[me];   // no entry of this chunk is applied before the next barrier
+    __syncthreads();
+    int slot = 0;
     if (t < m) {
-      sidx[t] = idx[c0 + t];
-      sval[t] = __fmul_rn(val[c0 + t], scale);
+      slot = (int)((me * 2654435761u) >> 21);
+      for (;;) {   // at most 1024 indices in 2048 slots: a free or matching slot comes
+        const int r = atomicCAS(&rep[slot], 0, t + 1);
+        if (r == 0 || sidx[r - 1] == me) break;
+        slot = (slot + 1) & (kSaSlots - 1);
+      }
+      atomicMin(&first[slot], t);
+      atomicAdd(&count[slot], 1);
     }
     __syncthreads();
-    if (t < m) {
-      const uint32_t me = sidx[t];
-      bool first = true;
-      for (int j = 0; j < t; ++j)
+    if (t < m && first[slot] == t) {
+      float d = __fadd_rn(d0, v);
+      int more = count[slot] - 1;
+      for (int j = t + 1; more > 0; ++j)
         if (sidx[j] == me) {
-          first = false;
-          break;
+          d = __fadd_rn(d, sval[j]);
+          --more;
         }
-      if (first) {
-        float d = dense[me];
-        for (int j = t; j < m; ++j)
-          if (sidx[j] == me) d = __fadd_rn(d, sval[j]);
-        dense[me] = d;
-      }
+      dense[me] = d;
     }
     __syncthreads();
   }
 }
 
-__global__ void bf16_from_f32_kernel(const float* __restrict__ x, uint16_t* __restrict__ o, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) o[i] = f32_to_bf16(x[i]);
-}
-__global__ void bf16_to_f32_kernel(const uint16_t* __restrict__ x, float* __restrict__ o, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) o[i] = bf16_to_f32(x[i]);
-}
-__global__ void bf16_update_kernel(uint16_t* __restrict__ w, const float* __restrict__ d, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) w[i] = f32_to_bf16(__fadd_rn(bf16_to_f32(w[i]), d[i]));
+// Elementwise kernels: eight elements per access (16 bytes of BF16, 32 of f32) and
+// kEwGroups of them in flight per thread where both arrays are 16-byte aligned;
+// one element per thread otherwise and for the last n % 8.  45 M elements, BF16
+// from f32 / f32 from BF16 (271 MB): 57 / 48 us, against 98 / 93 us with one
+// element per thread.
+constexpr int kEwGroups = 4;
+constexpr int kEwBlock = 256 * kEwGroups * 8;   // elements per block
+
+struct EwFromF32 {
+  using In = float;
+  using Out = uint16_t;
+  static __device__ __forceinline__ uint16_t at(float x, uint16_t) { return f32_to_bf16(x); }
+  static constexpr bool kReadOut = false;
+};
+struct EwToF32 {
+  using In = uint16_t;
+  using Out = float;
+  static __device__ __forceinline__ float at(uint16_t x, float) { return bf16_to_f32(x); }
+  static constexpr bool kReadOut = false;
+};
+struct EwUpdate {
+  using In = float;
+  using Out = uint16_t;
+  static __device__ __forceinline__ uint16_t at(float d, uint16_t w) {
+    return f32_to_bf16(__fadd_rn(bf16_to_f32(w), d));
+  }
+  static constexpr bool kReadOut = true;
+};
+
+template <typename T>
+struct alignas(16) EwVec {
+  T v[8];
+};
+
+template <typename Op>
+__global__ __launch_bounds__(256) void ew_vec_kernel(const typename Op::In* __restrict__ x,
+                                                     typename Op::Out* __restrict__ o, int64_t n) {
+  using VI = EwVec<typename Op::In>;
+  using VO = EwVec<typename Op::Out>;
+  const int64_t n8 = n / 8;
+  const int64_t g0 = (int64_t)blockIdx.x * 256 * kEwGroups + threadIdx.x;
+  const VI* __restrict__ xv = reinterpret_cast<const VI*>(x);
+  VO* __restrict__ ov = reinterpret_cast<VO*>(o);
+  VI a[kEwGroups];
+  VO r[kEwGroups];
+#pragma unroll
+  for (int u = 0; u < kEwGroups; ++u) {
+    const int64_t g = min(g0 + u * 256, n8 - 1);
+    a[u] = xv[g];
+    if (Op::kReadOut) r[u] = ov[g];
+  }
+#pragma unroll
+  for (int u = 0; u < kEwGroups; ++u) {
+    const int64_t g = g0 + u * 256;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[u].v[i] = Op::at(a[u].v[i], r[u].v[i]);
+    if (g < n8) ov[g] = r[u];
+  }
 }
 
-// Sequential chain per row (Bf16Weights::dot_f32 iterator sum from -0.0).
-__global__ void bf16_dot_f32_kernel(const uint16_t* __restrict__ w, int64_t rows, int64_t ldw,
-                                    const float* __restrict__ x, int64_t n, float* __restrict__ o) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
-  const uint16_t* wr = w + r * ldw;
-  float s = -0.0f;
-  for (int64_t i = 0; i < n; ++i) s = __fadd_rn(s, __fmul_rn(bf16_to_f32(wr[i]), x[i]));
-  o[r] = s;
+template <typename Op>
+__global__ __launch_bounds__(256) void ew_kernel(const typename Op::In* __restrict__ x,
+                                                 typename Op::Out* __restrict__ o, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) o[i] = Op::at(x[i], o[i]);
 }
 
-__global__ void bf16_full_dot_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
-                                     int64_t n, float* __restrict__ o) {
-  if (threadIdx.x != 0) return;
-  float s = -0.0f;
-  for (int64_t i = 0; i < n; ++i)
-    s = __fadd_rn(s, __fmul_rn(bf16_to_f32(a[i]), bf16_to_f32(b[i])));
-  *o = s;
+template <typename Op>
+static int ew_launch(const typename Op::In* x, typename Op::Out* o, int64_t n, hipStream_t st) {
+  int64_t done = 0;
+  if (n >= 8 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(o)) & 15) == 0) {
+    done = n / 8 * 8;
+    hipLaunchKernelGGL(ew_vec_kernel<Op>, dim3((unsigned)ceil_div(done, kEwBlock)), dim3(256), 0, st, x, o, n);
+    KH_LAUNCHED();
+  }
+  if (done < n) {
+    hipLaunchKernelGGL(ew_kernel<Op>, dim3((unsigned)ceil_div(n - done, 256)), dim3(256), 0, st, x + done, o + done,
+                       n - done);
+    KH_LAUNCHED();
+  }
+  return KH_OK;
+}
+
+// Sequential sums of rows (Bf16Weights::dot_f32's iterator sum from -0.0): a chain
+// of n dependent adds per row bounds a call, so producer waves form the products
+// in LDS, kChainAhead chunks of weights in flight, and wave 0 adds, four per read.
+// ROWS rows per block: 16 when there are several, 1 (and longer chunks) for one.
+// One row of 4096: 13.4 us (8.2 us of adds at 4.8 cycles), against 316 us with one
+// lane loading and adding.
+template <int ROWS>
+struct BdShape {
+  static constexpr int kStep = ROWS == 1 ? 512 : 128;
+  static constexpr int kProd = kStep / 4 * ROWS;
+  static constexpr int kThreads = 64 + kProd;
+};
+
+__device__ __forceinline__ float bd_f32(float x) { return x; }
+__device__ __forceinline__ float bd_f32(uint16_t x) { return bf16_to_f32(x); }
+template <typename T>
+struct alignas(4 * sizeof(T)) BdQuad {
+  T v[4];
+};
+// Elements k..k+3 of p (past n: the last one).  VEC: one access, n a multiple of 4
+// and p aligned to four elements.
+template <bool VEC, typename T>
+__device__ __forceinline__ BdQuad<T> bd_load(const T* __restrict__ p, int64_t k, int64_t n) {
+  if constexpr (VEC) return *reinterpret_cast<const BdQuad<T>*>(p + min(k, n - 4));
+  BdQuad<T> q;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q.v[i] = p[min(k + i, n - 1)];
+  return q;
+}
+
+template <int ROWS, bool VEC, typename TX>
+__global__ __launch_bounds__(BdShape<ROWS>::kThreads) void bf16_dot_kernel(
+    const uint16_t* __restrict__ w, int64_t rows, int64_t ldw, const TX* __restrict__ x, int64_t n,
+    float* __restrict__ o) {
+  constexpr int kStep = BdShape<ROWS>::kStep;
+  using Lds = ChainLds<kStep, ROWS>;
+  __shared__ Lds lds;
+  const int pt = (int)threadIdx.x - 64;
+  const int i = pt & (ROWS - 1), k4 = pt / ROWS;
+  const int64_t r0 = (int64_t)blockIdx.x * ROWS;
+  const uint16_t* __restrict__ wr = w + min(r0 + i, rows - 1) * ldw;
+  const int nch = (int)((n + kStep - 1) / kStep);
+  BdQuad<uint16_t> wv[kChainAhead];
+  BdQuad<TX> xv[kChainAhead];
+  auto fetch = [&](int64_t c, int u) {
+    const int64_t k = c * kStep + 4 * k4;
+    wv[u] = bd_load<VEC>(wr, k, n);
+    xv[u] = bd_load<VEC>(x, k, n);
+  };
+  if (pt >= 0 && nch > 0) {
+#pragma unroll
+    for (int u = 0; u < kChainAhead; ++u) fetch(u, u);
+  }
+  const float s = chain_run(lds, nch, -0.0f, [&](int c, int u) {
+    const int64_t k = (int64_t)c * kStep + 4 * k4;
+    float p[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = k + q < n ? __fmul_rn(bf16_to_f32(wv[u].v[q]), bd_f32(xv[u].v[q])) : -0.0f;
+    lds.q[c & 1][k4 * Lds::kStride + i] = make_float4(p[0], p[1], p[2], p[3]);
+    fetch(c + kChainAhead, u);
+  });
+  if (threadIdx.x < ROWS && r0 + (int)threadIdx.x < rows) o[r0 + threadIdx.x] = s;
+}
+
+template <typename TX>
+static int bf16_dot_launch(const uint16_t* w, int64_t rows, int64_t ldw, const TX* x, int64_t n, float* o,
+                           hipStream_t st) {
+  const bool vec = n > 0 && n % 4 == 0 && (rows == 1 || ldw % 4 == 0) &&
+                   reinterpret_cast<uintptr_t>(w) % (4 * sizeof(uint16_t)) == 0 &&
+                   reinterpret_cast<uintptr_t>(x) % (4 * sizeof(TX)) == 0;
+  if (rows == 1)
+    hipLaunchKernelGGL((vec ? bf16_dot_kernel<1, true, TX> : bf16_dot_kernel<1, false, TX>), dim3(1),
+                       dim3(BdShape<1>::kThreads), 0, st, w, rows, ldw, x, n, o);
+  else
+    hipLaunchKernelGGL((vec ? bf16_dot_kernel<16, true, TX> : bf16_dot_kernel<16, false, TX>),
+                       dim3((unsigned)ceil_div(rows, 16)), dim3(BdShape<16>::kThreads), 0, st, w, rows, ldw, x, n, o);
+  KH_LAUNCHED();
+  return KH_OK;
 }
 
 // f32::exp of every element, the same expf_glibc the predictor, SiLU and
@@ -162,7 +369,7 @@ extern "C" int kh_sparse_dot_dense(const uint32_t* idx_dev, const float* val_dev
                                    void* stream) {
   KH_CHECK_ARG(out_dev && dense_dev && (nnz == 0 || (idx_dev && val_dev)), "null argument");
   KH_CHECK_ARG(nnz >= 0 && dense_len >= 0, "bad shape");
-  hipLaunchKernelGGL(sparse_dot_kernel, dim3(1), dim3(64), 0, as_stream(stream), idx_dev, val_dev,
+  hipLaunchKernelGGL(sparse_dot_kernel, dim3(1), dim3(256), 0, as_stream(stream), idx_dev, val_dev,
                      nnz, dense_dev, out_dev);
   KH_LAUNCHED();
   return KH_OK;
@@ -179,32 +386,23 @@ extern "C" int kh_scatter_add(const uint32_t* idx_dev, const float* val_dev, int
   return KH_OK;
 }
 
-#define KH_ELEMENTWISE(kernel, ...)                                                     \
-  do {                                                                                  \
-    if (n == 0) return KH_OK;                                                           \
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,         \
-                       as_stream(stream), __VA_ARGS__);                                 \
-    KH_LAUNCHED();                                                                      \
-    return KH_OK;                                                                       \
-  } while (0)
-
 extern "C" int kh_bf16_from_f32(const float* x_dev, uint16_t* out_dev, int64_t n, void* stream) {
   KH_CHECK_ARG((x_dev && out_dev) || n == 0, "null argument");
   KH_CHECK_ARG(n >= 0, "bad n");
-  KH_ELEMENTWISE(bf16_from_f32_kernel, x_dev, out_dev, n);
+  return ew_launch<EwFromF32>(x_dev, out_dev, n, as_stream(stream));
 }
 
 extern "C" int kh_bf16_to_f32(const uint16_t* x_dev, float* out_dev, int64_t n, void* stream) {
   KH_CHECK_ARG((x_dev && out_dev) || n == 0, "null argument");
   KH_CHECK_ARG(n >= 0, "bad n");
-  KH_ELEMENTWISE(bf16_to_f32_kernel, x_dev, out_dev, n);
+  return ew_launch<EwToF32>(x_dev, out_dev, n, as_stream(stream));
 }
 
 extern "C" int kh_bf16_update_from_f32(uint16_t* w_dev, const float* delta_dev, int64_t n,
                                        void* stream) {
   KH_CHECK_ARG((w_dev && delta_dev) || n == 0, "null argument");
   KH_CHECK_ARG(n >= 0, "bad n");
-  KH_ELEMENTWISE(bf16_update_kernel, w_dev, delta_dev, n);
+  return ew_launch<EwUpdate>(delta_dev, w_dev, n, as_stream(stream));
 }
 
 extern "C" int kh_bf16_dot_f32(const uint16_t* w_dev, int64_t rows, int64_t ldw,
@@ -212,24 +410,21 @@ extern "C" int kh_bf16_dot_f32(const uint16_t* w_dev, int64_t rows, int64_t ldw,
   KH_CHECK_ARG(out_dev && ((w_dev && x_dev) || n == 0 || rows == 0), "null argument");
   KH_CHECK_ARG(rows >= 0 && n >= 0 && ldw >= n, "bad shape");
   if (rows == 0) return KH_OK;
-  hipLaunchKernelGGL(bf16_dot_f32_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0,
-                     as_stream(stream), w_dev, rows, ldw, x_dev, n, out_dev);
-  KH_LAUNCHED();
-  return KH_OK;
+  return bf16_dot_launch<float>(w_dev, rows, ldw, x_dev, n, out_dev, as_stream(stream));
 }
 
 extern "C" int kh_bf16_full_dot(const uint16_t* a_dev, const uint16_t* b_dev, int64_t n,
                                 float* out_dev, void* stream) {
   KH_CHECK_ARG(out_dev && (n == 0 || (a_dev && b_dev)), "null argument");
   KH_CHECK_ARG(n >= 0, "bad n");
-  hipLaunchKernelGGL(bf16_full_dot_kernel, dim3(1), dim3(64), 0, as_stream(stream), a_dev, b_dev,
-                     n, out_dev);
-  KH_LAUNCHED();
-  return KH_OK;
+  return bf16_dot_launch<uint16_t>(a_dev, 1, n, b_dev, n, out_dev, as_stream(stream));
 }
 
 extern "C" int kh_expf(const float* x_dev, float* y_dev, int64_t n, void* stream) {
   KH_CHECK_ARG((x_dev && y_dev) || n == 0, "null argument");
   KH_CHECK_ARG(n >= 0 && n <= ((int64_t)1 << 38), "bad n");
-  KH_ELEMENTWISE(expf_kernel, x_dev, y_dev, n);
+  if (n == 0) return KH_OK;
+  hipLaunchKernelGGL(expf_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, as_stream(stream), x_dev, y_dev, n);
+  KH_LAUNCHED();
+  return KH_OK;
 }

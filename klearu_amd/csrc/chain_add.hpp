@@ -41,4 +41,51 @@ __device__ __forceinline__ float chain_add_static(const float4* base, float r) {
   return r;
 }
 
+// Products of up to 64 chains in LDS, two chunks of STEP steps: quad q (steps
+// 4q..4q+3) of chain c at q[chunk & 1][q * kStride + c].
+constexpr int kChainAhead = 4;  // chunks in flight per producer thread
+template <int STEP, int CHAINS>
+struct ChainLds {
+  static constexpr int kStep = STEP, kChains = CHAINS;
+  static constexpr int kStride = CHAINS == 1 ? 1 : CHAINS + 1;
+  float4 q[2][STEP / 4 * kStride];
+};
+
+// The block steps through nch chunks: waves 1.. (producers) put chunk c's
+// products into LDS buffer c & 1 with make(c, u) (u = c % kChainAhead, the
+// thread's register slot) and there request chunk c + kChainAhead; wave 0 adds
+// the chunk before, lane l chain l, and returns s0 + every term in order.  The
+// loop has no branch around a load (chunks past the end are clamped, formed and
+// not added): behind a branch the compiler waits for every load in flight.
+template <typename Lds, typename Make>
+__device__ __forceinline__ float chain_run(Lds& lds, int nch, float s0, Make make) {
+  const int lane = threadIdx.x & 63;
+  float s = s0;
+  if (threadIdx.x >= 64) {
+    for (int c0 = 0; c0 < nch; c0 += kChainAhead) {
+#pragma unroll
+      for (int u = 0; u < kChainAhead; ++u) {
+        make(c0 + u, u);
+        lds_barrier();
+        // left alone, the scheduler forms every slot's products before the first
+        // barrier, and so waits for the last slot's loads there
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  } else {
+    const int last = (nch + kChainAhead - 1) / kChainAhead * kChainAhead;
+    for (int c = 0; c < last; ++c) {
+      lds_barrier();
+      if (c < nch) {
+        const float4* q = &lds.q[c & 1][min(lane, Lds::kChains - 1)];
+        constexpr int kGroup = Lds::kStep / 4 < 32 ? Lds::kStep / 4 : 32;
+#pragma unroll 1
+        for (int g = 0; g < Lds::kStep / 4; g += kGroup)
+          s = chain_add_static<kGroup, Lds::kStride>(q + g * Lds::kStride, s);
+      }
+    }
+  }
+  return s;
+}
+
 }  // namespace kh

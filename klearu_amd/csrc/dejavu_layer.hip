@@ -55,7 +55,7 @@ constexpr int kDlThreads = 256;
 // Few outputs: a chain of in_f dependent adds per output bounds the call (about
 // 6 cycles a step), so a block gives all else to other waves.  It owns 16 rows
 // x TB tokens, one chain per lane of wave 0 (the consumer); waves 1..8 hold the
-// weights of the next kDcAhead chunks of kDcStep steps in registers and form a
+// weights of the next kChainAhead chunks of kDcStep steps in registers and form a
 // chunk's products in LDS while wave 0 adds the chunk before, four per read.
 // Products past the end are -0.0, which leaves every sum unchanged.  A thread per
 // output with one load in flight per add took 107 us for a 1024-square Linear of
@@ -64,17 +64,12 @@ constexpr int kDlThreads = 256;
 // 1024 tokens: 11.8 -> 1.1 ms.
 constexpr int kDcRows = 16;                    // output rows (or columns) per block
 constexpr int kDcStep = 128;                   // steps per chunk
-constexpr int kDcAhead = 4;                    // chunks in flight per producer
 constexpr int kDcProd = kDcStep / 4 * kDcRows; // producer threads: one float4 of one row each
 constexpr int kDcThreads = 64 + kDcProd;
-constexpr int kDcQuads = kDcStep / 4;
-// Quads of one chunk [step / 4][chain], each quad row padded by one float4 so
-// that the down kernel's 4-byte writes fall in distinct banks.
+// Chunks of 16 * TB chains, padded by one float4 so that the down kernel's 4-byte
+// writes fall in distinct banks.
 template <int TB>
-struct DcLds {
-  static constexpr int kStride = kDcRows * TB + 1;
-  float4 q[2][kDcQuads * kStride];
-};
+using DcLds = ChainLds<kDcStep, kDcRows * TB>;
 
 struct DcMat {
   const float* w;     // rows kernel: [out][in]; down kernel: transposed [in][out]
@@ -98,33 +93,6 @@ __device__ __forceinline__ int64_t dc_row(const DcRows& a, int64_t at) {
   if (a.head_dim == 0) return a.rows[at];
   const int64_t h = at / a.head_dim;
   return a.rows[h] * a.head_dim + (at - h * a.head_dim);
-}
-
-// Eight producer waves and the consumer step through nch chunks: make(c, u) puts
-// chunk c's products (register slot u = c % kDcAhead) into LDS buffer c & 1 and
-// requests chunk c + kDcAhead.  The loop has no branch around a load (chunks past
-// the end are clamped, formed and not added): behind a branch the compiler waits
-// for every load in flight.
-template <int TB, typename Make>
-__device__ __forceinline__ float dc_run(DcLds<TB>& lds, int nch, float s0, Make make) {
-  const int lane = threadIdx.x & 63;
-  float s = s0;
-  if (threadIdx.x >= 64) {
-    for (int c0 = 0; c0 < nch; c0 += kDcAhead) {
-#pragma unroll
-      for (int u = 0; u < kDcAhead; ++u) {
-        make(c0 + u, u);
-        lds_barrier();
-      }
-    }
-  } else {
-    const int last = (nch + kDcAhead - 1) / kDcAhead * kDcAhead;
-    for (int c = 0; c < last; ++c) {
-      lds_barrier();
-      if (c < nch) s = chain_add_static<kDcQuads, DcLds<TB>::kStride>(&lds.q[c & 1][min(lane, kDcRows * TB - 1)], s);
-    }
-  }
-  return s;
 }
 
 // Four consecutive floats at p[k..k+3], k + i < n (others read p[n - 1]).
@@ -155,7 +123,7 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_rows_kernel(const DcRows 
   const float* __restrict__ xr[TB];
 #pragma unroll
   for (int t = 0; t < TB; ++t) xr[t] = a.x + min(b0 + t, a.batch - 1) * a.ldx;
-  float4 w[kDcAhead], x[kDcAhead][TB];
+  float4 w[kChainAhead], x[kChainAhead][TB];
   auto fetch = [&](int c, int u) {
     const int k = c * kDcStep + 4 * k4;
     w[u] = dc_load4<VEC>(wr, k, n);
@@ -164,9 +132,9 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_rows_kernel(const DcRows 
   };
   if (prod) {
 #pragma unroll
-    for (int u = 0; u < kDcAhead; ++u) fetch(u, u);
+    for (int u = 0; u < kChainAhead; ++u) fetch(u, u);
   }
-  float s = dc_run<TB>(lds, nch, -0.0f, [&](int c, int u) {
+  float s = chain_run(lds, nch, -0.0f, [&](int c, int u) {
     const int k = c * kDcStep + 4 * k4;
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
@@ -177,7 +145,7 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_rows_kernel(const DcRows 
       p.w = k + 3 < n ? w[u].w * x[u][t].w : -0.0f;
       lds.q[c & 1][k4 * DcLds<TB>::kStride + t * kDcRows + i] = p;
     }
-    fetch(c + kDcAhead, u);
+    fetch(c + kChainAhead, u);
   });
   if (threadIdx.x >= 64) return;
   const int64_t b = b0 + ((int)threadIdx.x >> 4);
@@ -209,9 +177,9 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_down_kernel(
   const float* __restrict__ hr[TB];
 #pragma unroll
   for (int t = 0; t < TB; ++t) hr[t] = h + min(b0 + t, batch - 1) * n;
-  int id[kDcAhead];                           // neuron of the chunk kDcAhead past the slot's
-  float4 w[kDcAhead];
-  float v[kDcAhead][TB];
+  int id[kChainAhead];                           // neuron of the chunk kChainAhead past the slot's
+  float4 w[kChainAhead];
+  float v[kChainAhead][TB];
   auto ids = [&](int c, int u) { id[u] = (int)sel[min(c * kDcStep + e, n - 1)]; };
   auto fetch = [&](int c, int u) {
     w[u] = dc_load4<VEC>(wdt + (size_t)id[u] * hidden, j0 + 4 * q, hidden);
@@ -220,13 +188,13 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_down_kernel(
   };
   if (prod && nch > 0) {
 #pragma unroll
-    for (int u = 0; u < kDcAhead; ++u) ids(u, u);
+    for (int u = 0; u < kChainAhead; ++u) ids(u, u);
 #pragma unroll
-    for (int u = 0; u < kDcAhead; ++u) fetch(u, u);
+    for (int u = 0; u < kChainAhead; ++u) fetch(u, u);
 #pragma unroll
-    for (int u = 0; u < kDcAhead; ++u) ids(u + kDcAhead, u);
+    for (int u = 0; u < kChainAhead; ++u) ids(u + kChainAhead, u);
   }
-  float s = dc_run<TB>(lds, nch, 0.0f, [&](int c, int u) {
+  float s = chain_run(lds, nch, 0.0f, [&](int c, int u) {
     float* dst = reinterpret_cast<float*>(&lds.q[c & 1][(e >> 2) * DcLds<TB>::kStride]) + (e & 3);
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
@@ -238,8 +206,8 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_down_kernel(
       d[8] = on ? w[u].z * v[u][t] : -0.0f;
       d[12] = on ? w[u].w * v[u][t] : -0.0f;
     }
-    fetch(c + kDcAhead, u);
-    ids(c + 2 * kDcAhead, u);
+    fetch(c + kChainAhead, u);
+    ids(c + 2 * kChainAhead, u);
   });
   const int lane = threadIdx.x;
   if (lane >= kDcRows * TB) return;
@@ -347,8 +315,8 @@ static unsigned grid_for(int64_t threads) {
 
 // Lists of up to kDlArgList indices travel in the launch itself: the caller's
 // list may be freed on return and nothing waits, where a copy from pageable host
-// memory made every call wait for its stream (f32 layer of 822 neurons and 6
-// heads, 3 tokens: see kh_dejavu_sparse_mlp_forward).  Longer lists are copied.
+// memory made every call wait for its stream (SparseMlp with 822 neurons, then
+// SparseAttention with 6 heads, 3 tokens: 61.8 -> 40.9 us).  Longer lists are copied.
 constexpr int kDlArgList = 960;
 struct DlList {
   int32_t v[kDlArgList];
