@@ -288,21 +288,26 @@ __global__ __launch_bounds__(kTrThreads) void tr_neuron_kernel(
 }
 
 // apply_softmax (layer.rs:286-308) over each row's active list (block r: rows
-// of `cap` entries, dense rows of dense_ld) in its order: max,
-// exp(z - max) with glibc's expf, the sequential sum (exact_seq_sum, 8192
-// terms a pass), then e / sum (or 1/n when the sum is not positive).  Lists
-// of up to 8192 stay in registers (32 per thread, all loads in flight);
-// longer ones go through `post` in passes.
-__global__ __launch_bounds__(kTrThreads) void tr_softmax_kernel(const float* __restrict__ pre,
+// of `cap` entries, dense rows of dense_ld) in its order: max, exp(z - max) with
+// glibc's expf, the sequential sum, then e / sum (or 1/n when the sum is not
+// positive).  Lists of up to kPass entries stay in registers (all loads in
+// flight); longer ones go through `post` in passes.  The sum: a plain chain of
+// adds up to kSmChain entries (2.5 us at 512), exact_seq_sum beyond.  Sixteen
+// waves, because the exps are double-precision chains: 4400 entries 16.0 -> 10.2 us
+// against four waves, 32 entries in 128 rows 21.6 -> 9.9 us.
+constexpr int kSmThreads = 1024;
+constexpr int kSmChain = 512;
+__global__ __launch_bounds__(kSmThreads) void tr_softmax_kernel(const float* __restrict__ pre,
                                                                 const uint32_t* __restrict__ aids,
                                                                 const int32_t* __restrict__ alen,
                                                                 int cap, float* __restrict__ post,
                                                                 float* __restrict__ dense,
                                                                 int64_t dense_ld) {
   constexpr int kPass = kSmCH * kSmM;
-  constexpr int kPer = kPass / kTrThreads;
+  constexpr int kPer = kPass / kSmThreads;
+  constexpr int kWaves = kSmThreads / 64;
   __shared__ EsLds<kSmCH, kSmM> es;
-  __shared__ float red[kTrThreads / 64];
+  __shared__ float red[kWaves];
   __shared__ uint64_t s_tab[32];  // kExp2Tab: the exps' table lookups stay in LDS
   const int64_t row = blockIdx.x;
   const int n = min(alen[row], cap);
@@ -316,10 +321,10 @@ __global__ __launch_bounds__(kTrThreads) void tr_softmax_kernel(const float* __r
   float mx = -INFINITY;
   if (n <= kPass) {
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) v[k] = pre[min(k * kTrThreads + static_cast<int>(threadIdx.x), n - 1)];
+    for (int k = 0; k < kPer; ++k) v[k] = pre[min(k * kSmThreads + static_cast<int>(threadIdx.x), n - 1)];
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
-      v[k] = k * kTrThreads + static_cast<int>(threadIdx.x) < n ? v[k] : -INFINITY;
+      v[k] = k * kSmThreads + static_cast<int>(threadIdx.x) < n ? v[k] : -INFINITY;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) mx = fmaxf(mx, v[k]);
   } else {
@@ -329,21 +334,31 @@ __global__ __launch_bounds__(kTrThreads) void tr_softmax_kernel(const float* __r
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
   __syncthreads();
   mx = red[0];
-  for (int i = 1; i < kTrThreads / 64; ++i) mx = fmaxf(mx, red[i]);
+  for (int i = 1; i < kWaves; ++i) mx = fmaxf(mx, red[i]);
   float s = -0.0f;
   if (n <= kPass) {
+    const bool chain = n <= kSmChain;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int a = k * kTrThreads + threadIdx.x;
+      const int a = k * kSmThreads + threadIdx.x;
       v[k] = a < n ? expf_glibc_t(v[k] - mx, s_tab) : -0.0f;
-      es.TP[es_slot<kSmCH, kSmM>(a)] = v[k];
+      if (!chain) es.TP[es_slot<kSmCH, kSmM>(a)] = v[k];
     }
-    __syncthreads();
-    s = exact_seq_sum<kTrThreads / 64, kSmCH, kSmM>(n, s, es);
+    if (chain) {
+      static_assert(kSmChain <= kSmThreads, "one term per thread");
+      if (threadIdx.x < kSmChain) es.TP[threadIdx.x] = v[0];   // -0.0 past n
+      __syncthreads();
+      const float4* q = reinterpret_cast<const float4*>(es.TP);
+#pragma unroll 1
+      for (int g = 0; g < n; g += 32) s = chain_add_static<8, 1>(q + g / 4, s);   // every wave: the same sum
+    } else {
+      __syncthreads();
+      s = exact_seq_sum<kWaves, kSmCH, kSmM>(n, s, es);
+    }
     const float u = 1.0f / static_cast<float>(n);
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int a = k * kTrThreads + threadIdx.x;
+      const int a = k * kSmThreads + threadIdx.x;
       if (a < n) {
         const float r = s > 0.0f ? v[k] / s : u;
         post[a] = r;
@@ -359,7 +374,7 @@ __global__ __launch_bounds__(kTrThreads) void tr_softmax_kernel(const float* __r
     for (int i = threadIdx.x; i < kPass; i += blockDim.x)
       es.TP[es_slot<kSmCH, kSmM>(i)] = i < cnt ? post[c0 + i] : -0.0f;
     __syncthreads();
-    s = exact_seq_sum<kTrThreads / 64, kSmCH, kSmM>(cnt, s, es);
+    s = exact_seq_sum<kWaves, kSmCH, kSmM>(cnt, s, es);
   }
   const float u = 1.0f / static_cast<float>(n);
   for (int a = threadIdx.x; a < n; a += blockDim.x) {
@@ -869,7 +884,7 @@ extern "C" int kh_slide_layer_backward(kh_slide_layer* l, const float* x_dev,
   if (!go || !lg || !post) return KH_ERR_ALLOC;
   if (l->act == KH_ACT_SOFTMAX) {
     // Layer::backward recomputes apply_softmax(pre_activations) (layer.rs:147)
-    hipLaunchKernelGGL(tr_softmax_kernel, dim3(1), dim3(kTrThreads), 0, st, pre_dev, act_ids_dev,
+    hipLaunchKernelGGL(tr_softmax_kernel, dim3(1), dim3(kSmThreads), 0, st, pre_dev, act_ids_dev,
                        n_act_dev, cap, post, nullptr, (int64_t)0);
     KH_LAUNCHED();
   }
@@ -1044,7 +1059,7 @@ static int net_forward_one(kh_slide_network* net, const float* x, hipStream_t st
                        t.nzi, t.nzv, t.xoff, t.aids, t.alen, t.as, l->act, t.pre, t.post, t.dense, (int64_t)0);
     KH_LAUNCHED();
     if (l->act == KH_ACT_SOFTMAX) {
-      hipLaunchKernelGGL(tr_softmax_kernel, dim3(1), dim3(kTrThreads), 0, st, t.pre, t.aids, t.alen,
+      hipLaunchKernelGGL(tr_softmax_kernel, dim3(1), dim3(kSmThreads), 0, st, t.pre, t.aids, t.alen,
                          t.as, t.post, t.dense, (int64_t)0);
       KH_LAUNCHED();
     }
@@ -1260,7 +1275,9 @@ static int net_predict_rows(kh_slide_network* net, const float* x_dev, const int
       if (rc != KH_OK) return rc;
       rc = query_launch(l->index, codes, nr, qids, qcnt, qs[i], qlen, st);
       if (rc != KH_OK) return rc;
-      rc = select_launch(l, qids, qcnt, qlen, qs[i], nr, aids, as[i], alen, true, nullptr, st);
+      // Only a softmax's sum depends on the list's order; elsewhere ascending ids,
+      // whose weights in a row of the transposed copy lie close together.
+      rc = select_launch(l, qids, qcnt, qlen, qs[i], nr, aids, as[i], alen, l->act == KH_ACT_SOFTMAX, nullptr, st);
       if (rc != KH_OK) return rc;
       float* dense = i + 1 < nl ? hidden[i & 1] : out_dev + e0 * net->out_dim;
       hipLaunchKernelGGL(fill_f32_kernel<>, dim3((unsigned)ceil_div(nr * l->n, 256)), dim3(256), 0, st, dense,
@@ -1279,7 +1296,7 @@ static int net_predict_rows(kh_slide_network* net, const float* x_dev, const int
                            nzoff, aids, alen, as[i], l->act, pre, post, dense, (int64_t)l->n);
       KH_LAUNCHED();
       if (l->act == KH_ACT_SOFTMAX) {
-        hipLaunchKernelGGL(tr_softmax_kernel, dim3((unsigned)nr), dim3(kTrThreads), 0, st, pre, aids, alen, as[i],
+        hipLaunchKernelGGL(tr_softmax_kernel, dim3((unsigned)nr), dim3(kSmThreads), 0, st, pre, aids, alen, as[i],
                            post, dense, (int64_t)l->n);
         KH_LAUNCHED();
       }
