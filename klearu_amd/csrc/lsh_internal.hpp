@@ -14,7 +14,6 @@ struct kh_hash_family {
   std::vector<uint32_t> perms_host;      // MinHash [L][dim]
   uint32_t* perms_dev = nullptr;
   std::vector<int8_t> planes_host;  // [L][k][dim]
-  int8_t* planes_dev = nullptr;     // [L*k][dim]
   // Nonzero lists of the planes, transposed so that the planes handled by
   // consecutive lanes are adjacent: entry j of plane p at ent_t[j*L*k + p],
   // (dim << 1) | (sign < 0), in dimension order; rows past a plane's nnz are 0.
@@ -25,11 +24,10 @@ struct kh_hash_family {
   // [ceil(dim/32)][ceil(L*k/16)][64 lanes] x 8 values; null otherwise.
   uint4* bt_dev = nullptr;
   int bt_ksteps = 0, bt_tiles = 0;
-  // 2-bit plane signs for the per-row LDS kernel (dim small enough to stage
-  // them): group g holds tables g*sg_tpb.. (planes q = 0..sg_tpb*k-1 of the
+  // 2-bit plane signs for the per-row kernels: group g holds tables g*sg_tpb.. (planes q = 0..sg_tpb*k-1 of the
   // group), as [dim][sg_words] words, plane q in bits 2(q%16), 2(q%16)+1 of
   // word q/16 (01 = +1, 11 = -1, 00 = no term); each group padded to sg_n4
-  // uint4.  Null when dim or k rule it out.
+  // uint4.  Null for the rank-based families.
   uint4* sg_dev = nullptr;
   int sg_tpb = 0, sg_groups = 0, sg_words = 0, sg_n4 = 0;
 };
@@ -71,6 +69,8 @@ int hash_sparse_launch(const kh_hash_family* h, const int64_t* xoff, const uint3
 int query_launch(const kh_lsh_index* idx, const uint32_t* qcodes, int64_t batch, uint32_t* qids,
                  uint32_t* qcnt, int stride, int32_t* ulen, hipStream_t st);
 int query_stride(const kh_lsh_index* idx);
+// Whether short dense batches hash with their signs staged in LDS.
+bool hash_dense_rows(const kh_hash_family* h);
 // The rank-based families (hash_rank.hip), called by the two launchers above.
 int rank_hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx, int64_t batch,
                            uint32_t* codes, hipStream_t st);

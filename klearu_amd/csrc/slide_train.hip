@@ -1269,7 +1269,7 @@ static int net_predict_rows(kh_slide_network* net, const float* x_dev, const int
         hipLaunchKernelGGL(tr_stage_csr_kernel, dim3((unsigned)nr), dim3(1024), 0, st, xoff, xidx, xval, e0,
                            l->dim, stride, nzi, nzv, nzoff, (float*)nullptr);
       KH_LAUNCHED();
-      int rc = in && h->kind == KH_FAMILY_TERNARY && h->sg_dev
+      int rc = in && hash_dense_rows(h)
                    ? hash_dense_launch(h, in, l->dim, nr, codes, st)
                    : hash_sparse_launch(h, nzoff, nzi, nzv, nr, codes, st, 2);
       if (rc != KH_OK) return rc;
