@@ -97,14 +97,20 @@ __device__ int select_topk_count_order(const uint32_t* __restrict__ ids,
 // clear_dense (training): the row's dense activation vector [num_neurons];
 // the entries of the previous active list (aids/alen still hold it) are
 // zeroed before the new list is written.  count_order: top-k picks in the
-// sampler's order instead of ascending ids.
-__global__ __launch_bounds__(kSlideThreads) void select_kernel(
+// sampler's order instead of ascending ids.  ids_below: every candidate id is
+// below num_neurons, so a selection of all candidates is a copy of the list
+// (one row of 4470 candidates: 3.4 us; 15 when each thread walked its own run
+// of them twice, with 256 threads).
+constexpr int kSelectThreads = 1024;       // rows up to kSelectFewRows; kSlideThreads beyond
+constexpr int64_t kSelectFewRows = 256;
+__global__ __launch_bounds__(kSelectThreads) void select_kernel(
     const uint32_t* __restrict__ qids, const uint32_t* __restrict__ qcnt,
     const int32_t* __restrict__ qlen, int qstride, int sampling, int top_k, int threshold,
     int num_neurons, int nbins, uint32_t* __restrict__ aids, int astride,
-    int32_t* __restrict__ alen, int count_order, float* __restrict__ clear_dense, int fallback) {
+    int32_t* __restrict__ alen, int count_order, float* __restrict__ clear_dense, int fallback,
+    int ids_below) {
   extern __shared__ unsigned hist[];
-  __shared__ int wsum[kSlideThreads / 64];
+  __shared__ int wsum[kSelectThreads / 64];
   __shared__ int s_total;
   __shared__ int s_cstar, s_take, s_best_id;
   const int64_t row = blockIdx.x;
@@ -115,7 +121,14 @@ __global__ __launch_bounds__(kSlideThreads) void select_kernel(
   if (clear_dense) {
     float* dn = clear_dense + row * (int64_t)num_neurons;
     const int old = alen[row];
-    for (int a = threadIdx.x; a < old; a += blockDim.x) dn[out[a]] = 0.0f;
+    constexpr int U = 4;
+    for (int a = threadIdx.x; a < old; a += blockDim.x * U) {
+      uint32_t id[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) id[u] = out[min(a + u * (int)blockDim.x, old - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) dn[id[u]] = 0.0f;
+    }
     __syncthreads();
   }
   int cstar = 0, take_eq = 0;  // topk: take count > cstar, plus take_eq of count == cstar
@@ -171,7 +184,17 @@ __global__ __launch_bounds__(kSlideThreads) void select_kernel(
   // n_pre counts the sampler's picks before ids >= num_neurons are dropped:
   // the all-neurons fallback (layer.rs:82-84) runs before that filter (:87).
   int n_sel = 0, n_pre = 0;
-  if (mode == KH_SAMPLING_THRESHOLD) {
+  if (mode == KH_SAMPLING_VANILLA && ids_below) {
+    constexpr int U = 4;
+    for (int i = threadIdx.x; i < m; i += blockDim.x * U) {
+      uint32_t id[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) id[u] = ids[min(i + u * (int)blockDim.x, m - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) out[min(i + u * (int)blockDim.x, m - 1)] = id[u];
+    }
+    n_sel = n_pre = m;
+  } else if (mode == KH_SAMPLING_THRESHOLD) {
     int base = 0, passed = 0;
     for (int c0 = 0; c0 < m; c0 += blockDim.x) {
       const int i = c0 + threadIdx.x;
@@ -385,17 +408,20 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
 // whose odd row stride makes the per-lane column reads conflict-free; lane j
 // then runs neuron j's sequential sum over the input's nonzeros (ascending, as
 // neuron_kernel does).  The next tile's loads are in flight during the sums.
+// With several blocks per row (gridDim.y) the tiles are dealt over them and a
+// softmax layer's activations are left to another kernel; `dense`, when given,
+// also gets the activations at their ids.
 constexpr int kTileN = 64;
 constexpr int kTileStride = 129;   // floats per LDS row
 constexpr int kTileMaxDim = 128;
-constexpr int kTileWaves = kSlideThreads / 64;
-constexpr size_t kTileLds = sizeof(float) * kTileWaves * kTileN * kTileStride;
+constexpr int kTileWaves = kSlideThreads / 64;   // waves per block at most (two at least)
+constexpr size_t tile_lds(int waves) { return sizeof(float) * waves * kTileN * kTileStride; }
 
 __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     const float* __restrict__ W, const float* __restrict__ bias, int dim, const float* __restrict__ x,
     uint32_t* __restrict__ aids, int astride, const int32_t* __restrict__ alen, int act,
     float* __restrict__ pre, float* __restrict__ post, int fb_n = 0,
-    int32_t* __restrict__ alen_out = nullptr) {
+    int32_t* __restrict__ alen_out = nullptr, float* __restrict__ dense = nullptr, int64_t dense_ld = 0) {
   extern __shared__ float tl[];
   __shared__ uint32_t nzi[kTileMaxDim];
   __shared__ float nzv[kTileMaxDim];
@@ -403,8 +429,9 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
   __shared__ int s_total;
   __shared__ float red[kTileWaves];
   const int64_t row = blockIdx.x;
+  const int waves = blockDim.x >> 6;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // the input's nonzeros in ascending order (dim <= kSlideThreads)
+  // the input's nonzeros in ascending order (dim <= blockDim.x)
   {
     const float v = (int)threadIdx.x < dim ? x[row * (int64_t)dim + threadIdx.x] : 0.0f;
     const int nz = v != 0.0f ? 1 : 0;
@@ -421,8 +448,8 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
   uint32_t* ids = aids + row * (int64_t)astride;
   float* prow = pre + row * (int64_t)astride;
   float* orow = post + row * (int64_t)astride;
-  if (alen_out && threadIdx.x == 0) alen_out[row] = n;
-  if (all)
+  if (alen_out && blockIdx.y == 0 && threadIdx.x == 0) alen_out[row] = n;
+  if (all && blockIdx.y == 0)
     for (int a = threadIdx.x; a < n; a += blockDim.x) ids[a] = (uint32_t)a;
   float* buf = tl + (size_t)wave * kTileN * kTileStride;
   const int q4 = dim >> 2;              // float4 per weight row (<= 32)
@@ -441,9 +468,10 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     }
   };
   float lmax = -INFINITY;
-  int t = wave;
+  int t = (int)blockIdx.y * waves + wave;
+  const int tstep = (int)gridDim.y * waves;
   if (t < ntiles) issue(t);
-  for (; t < ntiles; t += kTileWaves) {
+  for (; t < ntiles; t += tstep) {
     // the tile to LDS (column 4c..4c+3 of row 2r + half)
     if (c < q4) {
 #pragma unroll
@@ -455,13 +483,14 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
         dst[3] = v[r].w;
       }
     }
-    if (t + kTileWaves < ntiles) issue(t + kTileWaves);
+    if (t + tstep < ntiles) issue(t + tstep);
     const int a = t * kTileN + lane;
     const float* wr = buf + lane * kTileStride;
     float s = -0.0f;
     for (int e = 0; e < nnz; ++e) s = __fadd_rn(s, __fmul_rn(wr[nzi[e]], nzv[e]));
     if (a < n) {
-      const float z = __fadd_rn(s, bias[all ? (uint32_t)a : ids[a]]);
+      const uint32_t id = all ? (uint32_t)a : ids[a];
+      const float z = __fadd_rn(s, bias[id]);
       prow[a] = z;
       lmax = fmaxf(lmax, z);
       if (act != KH_ACT_SOFTMAX) {
@@ -471,10 +500,11 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
         else if (act == KH_ACT_TANH) r = tanhf(z);
         else r = z;
         orow[a] = r;
+        if (dense) dense[row * dense_ld + id] = r;
       }
     }
   }
-  if (act != KH_ACT_SOFTMAX) return;
+  if (act != KH_ACT_SOFTMAX || gridDim.y > 1) return;
   // softmax over the active set (layer.rs:286-308), as neuron_kernel
   lmax = wave_max(lmax);
   if (lane == 0) red[wave] = lmax;
@@ -507,10 +537,29 @@ static int tile_kernel_ready() {
   static int rc = KH_OK;
   std::call_once(once, [] {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(&neuron_tile_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds) != hipSuccess)
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)tile_lds(kTileWaves)) != hipSuccess)
       rc = KH_ERR_HIP;
   });
   return rc;
+}
+
+bool neuron_tile_ok(const kh_slide_layer* l) {
+  return l->dim <= kTileMaxDim && l->dim % 4 == 0 && tile_kernel_ready() == KH_OK;
+}
+
+// Two waves a block (a tile each): the few tiles of a short batch spread over as
+// many CUs as there are.  At least two blocks a row, so a softmax stays undone.
+int neuron_tile_launch(const kh_slide_layer* l, const float* x, int64_t rows, uint32_t* aids, int as,
+                       const int32_t* alen, float* pre, float* post, float* dense, int64_t dense_ld,
+                       hipStream_t st) {
+  constexpr int kFew = 2;
+  const int tiles = ceil_div(as, kTileN * kFew);
+  const int split = std::max(2, std::min(tiles, std::max(1, 1024 / (int)std::min<int64_t>(rows, 1024))));
+  hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)rows, (unsigned)split), dim3(64 * kFew), tile_lds(kFew), st,
+                     l->w, l->bias, l->dim, x, aids, as, alen, l->act, pre, post, 0, (int32_t*)nullptr, dense,
+                     dense_ld);
+  KH_LAUNCHED();
+  return KH_OK;
 }
 
 // Dense layer over CSR inputs: y[b][o] = act(sum_e val_e * W^T[idx_e][o] + bias[o]).
@@ -561,10 +610,12 @@ int select_launch_with(const kh_lsh_index* idx, int sampling, int top_k, int thr
   const int nbins = idx->L * idx->cap + 1;
   KH_CHECK_ARG(sampling != KH_SAMPLING_TOPK || nbins <= kMaxCountBins,
                "top-k sampling supports num_tables * bucket_capacity <= %d", kMaxCountBins - 1);
-  hipLaunchKernelGGL(select_kernel, dim3((unsigned)batch), dim3(kSlideThreads),
+  hipLaunchKernelGGL(select_kernel, dim3((unsigned)batch),
+                     dim3(batch <= kSelectFewRows ? kSelectThreads : kSlideThreads),
                      sampling == KH_SAMPLING_TOPK ? sizeof(unsigned) * nbins : 0, st, qids, qcnt,
                      qlen, qs, sampling, top_k, threshold, num_neurons, nbins, aids, as, alen,
-                     count_order ? 1 : 0, clear_dense, fallback ? 1 : 0);
+                     count_order ? 1 : 0, clear_dense, fallback ? 1 : 0,
+                     idx->id_bound <= (uint32_t)num_neurons ? 1 : 0);
   KH_LAUNCHED();
   return KH_OK;
 }
@@ -727,7 +778,7 @@ static int slide_forward_common(const kh_slide_layer* lc, const float* x, const 
                        l->bias, l->dim, x, nullptr, nullptr, nullptr, aids, as, ilen, act,
                        max_nz, pre, post, fb_n, olen);
   else if (l->dim <= kTileMaxDim && l->dim % 4 == 0 && tile_kernel_ready() == KH_OK)
-    hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)batch), dim3(kSlideThreads), kTileLds, st, l->w,
+    hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)batch), dim3(kSlideThreads), tile_lds(kTileWaves), st, l->w,
                        l->bias, l->dim, x, aids, as, ilen, act, pre, post, fb_n, olen);
   else
     hipLaunchKernelGGL((neuron_kernel<false, false>), ng, dim3(kSlideThreads), lds, st, l->w, l->n,

@@ -47,4 +47,12 @@ int select_launch_with(const kh_lsh_index* idx, int sampling, int top_k, int thr
                        int32_t* alen, bool count_order, float* clear_dense, bool fallback,
                        hipStream_t st);
 
+// Neuron sums of listed active neurons over dense input rows (rows of `as` list
+// entries; not the softmax), for layers neuron_tile_ok takes: pre, and for other
+// activations post and the dense activation rows.
+bool neuron_tile_ok(const kh_slide_layer* l);
+int neuron_tile_launch(const kh_slide_layer* l, const float* x, int64_t rows, uint32_t* aids, int as,
+                       const int32_t* alen, float* pre, float* post, float* dense, int64_t dense_ld,
+                       hipStream_t st);
+
 }  // namespace kh
