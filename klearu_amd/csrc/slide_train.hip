@@ -35,7 +35,6 @@ constexpr int kTrThreads = 256;
 constexpr int kTrMaxLabels = 1024;   // labels of one example
 constexpr int kTrLdsNz = 8192;       // staged input nonzeros at most (beyond: read from global)
 constexpr int kTrMaxNnz = 4096;      // stored entries of one sparse example
-constexpr int kGTile = 1024;         // grad_input: (id, lg) pairs per LDS tile
 constexpr int kSmCH = 64, kSmM = 128;  // exact softmax sum: 8192 terms per pass
 
 struct OptArgs {
@@ -430,125 +429,78 @@ __global__ __launch_bounds__(kTrThreads) void tr_loss_grad_kernel(
   }
 }
 
-// nq quads (a multiple of 8) as a loop over groups: the next group is read
-// into a second set of registers while the current one is added, then copied
-// over (measured faster than the copy-free pair loop for the long grad_input
-// chains).
-template <int C>
-__device__ __forceinline__ float chain_add_quads(const float4* base, int nq, float r) {
-  float4 v[8];
-#pragma unroll
-  for (int b = 0; b < 8; ++b) v[b] = base[b * C];
-  for (int g = 0; g < nq; g += 8) {
-    const float4* nb = base + min(g + 8, nq - 8) * C;  // the last group re-reads itself
-    float4 nv[8];
-#pragma unroll
-    for (int b = 0; b < 8; ++b) nv[b] = nb[b * C];
-    __builtin_amdgcn_sched_barrier(0);
-    r = add_quads8(v, r);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) v[b] = nv[b];
-  }
-  return r;
-}
-
 // The softmax branch of Layer::backward (layer.rs:141-175): output i's local
 // gradient is the sequential sum over j (from +0.0) of go_j*s_j*(1-s_j) when
-// j == i, else go_j*(-s_i*s_j).  A block owns 64 outputs, one chain per lane
-// of wave 0 (the consumer).  The terms depend on (i, j) through two rounded
-// products each, so waves 1..3 form them into LDS one chunk of kJStep steps
-// ahead of the consumer, whose only work per step is the dependent add (four
-// steps per LDS read); wave 4 loads the (s, go) pairs two chunks ahead into a
-// ring of three LDS slots, so no other wave waits on global memory.  Blocks
-// loop over groups of 64 outputs.
-constexpr int kJc = 64;                      // chains per block
-constexpr int kJStep = 96;                   // steps per chunk
-constexpr int kJProd = 3;                    // producer waves
-constexpr int kJThreads = 64 * (2 + kJProd); // consumer, producers, loader
-constexpr int kJBlocks = 256;                // grid (groups of 64 outputs are strided over it)
-static_assert((kJStep / 4) % kJProd == 0 && (kJStep / 4) % 8 == 0 && kJStep <= 128, "chunk layout");
+// j == i, else go_j*(-s_i*s_j).  The chain of n dependent adds bounds it.  A block
+// owns 32 outputs, one chain per lane of wave 0; the terms, two rounded products
+// each, are formed in LDS by six waves, which read (s, go) straight into registers
+// kJAhead chunks early.  Wave 4 only keeps the barriers: a block's waves go to the
+// SIMDs in turn, so wave 0 shares its SIMD with no producer.  Half a wave of
+// chains per block halves the LDS traffic per CU (64 chains would move 96 KB a
+// chunk, as long as the adds take) and spreads a list over more CUs.  Steps past
+// the list are -0.0, so the last chunk needs no loop of its own.
+// 4470 outputs: 16.4 us; 32.5 with 64 chains, three producer waves and a loader
+// wave.
+constexpr int kJc = 32;                      // chains per block
+constexpr int kJStep = 192;                  // steps per chunk
+constexpr int kJProd = 6;                    // producer waves (1-3 and 5-7)
+constexpr int kJThreads = 512;
+constexpr int kJAhead = 2;
+constexpr int kJPer = kJStep / 4 / (2 * kJProd);   // quads per producer half wave and chunk
+constexpr int kJBlocks = 256;                // grid (groups of 32 outputs are strided over it)
+static_assert(kJPer * 2 * kJProd * 4 == kJStep, "whole quads per producer");
+constexpr int kJPad = 4;                     // floats past a list that the quad loads may touch
 
 __device__ __forceinline__ float jac_off(float gj, float sj, float nsi) { return gj * (nsi * sj); }
 
 __global__ __launch_bounds__(kJThreads) void tr_softmax_jacobian_kernel(
     const float* __restrict__ s, const float* __restrict__ go, const int32_t* __restrict__ alen,
     int cap, float* __restrict__ lg) {
-  __shared__ float4 jb[2][kJStep / 4][kJc];    // two chunks of terms, [step/4][chain]
-  __shared__ float4 ring[3][2][kJStep / 4];    // (s, go) of three chunks
+  using Lds = ChainLds<kJStep, kJc>;
+  __shared__ Lds lds;
   const int n = min(alen[0], cap);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nch = (n + kJStep - 1) / kJStep;
-  const int p = wave - 1;                      // producer index (waves 1..kJProd)
-  const bool prod = wave >= 1 && wave <= kJProd, loader = wave == kJProd + 1;
-  // loader: chunk c's (s, go) into ring slot c % 3 (past n: the last pair,
-  // formed but never added)
-  auto load = [&](int c) {
-    float* rs = reinterpret_cast<float*>(&ring[c % 3][0][0]);
-    float* rg = reinterpret_cast<float*>(&ring[c % 3][1][0]);
-    for (int k = lane; k < kJStep; k += 64) {
-      const int j = min(c * kJStep + k, n - 1);
-      rs[k] = s[j];
-      rg[k] = go[j];
-    }
-  };
+  const bool prod = wave != 0 && wave != 4;
+  const int p = 2 * (wave < 4 ? wave - 1 : wave - 2) + (lane >> 5);  // producer half wave
   for (int i0 = blockIdx.x * kJc; i0 < n; i0 += gridDim.x * kJc) {
-    const int i = min(i0 + lane, n - 1);
+    const int i = min(i0 + (lane & (kJc - 1)), n - 1);
     const float si = s[i], gi = go[i];
     const float nsi = -si;
     const float dterm = (gi * si) * (1.0f - si);  // the diagonal term, j == i
-    // producer p forms quads p, p + kJProd, ... of chunk c
-    auto produce = [&](int c) {
-      const int jc = c * kJStep;
-      const bool diag = jc < i0 + kJc && i0 < jc + kJStep;  // the chunk meets this block's diagonal
-      constexpr int kQ = kJStep / 4 / kJProd;
-      float4 sv[kQ], gv[kQ];
+    float4 sv[kJAhead][kJPer], gv[kJAhead][kJPer];
+    // quads p, p + 2 kJProd, ... of chunk c (past the list: its last quad)
+    auto fetch = [&](int c, int u) {
 #pragma unroll
-      for (int u = 0; u < kQ; ++u) {
-        sv[u] = ring[c % 3][0][p + kJProd * u];
-        gv[u] = ring[c % 3][1][p + kJProd * u];
-      }
-#pragma unroll
-      for (int u = 0; u < kQ; ++u) {
-        const int q = p + kJProd * u;
-        float t0 = jac_off(gv[u].x, sv[u].x, nsi), t1 = jac_off(gv[u].y, sv[u].y, nsi);
-        float t2 = jac_off(gv[u].z, sv[u].z, nsi), t3 = jac_off(gv[u].w, sv[u].w, nsi);
-        if (diag) {
-          const int d = i0 + lane - (jc + 4 * q);
-          t0 = d == 0 ? dterm : t0;
-          t1 = d == 1 ? dterm : t1;
-          t2 = d == 2 ? dterm : t2;
-          t3 = d == 3 ? dterm : t3;
-        }
-        jb[c & 1][q][lane] = make_float4(t0, t1, t2, t3);
+      for (int e = 0; e < kJPer; ++e) {
+        const int q = min(c * (kJStep / 4) + p + 2 * kJProd * e, (n - 1) / 4);
+        sv[u][e] = reinterpret_cast<const float4*>(s)[q];
+        gv[u][e] = reinterpret_cast<const float4*>(go)[q];
       }
     };
-    float r = 0.0f;
-    lds_barrier();  // the previous group's last chunk is consumed
-    if (loader) {
-      load(0);
-      if (nch > 1) load(1);
+    lds_barrier();  // the group before is consumed
+    if (prod) {
+#pragma unroll
+      for (int u = 0; u < kJAhead; ++u) fetch(u, u);
     }
-    lds_barrier();
-    if (prod) produce(0);
-    lds_barrier();
-    for (int c = 0; c < nch; ++c) {
-      if (prod) {
-        if (c + 1 < nch) produce(c + 1);
-      } else if (loader) {
-        if (c + 2 < nch) load(c + 2);
-      } else if (wave == 0) {
-        const int cnt = min(kJStep, n - c * kJStep);
-        const float4(*src)[kJc] = jb[c & 1];
-        if (cnt == kJStep) {
-          r = chain_add_static<kJStep / 4, kJc>(&src[0][lane], r);
-        } else {
-          const float* sf = reinterpret_cast<const float*>(&src[0][0]);
-          for (int j = 0; j < cnt; ++j) r = r + sf[((j >> 2) * kJc + lane) * 4 + (j & 3)];
-        }
+    const float r = chain_run<kJAhead>(lds, nch, 0.0f, [&](int c, int u) {
+#pragma unroll
+      for (int e = 0; e < kJPer; ++e) {
+        const int q = p + 2 * kJProd * e;
+        const int j = c * kJStep + 4 * q;
+        const int d = i0 + (lane & (kJc - 1)) - j;   // step of the diagonal
+        const float4 a = sv[u][e], g = gv[u][e];
+        float4 t = make_float4(jac_off(g.x, a.x, nsi), jac_off(g.y, a.y, nsi), jac_off(g.z, a.z, nsi),
+                               jac_off(g.w, a.w, nsi));
+        t.x = d == 0 ? dterm : j < n ? t.x : -0.0f;
+        t.y = d == 1 ? dterm : j + 1 < n ? t.y : -0.0f;
+        t.z = d == 2 ? dterm : j + 2 < n ? t.z : -0.0f;
+        t.w = d == 3 ? dterm : j + 3 < n ? t.w : -0.0f;
+        lds.q[c & 1][q * Lds::kStride + (lane & (kJc - 1))] = t;
       }
-      lds_barrier();
-    }
-    if (wave == 0 && i0 + lane < n) lg[i0 + lane] = r;
+      fetch(c + kJAhead, u);
+    }, wave == 4);
+    if (wave == 0 && lane < kJc && i0 + lane < n) lg[i0 + lane] = r;
   }
 }
 
@@ -574,92 +526,63 @@ __global__ __launch_bounds__(kTrThreads) void tr_local_grad_kernel(
 
 // grad_input[j] = sum over the active list (in order, from +0.0) of
 // lg[a] * w[id_a][j], with the weights before this example's update
-// (layer.rs:203-207).  Each j is one chain of |A| dependent adds.  A block owns
-// kGc columns, one chain per lane of wave 0 (the consumer); waves 1..7 gather
-// the products for the next kGStep active rows into LDS (16 lanes read one
-// 64-byte piece of a weight row) while the consumer adds the current ones,
-// four per LDS read.
+// (layer.rs:203-207).  Each j is one chain of |A| dependent adds; a block owns
+// kGc columns, one chain per lane of wave 0, and the other waves gather the
+// products of kGStep active rows a chunk into LDS, kGAhead chunks of row pieces
+// (and the ids of as many more) in flight: 16 blocks at 128 columns have to pull
+// the rows at the chains' pace.  4470 rows of 128: 17.0 us, 25.5 with
+// 1024-row chunks and one chunk in flight.
+// VEC: dim a multiple of 4.
 constexpr int kGc = 8;          // columns (chains) per block
-constexpr int kGStep = 1024;    // active rows per chunk
-constexpr int kGThreads = 512;
+constexpr int kGStep = 128;     // active rows per chunk
+constexpr int kGAhead = 8;
+constexpr int kGThreads = 64 + kGStep * (kGc / 4);
 
+template <bool VEC>
 __global__ __launch_bounds__(kGThreads) void tr_grad_input_kernel(
     const float* __restrict__ W, int dim, const uint32_t* __restrict__ aids,
     const int32_t* __restrict__ alen, int cap, const float* __restrict__ lg,
     float* __restrict__ gi) {
-  __shared__ float4 gb[2][kGStep / 4][kGc];   // two chunks of products, [row/4][column]
-  constexpr int kProdThreads = kGThreads - 64;
-  constexpr int kSlots = kProdThreads / kGc;  // rows gathered per producer pass
-  constexpr int kPer = (kGStep + kSlots - 1) / kSlots;
+  using Lds = ChainLds<kGStep, kGc>;
+  __shared__ Lds lds;
   const int n = min(alen[0], cap);
   const int j0 = blockIdx.x * kGc;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nch = (n + kGStep - 1) / kGStep;
-  const int pt = static_cast<int>(threadIdx.x) - 64;   // producer thread
-  const int col = pt & (kGc - 1), slot = pt / kGc;
-  const int jc = min(j0 + col, dim - 1);
-  // A producer holds the weights and local gradients of the next chunk and
-  // the row ids of the one after (unconditional loads of clamped rows, all in
-  // flight at once), so each load has a chunk's worth of adds to arrive in.
-  uint32_t id[kPer];
-  float l[kPer], w[kPer], ln[kPer];
-  auto fetch_ids = [&](int c) {
-    const int r0 = c * kGStep;
-    const int cnt = min(kGStep, n - r0);
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int a = r0 + min(slot + u * kSlots, cnt - 1);
-      id[u] = aids[a];
-      ln[u] = lg[a];
-    }
+  const bool prod = threadIdx.x >= 64;
+  const int pt = static_cast<int>(threadIdx.x) - 64;
+  const int q = pt & (kGc / 4 - 1), e = pt / (kGc / 4);   // column quad, row within the chunk
+  const int jq = j0 + 4 * q;
+  uint32_t id[kGAhead];                                   // row of the chunk kGAhead past the slot's
+  float4 w[kGAhead];
+  float l[kGAhead];
+  auto ids = [&](int c, int u) { id[u] = aids[min(c * kGStep + e, n - 1)]; };
+  auto fetch = [&](int c, int u) {
+    const float* __restrict__ r = W + static_cast<size_t>(id[u]) * dim;
+    if constexpr (VEC)
+      w[u] = *reinterpret_cast<const float4*>(r + min(jq, dim - 4));
+    else
+      w[u] = make_float4(r[min(jq, dim - 1)], r[min(jq + 1, dim - 1)], r[min(jq + 2, dim - 1)], r[min(jq + 3, dim - 1)]);
+    l[u] = lg[min(c * kGStep + e, n - 1)];
   };
-  auto fetch_w = [&]() {
+  if (prod && nch > 0) {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      w[u] = W[static_cast<size_t>(id[u]) * dim + jc];
-      l[u] = ln[u];
-    }
-  };
-  auto produce = [&](int c) {
-    float wc[kPer], lc[kPer];
+    for (int u = 0; u < kGAhead; ++u) ids(u, u);
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      wc[u] = w[u];
-      lc[u] = l[u];
-    }
-    if (c + 1 < nch) fetch_w();           // chunk c + 1 (its ids arrived a chunk ago)
-    if (c + 2 < nch) fetch_ids(c + 2);
-    float* dst = reinterpret_cast<float*>(&gb[c & 1][0][0]);
+    for (int u = 0; u < kGAhead; ++u) fetch(u, u);
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int rr = slot + u * kSlots;
-      if (rr < kGStep) dst[((rr >> 2) * kGc + col) * 4 + (rr & 3)] = lc[u] * wc[u];
-    }
-  };
-  if (wave > 0 && nch > 0) {
-    fetch_ids(0);
-    fetch_w();
-    if (nch > 1) fetch_ids(1);
-    produce(0);
+    for (int u = 0; u < kGAhead; ++u) ids(u + kGAhead, u);
   }
-  lds_barrier();
-  float r = 0.0f;
-  for (int c = 0; c < nch; ++c) {
-    if (wave > 0) {
-      if (c + 1 < nch) produce(c + 1);
-    } else if (lane < kGc) {
-      const int cnt = min(kGStep, n - c * kGStep);
-      const float4(*src)[kGc] = gb[c & 1];
-      if (cnt == kGStep) {
-        r = chain_add_quads<kGc>(&src[0][lane], kGStep / 4, r);
-      } else {
-        const float* sf = reinterpret_cast<const float*>(&src[0][0]);
-        for (int j = 0; j < cnt; ++j) r = r + sf[((j >> 2) * kGc + lane) * 4 + (j & 3)];
-      }
-    }
-    lds_barrier();
-  }
-  if (wave == 0 && lane < kGc && j0 + lane < dim) gi[j0 + lane] = r;
+  const float r = chain_run<kGAhead>(lds, nch, 0.0f, [&](int c, int u) {
+    const bool on = c * kGStep + e < n;
+    float* d = reinterpret_cast<float*>(&lds.q[c & 1][(e >> 2) * Lds::kStride + 4 * q]) + (e & 3);
+    d[0] = on ? l[u] * w[u].x : -0.0f;
+    d[4] = on ? l[u] * w[u].y : -0.0f;
+    d[8] = on ? l[u] * w[u].z : -0.0f;
+    d[12] = on ? l[u] * w[u].w : -0.0f;
+    fetch(c + kGAhead, u);
+    ids(c + 2 * kGAhead, u);
+  });
+  if (threadIdx.x < kGc && j0 + static_cast<int>(threadIdx.x) < dim) gi[j0 + threadIdx.x] = r;
 }
 
 // Optimizer::update of every active neuron (layer.rs:209-222): grad_weights[j]
@@ -717,8 +640,8 @@ static int layer_backward_launch(kh_slide_layer* l, const float* x, const uint32
     KH_LAUNCHED();
   }
   if (gi) {
-    hipLaunchKernelGGL(tr_grad_input_kernel, dim3((unsigned)ceil_div(l->dim, kGc)), dim3(kGThreads), 0, st,
-                       l->w, l->dim, aids, alen, cap, lg, gi);
+    hipLaunchKernelGGL((l->dim % 4 == 0 ? tr_grad_input_kernel<true> : tr_grad_input_kernel<false>),
+                       dim3((unsigned)ceil_div(l->dim, kGc)), dim3(kGThreads), 0, st, l->w, l->dim, aids, alen, cap, lg, gi);
     KH_LAUNCHED();
   }
   const int xs = ceil_div(l->dim, kUCols);
@@ -878,9 +801,9 @@ extern "C" int kh_slide_layer_backward(kh_slide_layer* l, const float* x_dev,
   // An active list holds distinct neuron ids, so at most n entries.
   const int cap = l->n;
   WsSet* w = l->ws.get(st);
-  float* go = static_cast<float*>(w->get(0, sizeof(float) * cap));
+  float* go = static_cast<float*>(w->get(0, sizeof(float) * (cap + kJPad)));
   float* lg = static_cast<float*>(w->get(1, sizeof(float) * cap));
-  float* post = static_cast<float*>(w->get(2, sizeof(float) * cap));
+  float* post = static_cast<float*>(w->get(2, sizeof(float) * (cap + kJPad)));
   if (!go || !lg || !post) return KH_ERR_ALLOC;
   if (l->act == KH_ACT_SOFTMAX) {
     // Layer::backward recomputes apply_softmax(pre_activations) (layer.rs:147)
@@ -983,9 +906,9 @@ extern "C" int kh_slide_network_create(kh_slide_layer* const* layers, int n_laye
     t.aids = net->alloc<uint32_t>(t.as, true);
     t.alen = net->alloc<int32_t>(1, true);
     t.pre = net->alloc<float>(t.as);
-    t.post = net->alloc<float>(t.as);
+    t.post = net->alloc<float>(t.as + kJPad);
     t.dense = net->alloc<float>(l->n, true);
-    t.go = net->alloc<float>(t.as);
+    t.go = net->alloc<float>(t.as + kJPad);
     t.lg = net->alloc<float>(t.as);
     t.gi = net->alloc<float>(l->dim);
     t.nzi = net->alloc<uint32_t>(l->dim);
@@ -1049,7 +972,8 @@ static int net_forward_one(kh_slide_network* net, const float* x, hipStream_t st
                          t.nzi, t.nzv, t.xoff);
       KH_LAUNCHED();
     }
-    int rc = hash_sparse_launch(l->index->h, t.xoff, t.nzi, t.nzv, 1, t.codes, st);
+    int rc = tile ? hash_dense_launch(l->index->h, in, l->dim, 1, t.codes, st)
+                  : hash_sparse_launch(l->index->h, t.xoff, t.nzi, t.nzv, 1, t.codes, st);
     if (rc != KH_OK) return rc;
     const int qs = query_stride(l->index);
     rc = query_launch(l->index, t.codes, 1, t.qids, t.qcnt, qs, t.qlen, st);
