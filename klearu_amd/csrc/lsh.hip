@@ -15,9 +15,8 @@
 // Large dense batches (index builds and rebuilds) hash on the matrix cores
 // instead: x is split into BF16 hi + lo terms, the ternary planes are exact in
 // BF16, and v_mfma_f32_16x16x32_bf16 gives every (row, plane) sum S' with
-// |S' - S| and |s_seq - S| both below a bound c * sum|x| (S the exact sum,
-// s_seq the reference's sequential f32 sum).  Where |S'| exceeds twice that
-// bound the sign of s_seq is the sign of S'; every other (row, plane) -- ties
+// |S' - S| + |s_seq - S| below a bound c * sum|x| (S the exact sum, s_seq the
+// reference's sequential f32 sum).  Where |S'| exceeds that bound the sign of s_seq is the sign of S'; every other (row, plane) -- ties
 // near zero, non-finite input -- replays the sequential sum in its lane, so
 // codes stay bit-identical.
 //
@@ -294,7 +293,7 @@ constexpr int kHmGroup = 8;
 constexpr int kHmMaxPlanes = 1024;
 constexpr int kHmMaxDim = 8192;
 constexpr int kHmQueue = 1024;          // queued replays per block
-constexpr int kHmBatch = 8;             // plane entries in flight per replay
+constexpr int kHmBatch = 4;             // sign words (16 dimensions each) in flight per replay
 constexpr int64_t kHmMinBatch = 1024;   // smaller batches take the per-plane kernel
 
 // Eight x values of row xr at dims d0..d0+7 (0 past dim); VEC: two aligned
@@ -316,30 +315,233 @@ __device__ __forceinline__ void hm_load8(const float* __restrict__ xr, int d0, i
   }
 }
 
-// The reference's sequential sum for one (row, plane): its sign bit.
-__device__ __forceinline__ bool hm_replay(const float* __restrict__ xr, const int32_t* __restrict__ nnz,
-                                          const uint32_t* __restrict__ ent_t, int P, int pl) {
+// The reference's sequential sum for one (row, plane): its sign bit.  `spw` are the
+// plane's 2-bit signs (kh_hash_family::sp_dev); a dimension without a coefficient
+// adds a zero of either sign, which leaves every later sum and the sign test alone,
+// and its x is masked off, so inf and NaN add nothing there.  Both are read in
+// whole pieces, NB words (16 dimensions each) in flight.
+template <bool VEC, int NB>
+__device__ __forceinline__ bool hm_replay(const float* __restrict__ xr, const uint32_t* __restrict__ spw, int dim) {
   float s = 0.0f;
-  const int e1 = nnz[pl];
-  for (int e0 = 0; e0 < e1; e0 += kHmBatch) {
-    uint32_t v[kHmBatch];
-    float xd[kHmBatch];
+  const int nw = (dim + 15) / 16;
+  for (int w0 = 0; w0 < nw; w0 += NB) {
+    uint32_t w[NB];
+    float4 x[NB][4];
 #pragma unroll
-    for (int j = 0; j < kHmBatch; ++j) v[j] = ent_t[(size_t)min(e0 + j, e1 - 1) * P + pl];
+    for (int j = 0; j < NB; ++j) {
+      w[j] = w0 + j < nw ? spw[w0 + j] : 0u;
+      const int d = 16 * min(w0 + j, nw - 1);
+      hm_load8<VEC>(xr, d, dim, x[j][0], x[j][1]);
+      hm_load8<VEC>(xr, VEC ? min(d + 8, dim - 8) : d + 8, dim, x[j][2], x[j][3]);
+    }
 #pragma unroll
-    for (int j = 0; j < kHmBatch; ++j) xd[j] = xr[v[j] >> 1];
+    for (int j = 0; j < NB; ++j) {
 #pragma unroll
-    for (int j = 0; j < kHmBatch; ++j)
-      if (e0 + j < e1) s = (v[j] & 1u) ? __fsub_rn(s, xd[j]) : __fadd_rn(s, xd[j]);
+      for (int q = 0; q < 4; ++q) {
+        const float v[4] = {x[j][q].x, x[j][q].y, x[j][q].z, x[j][q].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t c = w[j] >> (2 * (4 * q + i));   // bit 0: a term, bit 1: negative
+          const uint32_t on = 0u - (c & 1u);
+          s = __fadd_rn(s, __uint_as_float((__float_as_uint(v[i]) & on) ^ ((c & 2u) << 30)));
+        }
+      }
+    }
   }
   return s >= 0.0f;
 }
 
+// |S' - S| <= sum|x| * (2^-17 + 64 ksteps * 2^-23): the lo term's residual, and an
+// ulp (twice a rounded add's error) for each of the 2 * 32 * ksteps accumulated
+// products.  |s_seq - S| <= sum|x| * dim * 2^-24.  A quarter more for the rounding
+// of the bound's own sums; plus an absolute term for denormals flushed by the
+// matrix cores.
+__device__ __forceinline__ float hm_bound(float sum_abs, int ksteps, int dim) {
+  const float rel = 1.25f * (0x1p-17f + (float)(64 * ksteps) * 0x1p-23f + (float)dim * 0x1p-24f);
+  return sum_abs * rel + (float)(4 * 32 * ksteps + 16) * 0x1p-120f;
+}
+
+// Matrix-core hashing with the planes resident: 450 planes of 128 dimensions are 116
+// KB of operands, which hash_dense_mfma_kernel reads again for every 16 rows
+// (1.45 GB through L2 for 200000 rows).  Here a block of sixteen waves keeps them
+// in LDS and every wave walks its own tiles of 16 rows.  What then counts is
+// instructions per sum: a sign costs a compare into a lane mask and its share of one
+// margin test for kHrGroup plane tiles; the undecided ones (about 7 in 10000) queue
+// per wave and are replayed in its lanes, which set or clear their bit.
+// 200003 rows: 113 us, 224 before.
+constexpr int kHrWaves = 16;
+constexpr int kHrGroup = 4;      // plane tiles in flight per wave
+constexpr int kHrQueue = 512;    // queued replays per wave; emptied when over kHrFull
+constexpr int kHrFull = kHrQueue - 256;   // a plane tile adds at most 256
+constexpr int kHrMaxSteps = 4;   // k steps whose A operands fit 128 registers (unaligned rows: half)
+constexpr int kHrBatch = 2;      // sign words in flight per replay
+// Words of plane bits per row: 32 planes each, and one to read past the last.
+__host__ __device__ constexpr int hr_words(int ntiles) { return (ntiles + 1) / 2 + 1; }
+static size_t hr_lds(int ksteps, int ntiles) {
+  return (size_t)ksteps * ntiles * 1024 + kHrWaves * (sizeof(uint32_t) * 16 * hr_words(ntiles) + sizeof(uint16_t) * kHrQueue);
+}
+
+// Orders a wave's LDS accesses (of any type) before and after it.
+__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <int KS, bool VEC>
+__global__ __launch_bounds__(64 * kHrWaves) void hash_dense_resident_kernel(
+    const uint4* __restrict__ bt, int ksteps, int ntiles, const uint32_t* __restrict__ sp, int spn, int k, int L,
+    int dim, const float* __restrict__ x, int64_t ldx, int64_t batch, uint32_t* __restrict__ codes, int64_t row_stride,
+    int64_t table_stride) {
+  extern __shared__ uint4 hr_lds_buf[];
+  __shared__ int nq[kHrWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int nb = ksteps * ntiles * 64, words = hr_words(ntiles);
+  uint4* B = hr_lds_buf;
+  uint32_t* pm = reinterpret_cast<uint32_t*>(B + nb) + wave * 16 * words;
+  uint16_t* queue = reinterpret_cast<uint16_t*>(reinterpret_cast<uint32_t*>(B + nb) + kHrWaves * 16 * words) +
+                    wave * kHrQueue;
+  for (int i0 = threadIdx.x; i0 < nb; i0 += 64 * kHrWaves * 4) {
+    uint4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = bt[min(i0 + u * 64 * kHrWaves, nb - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) B[min(i0 + u * 64 * kHrWaves, nb - 1)] = v[u];
+  }
+  for (int i = lane; i < 16 * words; i += 64) pm[i] = 0u;
+  __syncthreads();
+  const int P = L * k;
+  const int kq = (lane >> 4) * 8;
+  const int64_t tiles = (batch + 15) / 16, step = (int64_t)gridDim.x * kHrWaves;
+  for (int64_t tile = (int64_t)blockIdx.x * kHrWaves + wave; tile < tiles; tile += step) {
+    const int64_t r0 = tile * 16;
+    uint4 hi[KS], lo[KS];
+    float ax = 0.0f;
+    {
+      const float* __restrict__ xr = x + min(r0 + (lane & 15), batch - 1) * ldx;
+      float4 xa[KS], xb[KS];
+#pragma unroll
+      for (int st = 0; st < KS; ++st)
+        hm_load8<VEC>(xr, VEC ? min(st * 32 + kq, dim - 8) : st * 32 + kq, dim, xa[st], xb[st]);
+#pragma unroll
+      for (int st = 0; st < KS; ++st) {
+        const float4 a = xa[st], b = xb[st];
+        const float s = (fabsf(a.x) + fabsf(a.y)) + (fabsf(a.z) + fabsf(a.w)) + (fabsf(b.x) + fabsf(b.y)) + (fabsf(b.z) + fabsf(b.w));
+        ax += st < ksteps ? s : 0.0f;
+        split_bf16x8(a, b, hi[st], lo[st]);
+      }
+    }
+    ax += __shfl_xor(ax, 16);
+    ax += __shfl_xor(ax, 32);
+    float bound[4];
+    bool odd_row = false;   // inf, NaN or sums near overflow: no sign of the row is decided
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float a = __shfl(ax, (lane >> 4) * 4 + q);
+      const bool fine = a < 1e37f;
+      bound[q] = fine ? hm_bound(a, ksteps, dim) : INFINITY;
+      odd_row = odd_row || !fine;
+    }
+    const bool any_odd = __ballot(odd_row) != 0ull;
+    if (lane == 0) nq[wave] = 0;
+    wave_lds_fence();
+    int t0 = 0;
+    do {
+      for (bool room = true; room && t0 < ntiles; t0 += kHrGroup) {
+        kh_f32x4 c[kHrGroup];
+#pragma unroll
+        for (int u = 0; u < kHrGroup; ++u) c[u] = kh_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int st = 0; st < KS; ++st) {
+          if (st < ksteps) {
+            uint4 w[kHrGroup];
+#pragma unroll
+            for (int u = 0; u < kHrGroup; ++u) w[u] = B[(st * ntiles + min(t0 + u, ntiles - 1)) * 64 + lane];
+#pragma unroll
+            for (int u = 0; u < kHrGroup; ++u)
+              c[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(hi[st]), as_bf16x8(w[u]), c[u], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < kHrGroup; ++u)
+              c[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(lo[st]), as_bf16x8(w[u]), c[u], 0, 0, 0);
+          }
+        }
+        if (t0 + kHrGroup >= ntiles) {   // planes that do not exist: decided (their bits are not read)
+#pragma unroll
+          for (int u = 0; u < kHrGroup; ++u)
+            if ((t0 + u) * 16 + (lane & 15) >= P)
+#pragma unroll
+              for (int q = 0; q < 4; ++q) c[u][q] = 3e38f;
+        }
+        float margin = INFINITY;
+#pragma unroll
+        for (int u = 0; u < kHrGroup; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) margin = fminf(margin, fabsf(c[u][q]) - bound[q]);
+        const bool check = any_odd || __ballot(!(margin > 0.0f)) != 0ull;
+#pragma unroll
+        for (int u = 0; u < kHrGroup; ++u) {
+          const int t = t0 + u;
+          if (t < ntiles) {
+            uint64_t m[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) m[q] = __ballot(c[u][q] > 0.0f);
+            // row 4g + i of the tile: bits 16g.. of m[i]
+            if (lane < 16) {
+              const uint64_t mm = (lane & 2) ? ((lane & 1) ? m[3] : m[2]) : ((lane & 1) ? m[1] : m[0]);
+              reinterpret_cast<uint16_t*>(pm)[2 * lane * words + t] = (uint16_t)(mm >> (16 * (lane >> 2)));
+            }
+          }
+        }
+        if (check) {
+#pragma unroll
+          for (int u = 0; u < kHrGroup; ++u) {
+            const int pl = (t0 + u) * 16 + (lane & 15);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const int rr = (lane >> 4) * 4 + q;
+              if (!(fabsf(c[u][q]) > bound[q]) && pl < P && t0 + u < ntiles && r0 + rr < batch)
+                queue[atomicAdd(&nq[wave], 1) & (kHrQueue - 1)] = (uint16_t)(rr << 10 | pl);
+            }
+            wave_lds_fence();
+            if (nq[wave] > kHrFull) room = false;
+            // a group whose later tiles might not fit starts over after the replay
+            if (!room) {
+              t0 += u + 1 - kHrGroup;
+              break;
+            }
+          }
+        }
+      }
+      wave_lds_fence();
+      const int n = nq[wave];
+      for (int i = lane; i < n; i += 64) {
+        const uint32_t e = queue[i];
+        const int rr = (int)(e >> 10), pl = (int)(e & 1023u);
+        const uint32_t bit = 1u << (pl & 31);
+        if (hm_replay<VEC, kHrBatch>(x + (r0 + rr) * ldx, sp + (int64_t)pl * spn, dim)) atomicOr(&pm[rr * words + (pl >> 5)], bit);
+        else atomicAnd(&pm[rr * words + (pl >> 5)], ~bit);
+      }
+      wave_lds_fence();
+      if (lane == 0) nq[wave] = 0;
+      wave_lds_fence();
+    } while (t0 < ntiles);
+    // codes: table t takes planes t*k .. t*k+k-1 of its row; a lane a row, four tables at once
+    const int r = lane & 15;
+    const uint32_t mask = (uint32_t)((1ull << k) - 1ull);
+    if (r0 + r < batch) {
+      uint32_t* __restrict__ out = codes + (r0 + r) * row_stride;
+      const uint32_t* pr = pm + r * words;
+      for (int tb = lane >> 4; tb < L; tb += 4) {
+        const int p0 = tb * k;
+        const uint64_t win = (uint64_t)pr[p0 >> 5] | ((uint64_t)pr[(p0 >> 5) + 1] << 32);
+        out[tb * table_stride] = (uint32_t)(win >> (p0 & 31)) & mask;
+      }
+    }
+    wave_lds_fence();
+  }
+}
+
 template <bool VEC>
 __global__ __launch_bounds__(256) void hash_dense_mfma_kernel(
-    const uint4* __restrict__ bt, int ksteps, int ntiles, const int32_t* __restrict__ nnz,
-    const uint32_t* __restrict__ ent_t, int k, int L, int dim, const float* __restrict__ x,
-    int64_t ldx, int64_t batch, uint32_t* __restrict__ codes) {
+    const uint4* __restrict__ bt, int ksteps, int ntiles, const uint32_t* __restrict__ sp, int spn, int k, int L,
+    int dim, const float* __restrict__ x, int64_t ldx, int64_t batch, uint32_t* __restrict__ codes,
+    int64_t row_stride, int64_t table_stride) {
   constexpr int kW = kHmMaxPlanes / 32 + 1;  // 32-plane words per row (one spare for the code window)
   __shared__ uint32_t pm[kHmRows][kW];
   __shared__ uint32_t queue[kHmQueue];
@@ -363,18 +565,12 @@ __global__ __launch_bounds__(256) void hash_dense_mfma_kernel(
   }
   ax += __shfl_xor(ax, 16);
   ax += __shfl_xor(ax, 32);
-  // Bound on |S' - S| + |s_seq - S| per unit of sum|x|, generous: the lo term's
-  // residual (2^-17), the matrix cores' f32 accumulation over 2 * 32 * ksteps
-  // products (an ulp per add), the sequential sum's dim adds (half an ulp each),
-  // doubled; plus an absolute term for denormals flushed by the matrix cores.
-  const float rel = 2.0f * (0x1p-17f + (float)(2 * 32 * ksteps + dim) * 0x1p-23f);
-  const float abs_t = (float)(4 * 32 * ksteps + 16) * 0x1p-120f;
   float bound[4];
   bool fin[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const float a = __shfl(ax, (lane >> 4) * 4 + q);
-    bound[q] = a * 1.01f * rel + abs_t;
+    bound[q] = hm_bound(a, ksteps, dim);
     fin[q] = a < 1e37f;   // also false for inf / NaN
   }
   __syncthreads();
@@ -424,7 +620,7 @@ __global__ __launch_bounds__(256) void hash_dense_mfma_kernel(
             queue[slot] = ((uint32_t)rr << 16) | (uint32_t)pl;
             bit = false;   // set by the replay below
           } else {
-            bit = hm_replay(x + (rb + rr) * ldx, nnz, ent_t, P, pl);
+            bit = hm_replay<VEC, kHmBatch>(x + (rb + rr) * ldx, sp + (int64_t)pl * spn, dim);
           }
         }
         const uint64_t m = __ballot(bit && pl < P);
@@ -438,7 +634,7 @@ __global__ __launch_bounds__(256) void hash_dense_mfma_kernel(
   for (int i = threadIdx.x; i < nrep; i += blockDim.x) {
     const uint32_t e = queue[i];
     const int rr = (int)(e >> 16), pl = (int)(e & 0xffffu);
-    if (hm_replay(x + (rb + rr) * ldx, nnz, ent_t, P, pl)) atomicOr(&pm[rr][pl >> 5], 1u << (pl & 31));
+    if (hm_replay<VEC, kHmBatch>(x + (rb + rr) * ldx, sp + (int64_t)pl * spn, dim)) atomicOr(&pm[rr][pl >> 5], 1u << (pl & 31));
   }
   __syncthreads();
   // codes: table t takes planes t*k .. t*k+k-1 of its row
@@ -447,7 +643,7 @@ __global__ __launch_bounds__(256) void hash_dense_mfma_kernel(
     if (rb + r >= batch) continue;
     const int p0 = t * k, w0 = p0 >> 5;
     const uint64_t win = (uint64_t)pm[r][w0] | ((uint64_t)pm[r][w0 + 1] << 32);
-    codes[(rb + r) * L + t] = (uint32_t)((win >> (p0 & 31)) & ((1ull << k) - 1ull));
+    codes[(rb + r) * row_stride + t * table_stride] = (uint32_t)((win >> (p0 & 31)) & ((1ull << k) - 1ull));
   }
 }
 
@@ -1016,22 +1212,52 @@ __global__ __launch_bounds__(256) void csr_pack_kernel(
 }
 
 // ------------------------------------------------------------------ host helpers
+// The matrix-core kernels, codes[row * row_stride + table * table_stride].  Planes
+// that fit LDS with their waves' marks stay resident.
+static int hash_matrix_launch(const kh_hash_family* h, const float* x, int64_t ldx, int64_t batch, uint32_t* codes,
+                              int64_t row_stride, int64_t table_stride, hipStream_t st) {
+  const bool vec = h->dim % 32 == 0 && ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const int spn = (h->dim + 15) / 16;
+  const size_t lds = hr_lds(h->bt_ksteps, h->bt_tiles);
+  if (h->bt_ksteps <= (vec ? kHrMaxSteps : kHrMaxSteps / 2) && lds <= (size_t)kMaxDynLds) {
+    using Fn = decltype(&hash_dense_resident_kernel<1, true>);
+    static const Fn fns[3][2] = {{hash_dense_resident_kernel<1, false>, hash_dense_resident_kernel<1, true>},
+                                 {hash_dense_resident_kernel<2, false>, hash_dense_resident_kernel<2, true>},
+                                 {nullptr, hash_dense_resident_kernel<4, true>}};
+    static std::once_flag once;
+    static hipError_t attr_rc = hipSuccess;
+    std::call_once(once, [] {
+      for (const auto& f : fns)
+        for (const Fn g : f)
+          if (g && attr_rc == hipSuccess)
+            attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(g), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          kMaxDynLds);
+    });
+    KH_HIP(attr_rc);
+    const int ks = h->bt_ksteps;
+    const Fn fn = fns[ks <= 1 ? 0 : ks <= 2 ? 1 : 2][vec ? 1 : 0];
+    const int blocks = (int)std::min<int64_t>(256, (batch + 16 * kHrWaves - 1) / (16 * kHrWaves));
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * kHrWaves), lds, st, h->bt_dev, ks, h->bt_tiles, h->sp_dev,
+                       spn, h->k, h->L, h->dim, x, ldx, batch, codes, row_stride, table_stride);
+    KH_LAUNCHED();
+    return KH_OK;
+  }
+  for (int64_t b0 = 0; b0 < batch; b0 += (int64_t)65535 * kHmRows) {
+    const int64_t nb = std::min<int64_t>(batch - b0, (int64_t)65535 * kHmRows);
+    hipLaunchKernelGGL(vec ? hash_dense_mfma_kernel<true> : hash_dense_mfma_kernel<false>,
+                       dim3((unsigned)ceil_div(nb, kHmRows)), dim3(256), 0, st, h->bt_dev, h->bt_ksteps,
+                       h->bt_tiles, h->sp_dev, spn, h->k, h->L, h->dim, x + b0 * ldx, ldx, nb,
+                       codes + b0 * row_stride, row_stride, table_stride);
+    KH_LAUNCHED();
+  }
+  return KH_OK;
+}
+
 int hash_dense_launch(const kh_hash_family* h, const float* x, int64_t ldx, int64_t batch,
                       uint32_t* codes, hipStream_t st) {
   if (batch == 0) return KH_OK;
   if (h->kind != KH_FAMILY_TERNARY) return rank_hash_dense_launch(h, x, ldx, batch, codes, st);
-  if (h->bt_dev && batch >= kHmMinBatch) {
-    for (int64_t b0 = 0; b0 < batch; b0 += (int64_t)65535 * kHmRows) {
-      const int64_t nb = std::min<int64_t>(batch - b0, (int64_t)65535 * kHmRows);
-      const bool vec = h->dim % 32 == 0 && ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-      hipLaunchKernelGGL(vec ? hash_dense_mfma_kernel<true> : hash_dense_mfma_kernel<false>,
-                         dim3((unsigned)ceil_div(nb, kHmRows)), dim3(256), 0, st, h->bt_dev, h->bt_ksteps,
-                         h->bt_tiles, h->nnz, h->ent_t, h->k, h->L, h->dim, x + b0 * ldx, ldx, nb,
-                         codes + b0 * h->L);
-      KH_LAUNCHED();
-    }
-    return KH_OK;
-  }
+  if (h->bt_dev && batch >= kHmMinBatch) return hash_matrix_launch(h, x, ldx, batch, codes, h->L, 1, st);
   if (h->dim <= kHlMaxDim) {
     const size_t lds = sizeof(uint4) * h->sg_n4 + sizeof(uint2) * hl_pad(h->dim) + sizeof(uint32_t) * h->sg_tpb;
     if (lds <= (size_t)kMaxDynLds) {
@@ -1212,12 +1438,21 @@ static int family_finish(kh_hash_family* h, kh_hash_family** out) {
             bt[(((size_t)st * h->bt_tiles + tile) * 64 + l) * 8 + i] = v == 1 ? 0x3F80 : (v == -1 ? 0xBF80 : 0);
           }
         }
+    const int spn = (h->dim + 15) / 16;
+    std::vector<uint32_t> sp((size_t)P * spn, 0u);
+    for (int p = 0; p < P; ++p)
+      for (int d = 0; d < h->dim; ++d) {
+        const int8_t v = h->planes_host[(size_t)p * h->dim + d];
+        sp[(size_t)p * spn + d / 16] |= (v == 1 ? 1u : v == -1 ? 3u : 0u) << (2 * (d % 16));
+      }
     h->bt_dev = static_cast<uint4*>(dev_alloc(sizeof(uint16_t) * bt.size()));
-    if (!h->bt_dev) {
+    h->sp_dev = static_cast<uint32_t*>(dev_alloc(sizeof(uint32_t) * sp.size()));
+    if (!h->bt_dev || !h->sp_dev) {
       kh_hash_family_destroy(h);
       return KH_ERR_ALLOC;
     }
-    if (hipMemcpy(h->bt_dev, bt.data(), sizeof(uint16_t) * bt.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMemcpy(h->bt_dev, bt.data(), sizeof(uint16_t) * bt.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(h->sp_dev, sp.data(), sizeof(uint32_t) * sp.size(), hipMemcpyHostToDevice) != hipSuccess) {
       set_error("plane upload failed");
       kh_hash_family_destroy(h);
       return KH_ERR_HIP;
@@ -1326,6 +1561,7 @@ extern "C" int kh_hash_family_destroy(kh_hash_family* h) {
   dev_free(h->ent_t);
   dev_free(h->bt_dev);
   dev_free(h->sg_dev);
+  dev_free(h->sp_dev);
   dev_free(h->windows_dev);
   dev_free(h->fallback_dev);
   dev_free(h->perms_dev);

@@ -24,6 +24,9 @@ struct kh_hash_family {
   // [ceil(dim/32)][ceil(L*k/16)][64 lanes] x 8 values; null otherwise.
   uint4* bt_dev = nullptr;
   int bt_ksteps = 0, bt_tiles = 0;
+  // The same planes' 2-bit signs plane by plane, [L*k][ceil(dim/16)] words (01 = +1,
+  // 11 = -1), for the sums the matrix cores leave undecided.
+  uint32_t* sp_dev = nullptr;
   // 2-bit plane signs for the per-row kernels: group g holds tables g*sg_tpb.. (planes q = 0..sg_tpb*k-1 of the
   // group), as [dim][sg_words] words, plane q in bits 2(q%16), 2(q%16)+1 of
   // word q/16 (01 = +1, 11 = -1, 00 = no term); each group padded to sg_n4
