@@ -1034,45 +1034,89 @@ __global__ void attn_set_len_kernel(int32_t* __restrict__ lens, int n, int value
   if (i < n) lens[i] = value;
 }
 
-// src [nkv][len][D] f32 -> one sequence's cache rows 0..len-1 (dst [nkv][max_seq][D]).
-template <typename KV>
-__global__ __launch_bounds__(256) void attn_fill_cache_kernel(const float* __restrict__ src,
-                                                              int64_t len, int D, int64_t total,
-                                                              int max_seq, KV* __restrict__ dst) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const int64_t per = len * D;
-  const int64_t h = i / per, r = i - h * per;
-  store_kv(dst + (h * max_seq) * (int64_t)D + r, src[i]);
-}
-
-// Device-loaded rows of a KH_KV_BF16 handle: both the f32 and the BF16 copy
-// are written, and *notbf records whether any value of k or v carries bits a
-// BF16 cannot hold; attn_set_pre_kernel then makes the rows a BF16 prefix
-// only when none does (so the cache always holds the values exactly).
-__global__ __launch_bounds__(256) void attn_fill_cache2_kernel(
-    const float* __restrict__ k, const float* __restrict__ v, int64_t len, int D, int64_t total,
-    int max_seq, float* __restrict__ k32, float* __restrict__ v32, uint16_t* __restrict__ k16,
-    uint16_t* __restrict__ v16, int32_t* __restrict__ notbf) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool bad = false;
-  if (i < total) {
-    const int64_t per = len * D;
-    const int64_t h = i / per, r = i - h * per;
-    const int64_t o = (h * max_seq) * (int64_t)D + r;
-    const uint32_t kb = __float_as_uint(k[i]), vb = __float_as_uint(v[i]);
-    k32[o] = k[i];
-    v32[o] = v[i];
-    k16[o] = static_cast<uint16_t>(kb >> 16);
-    v16[o] = static_cast<uint16_t>(vb >> 16);
-    bad = ((kb | vb) & 0xffffu) != 0;
+// Device-loaded rows: k, v [nkv][len][D] f32 -> one sequence's cache rows 0..len-1
+// ([nkv][max_seq][D]).  Bound by the bytes: 8 of f32 read and 4 of BF16 written per
+// pair of values, so a KH_KV_BF16 handle first writes the BF16 copy alone
+// (attn_load16_kernel) and records per block whether any value carries bits that a
+// BF16 cannot hold; attn_load32_kernel then makes the rows a BF16 prefix when none
+// does, and otherwise reads them again into the f32 cache (so the cache always holds
+// the values exactly; every load of a KH_KV_F32 handle goes that way).  It also sets
+// the lengths.  Each block writes its own flag word, so nothing is cleared first.
+// Grid (blocks per head, nkv), eight values of k and of v per thread and step.
+// 2 x 32 x 2048 x 128 values: 16.8 + 3.7 us (two launches), against 31 + 4.5 us and
+// two more launches when both copies were always written, a value per thread.
+constexpr int kLoadBlocks = 1024;   // four blocks of 256 threads per CU
+static_assert(kMaxAttnHeads <= kLoadBlocks);
+template <bool VEC>
+__device__ __forceinline__ void load8(const float* __restrict__ p, float (&r)[8]) {
+  if constexpr (VEC) {
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+    r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = p[e];
   }
-  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(notbf, 1);
 }
 
-__global__ void attn_set_pre_kernel(int32_t* __restrict__ pre, const int32_t* __restrict__ notbf,
-                                    int len) {
-  if (threadIdx.x == 0) pre[0] = notbf[0] ? 0 : len;
+template <bool VEC>
+__global__ __launch_bounds__(256) void attn_load16_kernel(const float* __restrict__ k, const float* __restrict__ v,
+                                                          int64_t per, int64_t head_stride, uint16_t* __restrict__ k16,
+                                                          uint16_t* __restrict__ v16, int32_t* __restrict__ notbf) {
+  const float* __restrict__ src[2] = {k + blockIdx.y * per, v + blockIdx.y * per};
+  uint16_t* __restrict__ dst[2] = {k16 + blockIdx.y * head_stride, v16 + blockIdx.y * head_stride};
+  constexpr int U = 2;
+  const int64_t step = (int64_t)gridDim.x * 256 * 8;
+  uint32_t low = 0u;
+  for (int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i0 < per; i0 += step * U) {
+    float r[U][2][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u)   // the last 8 values again past the end, stored twice alike
+#pragma unroll
+      for (int s = 0; s < 2; ++s) load8<VEC>(src[s] + min(i0 + u * step, per - 8), r[u][s]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t lo = __float_as_uint(r[u][s][2 * e]), hi = __float_as_uint(r[u][s][2 * e + 1]);
+          low |= lo | hi;
+          w[e] = (lo >> 16) | (hi & 0xffff0000u);
+        }
+        *reinterpret_cast<uint4*>(dst[s] + min(i0 + u * step, per - 8)) = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+  }
+  const int bad = __syncthreads_or((low & 0xffffu) != 0u);
+  if (threadIdx.x == 0) notbf[blockIdx.y * gridDim.x + blockIdx.x] = bad;
+}
+
+// nflags = 0: f32 rows always.
+template <bool VEC>
+__global__ __launch_bounds__(256) void attn_load32_kernel(const float* __restrict__ k, const float* __restrict__ v,
+                                                          int64_t per, int64_t head_stride,
+                                                          const int32_t* __restrict__ notbf, int nflags, int len,
+                                                          float* __restrict__ k32, float* __restrict__ v32,
+                                                          int32_t* __restrict__ pre, int32_t* __restrict__ lens) {
+  int any = nflags == 0;
+  for (int i = threadIdx.x; i < nflags; i += 256) any |= notbf[i];
+  const int f32 = __syncthreads_or(any);
+  if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+    *pre = f32 ? 0 : len;
+    *lens = len;
+  }
+  if (!f32) return;
+  const float* __restrict__ src[2] = {k + blockIdx.y * per, v + blockIdx.y * per};
+  float* __restrict__ dst[2] = {k32 + blockIdx.y * head_stride, v32 + blockIdx.y * head_stride};
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < per; i += (int64_t)gridDim.x * 256 * 8)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float r[8];
+      load8<VEC>(src[s] + i, r);
+      reinterpret_cast<float4*>(dst[s] + i)[0] = make_float4(r[0], r[1], r[2], r[3]);
+      reinterpret_cast<float4*>(dst[s] + i)[1] = make_float4(r[4], r[5], r[6], r[7]);
+    }
 }
 
 // o_proj for batch <= 2 with the chunk merge folded in: gather_rows_kernel's
@@ -1254,7 +1298,7 @@ struct kh_sparse_attn {
   float* kc32 = nullptr;
   float* vc32 = nullptr;
   int32_t* pre = nullptr;    // [max_batch]
-  int32_t* notbf = nullptr;  // [1] device-side load check (kh_sparse_attn_load_cache_dev)
+  int32_t* notbf = nullptr;  // [max_batch][kLoadBlocks] flags of kh_sparse_attn_load_cache_dev
   float* cos_t = nullptr;    // [max_seq][d/2]
   float* sin_t = nullptr;
   int32_t* lens = nullptr;   // [max_batch]
@@ -1329,7 +1373,7 @@ static int attn_alloc(int hidden, int num_heads, int num_kv_heads, int head_dim,
   a->kc32 = static_cast<float*>(dev_alloc(sizeof(float) * a->seq_elems() * max_batch));
   a->vc32 = static_cast<float*>(dev_alloc(sizeof(float) * a->seq_elems() * max_batch));
   a->pre = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * max_batch));
-  a->notbf = static_cast<int32_t*>(dev_alloc(sizeof(int32_t)));
+  a->notbf = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * kLoadBlocks * max_batch));
   a->cos_t = static_cast<float*>(dev_alloc(sizeof(float) * max_seq * half));
   a->sin_t = static_cast<float*>(dev_alloc(sizeof(float) * max_seq * half));
   a->lens = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * max_batch));
@@ -1492,29 +1536,19 @@ extern "C" int kh_sparse_attn_load_cache_dev(kh_sparse_attn* a, int64_t b, const
   KH_CHECK_ARG(len >= 0 && len <= a->max_seq, "len %lld not in [0,%d]", (long long)len, a->max_seq);
   KH_CHECK_ARG(len == 0 || (k_dev && v_dev), "null cache data");
   hipStream_t st = as_stream(stream);
-  const int64_t total = (int64_t)a->nkv * len * a->d;
-  const unsigned blocks = static_cast<unsigned>((total + 255) / 256);
   const size_t off = (size_t)b * a->seq_elems();
-  if (total > 0 && !a->kv_f32) {
-    // both copies, and on the device: a BF16 prefix when every value is a
-    // BF16 value (a BF16 model's prefill), else f32 rows (pre = 0)
-    hipLaunchKernelGGL(attn_set_len_kernel, dim3(1), dim3(64), 0, st, a->notbf, 1, 0);
-    hipLaunchKernelGGL(attn_fill_cache2_kernel, dim3(blocks), dim3(256), 0, st, k_dev, v_dev, len, a->d,
-                       total, a->max_seq, a->kc32 + off, a->vc32 + off, a->kc16 + off, a->vc16 + off,
-                       a->notbf);
-    hipLaunchKernelGGL(attn_set_pre_kernel, dim3(1), dim3(64), 0, st, a->pre + b, a->notbf,
-                       static_cast<int>(len));
-  } else {
-    if (total > 0) {
-      hipLaunchKernelGGL(attn_fill_cache_kernel<float>, dim3(blocks), dim3(256), 0, st, k_dev, len, a->d,
-                         total, a->max_seq, a->kc32 + off);
-      hipLaunchKernelGGL(attn_fill_cache_kernel<float>, dim3(blocks), dim3(256), 0, st, v_dev, len, a->d,
-                         total, a->max_seq, a->vc32 + off);
-    }
-    hipLaunchKernelGGL(attn_set_len_kernel, dim3(1), dim3(64), 0, st, a->pre + b, 1, 0);
-  }
-  hipLaunchKernelGGL(attn_set_len_kernel, dim3(1), dim3(64), 0, st, a->lens + b, 1,
-                     static_cast<int>(len));
+  const int64_t per = len * a->d, hs = (int64_t)a->max_seq * a->d;   // multiples of 64
+  const bool vec = ((reinterpret_cast<uintptr_t>(k_dev) | reinterpret_cast<uintptr_t>(v_dev)) & 15) == 0;
+  const int64_t bx = std::max<int64_t>(1, std::min<int64_t>(kLoadBlocks / a->nkv, (per / 8 + 255) / 256));
+  const dim3 grid((unsigned)bx, (unsigned)a->nkv);
+  int32_t* flags = a->notbf + b * kLoadBlocks;
+  const int nflags = a->kv_f32 || len == 0 ? 0 : (int)bx * a->nkv;
+  if (nflags)
+    hipLaunchKernelGGL(vec ? attn_load16_kernel<true> : attn_load16_kernel<false>, grid, dim3(256), 0, st, k_dev, v_dev,
+                       per, hs, a->kc16 + off, a->vc16 + off, flags);
+  hipLaunchKernelGGL(vec ? attn_load32_kernel<true> : attn_load32_kernel<false>, len ? grid : dim3(1), dim3(256), 0, st,
+                     k_dev, v_dev, per, hs, flags, nflags, (int)len, a->kc32 + off, a->vc32 + off, a->pre + b,
+                     a->lens + b);
   KH_LAUNCHED();
   a->len_host[b] = len;
   a->pre_host[b] = -1;  // decided on the device
