@@ -58,6 +58,8 @@ struct kh_lsh_index {
   uint32_t id_bound = 0;      // 1 + largest id inserted so far (ids are below 2^31)
   mutable kh::StreamWs ws;    // query scratch per stream
   kh::ScratchArena arena;     // insert / remove / rebuild scratch, kept between calls
+  uint32_t* mx_host = nullptr;  // pinned: the largest id of an insert call
+  hipEvent_t mx_done = nullptr; // recorded when it is written
 };
 
 namespace kh {
