@@ -1377,7 +1377,6 @@ __global__ void csr_copy_f32_kernel(const float* __restrict__ src, int stride,
 // off[row] (and the last row off[batch]), and every block copies its share of
 // the row into each destination given.  The same result as csr_offsets_kernel
 // followed by one csr_copy kernel per array.
-constexpr int kCsrPackMax = 4096;
 __global__ __launch_bounds__(256) void csr_pack_kernel(
     const int32_t* __restrict__ lens, int64_t batch, int stride, int64_t capacity,
     int64_t* __restrict__ off, const uint32_t* __restrict__ s0, uint32_t* __restrict__ d0,
@@ -1583,6 +1582,10 @@ int csr_finish(const uint32_t* qids, const uint32_t* qcnt, const float* f1, cons
     if (o2 && f2) hipLaunchKernelGGL(csr_copy_f32_kernel, g, dim3(256), 0, st, f2, stride, ulen, off, capacity, o2);
     KH_LAUNCHED();
   }
+  return csr_check(off, batch, stride, capacity, st);
+}
+
+int csr_check(const int64_t* off, int64_t batch, int stride, int64_t capacity, hipStream_t st) {
   // Every row holds at most `stride` entries: with room for that many, no
   // overflow is possible and the call stays asynchronous (no host round trip;
   // capturable in a graph).  Otherwise the total is read back to report one.

@@ -86,5 +86,9 @@ int rank_hash_sparse_launch(const kh_hash_family* h, const int64_t* xoff, const 
 int csr_finish(const uint32_t* qids, const uint32_t* qcnt, const float* f1, const float* f2,
                int stride, const int32_t* ulen, int64_t batch, int64_t* off, uint32_t* ids,
                uint32_t* cnts, float* o1, float* o2, int64_t capacity, hipStream_t st);
+// csr_finish's capacity check alone, for kernels that write CSR rows themselves.
+int csr_check(const int64_t* off, int64_t batch, int stride, int64_t capacity, hipStream_t st);
+// Rows of a batch up to which a block sums the lengths before its row itself.
+constexpr int kCsrPackMax = 4096;
 
 }  // namespace kh

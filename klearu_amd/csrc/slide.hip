@@ -288,6 +288,59 @@ __device__ __forceinline__ int vanilla_len(const int32_t* alen, int64_t row, int
   all = fb_n > 0 && n == 0;
   return all ? fb_n : n;
 }
+// Where a forward's CSR rows go.  A block sums the lengths before its row itself (up to
+// kCsrPackMax rows; longer batches and off == nullptr leave rows in pre / post for a
+// packing launch), so entries are written once, in place; a row that does not fit
+// below `capacity` is worked out in pre / post and its head copied, the caller then
+// reports the overflow.  The packing launch took 4 us (128 rows of 1000) and 18 us
+// (256 rows of 6400) besides the second pass over the values.
+struct CsrOut {
+  int64_t* off;
+  uint32_t* ids;
+  float *pre, *act;
+  int64_t batch, capacity;
+};
+struct CsrRow {
+  int64_t o;       // the row's first entry
+  bool direct;     // it fits
+  float *pre, *act;
+};
+// Before a barrier: this wave's part of the lengths before `row`.
+__device__ __forceinline__ void csr_part(const CsrOut& co, const int32_t* alen, int64_t row, int fb_n, long long* part) {
+  if (!co.off) return;
+  long long s = 0;
+  for (int64_t r = threadIdx.x; r < row; r += blockDim.x) {
+    bool all;
+    s += vanilla_len(alen, r, fb_n, all);
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+}
+// After it.
+__device__ __forceinline__ CsrRow csr_row(const CsrOut& co, int64_t row, int n, const long long* part, float* pre,
+                                          float* post) {
+  CsrRow r{0, false, pre, post};
+  if (!co.off) return r;
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) r.o += part[w];
+  if (blockIdx.y == 0 && threadIdx.x == 0) {
+    co.off[row] = r.o;
+    if (row == co.batch - 1) co.off[co.batch] = r.o + n;
+  }
+  r.direct = r.o + n <= co.capacity;
+  if (r.direct && co.pre) r.pre = co.pre + r.o;
+  if (r.direct && co.act) r.act = co.act + r.o;
+  return r;
+}
+// The head of a row that does not fit, each thread the entries a0, a0 + astep, ...
+__device__ __forceinline__ void csr_spill(const CsrOut& co, const CsrRow& r, int n, int a0, int astep) {
+  if (!co.off || r.direct) return;
+  for (int a = a0; a < n && r.o + a < co.capacity; a += astep) {
+    if (co.pre) co.pre[r.o + a] = r.pre[a];
+    if (co.act) co.act[r.o + a] = r.act[a];
+  }
+}
+
 // Latency bound: few waves, each a chain of loads.  So a row of x is read kRowLoads
 // values a thread at a time and its nonzeros placed by ballots and one barrier, and
 // the weights of kEntries nonzeros are in flight while those before them are summed
@@ -366,16 +419,18 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     const float* __restrict__ x, const int64_t* __restrict__ xoff,
     const uint32_t* __restrict__ xidx, const float* __restrict__ xval,
     uint32_t* __restrict__ aids, int astride, const int32_t* __restrict__ alen, int act,
-    int max_nz, float* __restrict__ pre, float* __restrict__ post, int fb_n = 0,
-    int32_t* __restrict__ alen_out = nullptr) {
+    int max_nz, float* __restrict__ pre, float* __restrict__ post, int fb_n,
+    int32_t* __restrict__ alen_out, CsrOut co) {
   extern __shared__ unsigned char smem[];   // max_nz: a multiple of 2 * kEntries
   uint32_t* nzi = reinterpret_cast<uint32_t*>(smem);
   float* nzv = reinterpret_cast<float*>(smem + sizeof(uint32_t) * max_nz);
   __shared__ int wcnt[kRowLoads * (kSlideThreads / 64)];
   __shared__ float red[kSlideThreads / 64];
+  __shared__ long long part[kSlideThreads / 64];
   const int64_t row = blockIdx.x;
   bool all;
   const int n = vanilla_len(alen, row, fb_n, all);
+  csr_part(co, alen, row, fb_n, part);
   int nnz;
   int64_t xa = 0;
   if (SPARSE) {
@@ -398,14 +453,18 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     }
   __syncthreads();
   uint32_t* ids = aids + row * (int64_t)astride;
-  float* prow = pre + row * (int64_t)astride;
-  float* orow = post + row * (int64_t)astride;
+  const CsrRow cr = csr_row(co, row, n, part, pre + row * (int64_t)astride, post + row * (int64_t)astride);
+  float *prow = cr.pre, *orow = cr.act;
   if (alen_out && blockIdx.y == 0 && threadIdx.x == 0) alen_out[row] = n;
   float lmax = -INFINITY;
   const int a0 = threadIdx.x + blockIdx.y * blockDim.x, astep = blockDim.x * gridDim.y;
   for (int a = a0; a < n; a += astep) {
     const uint32_t id = all ? (uint32_t)a : ids[a];
-    if (all) ids[a] = id;
+    if (!co.off) {
+      if (all) ids[a] = id;
+    } else if (cr.o + a < co.capacity) {
+      co.ids[cr.o + a] = id;
+    }
     const float bi = bias[id];
     const float* __restrict__ wl = TRANS ? W + id : W + (size_t)id * dim;   // this lane's weights
     float s = -0.0f;
@@ -428,7 +487,7 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     else if (act == KH_ACT_TANH) orow[a] = tanhf(z);
     else if (act != KH_ACT_SOFTMAX) orow[a] = z;
   }
-  if (act != KH_ACT_SOFTMAX) return;
+  if (act != KH_ACT_SOFTMAX) return csr_spill(co, cr, n, a0, astep);
   // softmax over the active set (layer.rs:286-308)
   lmax = wave_max(lmax);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lmax;
@@ -453,6 +512,7 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     const float u = 1.0f / (float)n;
     for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = u;
   }
+  csr_spill(co, cr, n, threadIdx.x, blockDim.x);   // its own entries (one block per row)
 }
 
 // Row-major layers over dense inputs of at most kTileMaxDim features (cfg5's
@@ -477,16 +537,18 @@ constexpr size_t tile_lds(int waves) { return sizeof(float) * waves * kTileN * k
 __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     const float* __restrict__ W, const float* __restrict__ bias, int dim, const float* __restrict__ x,
     uint32_t* __restrict__ aids, int astride, const int32_t* __restrict__ alen, int act,
-    float* __restrict__ pre, float* __restrict__ post, int fb_n = 0,
-    int32_t* __restrict__ alen_out = nullptr, float* __restrict__ dense = nullptr, int64_t dense_ld = 0) {
+    float* __restrict__ pre, float* __restrict__ post, int fb_n, int32_t* __restrict__ alen_out,
+    float* __restrict__ dense, int64_t dense_ld, CsrOut co) {
   extern __shared__ float tl[];
   __shared__ uint32_t nzi[kTileMaxDim];   // a multiple of 2 * kEntries
   __shared__ float nzv[kTileMaxDim];
   __shared__ int wcnt[kRowLoads * kTileWaves];
   __shared__ float red[kTileWaves];
+  __shared__ long long part[kTileWaves];
   const int64_t row = blockIdx.x;
   const int waves = blockDim.x >> 6;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  csr_part(co, alen, row, fb_n, part);
   const int nnz = row_nonzeros(x + row * (int64_t)dim, dim, nzi, nzv, wcnt);
   for (int i = nnz + threadIdx.x; i < entries_padded(nnz); i += blockDim.x) {
     nzi[i] = 0u;
@@ -496,10 +558,10 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
   bool all;
   const int n = vanilla_len(alen, row, fb_n, all);
   uint32_t* ids = aids + row * (int64_t)astride;
-  float* prow = pre + row * (int64_t)astride;
-  float* orow = post + row * (int64_t)astride;
+  const CsrRow cr = csr_row(co, row, n, part, pre + row * (int64_t)astride, post + row * (int64_t)astride);
+  float *prow = cr.pre, *orow = cr.act;
   if (alen_out && blockIdx.y == 0 && threadIdx.x == 0) alen_out[row] = n;
-  if (all && blockIdx.y == 0)
+  if (all && !co.off && blockIdx.y == 0)
     for (int a = threadIdx.x; a < n; a += blockDim.x) ids[a] = (uint32_t)a;
   float* buf = tl + (size_t)wave * kTileN * kTileStride;
   const int q4 = dim >> 2;              // float4 per weight row (<= 32)
@@ -553,6 +615,7 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     if (a < n) {
       const float z = __fadd_rn(s, bi);
       prow[a] = z;
+      if (co.off && cr.o + a < co.capacity) co.ids[cr.o + a] = id;
       lmax = fmaxf(lmax, z);
       if (act != KH_ACT_SOFTMAX) {
         float r;
@@ -565,7 +628,11 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
       }
     }
   }
-  if (act != KH_ACT_SOFTMAX || gridDim.y > 1) return;
+  if (act != KH_ACT_SOFTMAX || gridDim.y > 1) {
+    if (!co.off || cr.direct) return;
+    __syncthreads();   // the entries are other lanes'
+    return csr_spill(co, cr, n, threadIdx.x, blockDim.x);   // (one block per row with a CsrOut)
+  }
   // softmax over the active set (layer.rs:286-308), as neuron_kernel
   lmax = wave_max(lmax);
   if (lane == 0) red[wave] = lmax;
@@ -590,6 +657,7 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     const float u = 1.0f / (float)n;
     for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = u;
   }
+  csr_spill(co, cr, n, threadIdx.x, blockDim.x);
 }
 
 // neuron_tile_kernel's LDS (above 64 KB) is allowed once per process.
@@ -617,8 +685,8 @@ int neuron_tile_launch(const kh_slide_layer* l, const float* x, int64_t rows, ui
   const int tiles = ceil_div(as, kTileN * kFew);
   const int split = std::max(2, std::min(tiles, std::max(1, 1024 / (int)std::min<int64_t>(rows, 1024))));
   hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)rows, (unsigned)split), dim3(64 * kFew), tile_lds(kFew), st,
-                     l->w, l->bias, l->dim, x, aids, as, alen, l->act, pre, post, 0, (int32_t*)nullptr, dense,
-                     dense_ld);
+                     l->w, l->bias, l->dim, x, aids, as, alen, l->act, pre, post, 0, nullptr, dense,
+                     dense_ld, CsrOut{});
   KH_LAUNCHED();
   return KH_OK;
 }
@@ -798,9 +866,11 @@ static int slide_forward_common(const kh_slide_layer* lc, const float* x, const 
   const int as = std::max(qs, l->n);
   uint32_t* aids = static_cast<uint32_t*>(w->get(4, sizeof(uint32_t) * batch * as));
   int32_t* alen = static_cast<int32_t*>(w->get(5, sizeof(int32_t) * batch));
-  float* pre = static_cast<float*>(w->get(6, sizeof(float) * batch * as));
-  float* post = static_cast<float*>(w->get(7, sizeof(float) * batch * as));
-  if (!codes || !qids || !qcnt || !qlen || !aids || !alen || !pre || !post) return KH_ERR_ALLOC;
+  const bool packed = batch <= kCsrPackMax;   // the kernel writes the CSR rows itself
+  const bool spill = !(packed && pre_out && act_out && capacity >= batch * (int64_t)as);
+  float* pre = spill ? static_cast<float*>(w->get(6, sizeof(float) * batch * as)) : nullptr;
+  float* post = spill ? static_cast<float*>(w->get(7, sizeof(float) * batch * as)) : nullptr;
+  if (!codes || !qids || !qcnt || !qlen || !aids || !alen || (spill && (!pre || !post))) return KH_ERR_ALLOC;
   int rc = xoff ? hash_sparse_launch(idx->h, xoff, xidx, xval, batch, codes, st)
                 : hash_dense_launch(idx->h, x, l->dim, batch, codes, st);
   if (rc != KH_OK) return rc;
@@ -825,27 +895,30 @@ static int slide_forward_common(const kh_slide_layer* lc, const float* x, const 
   // kernel's, and the kernel writes the lengths the outputs use
   const int32_t* ilen = direct ? qlen : alen;
   const int fb_n = direct ? l->n : 0;
-  int32_t* olen = direct ? alen : nullptr;
+  int32_t* olen = direct && !packed ? alen : nullptr;
+  CsrOut co{};
+  if (packed) co = {off, act_ids, pre_out, act_out, batch, capacity};
   if (xoff && l->wtn)
     hipLaunchKernelGGL((neuron_kernel<true, true>), ng, dim3(kSlideThreads), lds, st, l->wtn, l->n,
                        l->bias, l->dim, nullptr, xoff, xidx, xval, aids, as, ilen, act, max_nz,
-                       pre, post, fb_n, olen);
+                       pre, post, fb_n, olen, co);
   else if (xoff)
     hipLaunchKernelGGL((neuron_kernel<true, false>), ng, dim3(kSlideThreads), lds, st, l->w, l->n,
                        l->bias, l->dim, nullptr, xoff, xidx, xval, aids, as, ilen, act, max_nz,
-                       pre, post, fb_n, olen);
+                       pre, post, fb_n, olen, co);
   else if (l->wtn)
     hipLaunchKernelGGL((neuron_kernel<false, true>), ng, dim3(kSlideThreads), lds, st, l->wtn, l->n,
                        l->bias, l->dim, x, nullptr, nullptr, nullptr, aids, as, ilen, act,
-                       max_nz, pre, post, fb_n, olen);
+                       max_nz, pre, post, fb_n, olen, co);
   else if (l->dim <= kTileMaxDim && l->dim % 4 == 0 && tile_kernel_ready() == KH_OK)
     hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)batch), dim3(kSlideThreads), tile_lds(kTileWaves), st, l->w,
-                       l->bias, l->dim, x, aids, as, ilen, act, pre, post, fb_n, olen);
+                       l->bias, l->dim, x, aids, as, ilen, act, pre, post, fb_n, olen, nullptr, 0, co);
   else
     hipLaunchKernelGGL((neuron_kernel<false, false>), ng, dim3(kSlideThreads), lds, st, l->w, l->n,
                        l->bias, l->dim, x, nullptr, nullptr, nullptr, aids, as, ilen, act,
-                       max_nz, pre, post, fb_n, olen);
+                       max_nz, pre, post, fb_n, olen, co);
   KH_LAUNCHED();
+  if (packed) return csr_check(off, batch, as, capacity, st);
   return csr_finish(aids, nullptr, pre, post, as, alen, batch, off, act_ids, nullptr, pre_out,
                     act_out, capacity, st);
 }
