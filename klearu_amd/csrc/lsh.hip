@@ -1606,22 +1606,29 @@ using namespace kh;
 
 // ====================================================================== families
 static int family_finish(kh_hash_family* h, kh_hash_family** out) {
+  // Every loop runs along a plane's bytes without branches on them: a coefficient's
+  // 2-bit sign is its byte & 3 (1: 1, -1: 3), its presence byte & 1.
   const int P = h->L * h->k;
+  const uint8_t* planes = reinterpret_cast<const uint8_t*>(h->planes_host.data());
   std::vector<int32_t> nnz(P, 0);
   for (int p = 0; p < P; ++p) {
-    const int8_t* pl = h->planes_host.data() + (size_t)p * h->dim;
-    for (int d = 0; d < h->dim; ++d) nnz[p] += pl[d] != 0;
+    const uint8_t* pl = planes + (size_t)p * h->dim;
+    int32_t m = 0;
+    for (int d = 0; d < h->dim; ++d) m += pl[d] & 1;
+    nnz[p] = m;
   }
   const int mx = P ? *std::max_element(nnz.begin(), nnz.end()) : 0;
   h->ent_rows = std::max(kHashBatch, (mx + kHashBatch - 1) / kHashBatch * kHashBatch);
-  std::vector<uint32_t> ent((size_t)h->ent_rows * P, 0u);
+  const size_t ent_n = (size_t)h->ent_rows * P;
+  std::vector<uint32_t> ent(ent_n + P, 0u);   // a row more: each dimension is written, then kept or not
   for (int p = 0; p < P; ++p) {
-    const int8_t* pl = h->planes_host.data() + (size_t)p * h->dim;
-    size_t j = 0;
+    const uint8_t* pl = planes + (size_t)p * h->dim;
+    uint32_t* e = ent.data() + p;
     for (int d = 0; d < h->dim; ++d) {
-      if (pl[d] == 1) ent[j++ * P + p] = (uint32_t)d << 1;
-      else if (pl[d] == -1) ent[j++ * P + p] = ((uint32_t)d << 1) | 1u;
+      *e = ((uint32_t)d << 1) | (pl[d] >> 7);
+      e += (size_t)P * (pl[d] & 1);
     }
+    *e = 0u;
   }
   // BF16 copy of the planes in the matrix-core operand order (hashing large
   // dense batches): entry (step, tile, lane) holds 8 k values of one plane
@@ -1630,23 +1637,25 @@ static int family_finish(kh_hash_family* h, kh_hash_family** out) {
     h->bt_ksteps = (h->dim + 31) / 32;
     h->bt_tiles = (P + 15) / 16;
     bt.assign((size_t)h->bt_ksteps * h->bt_tiles * 64 * 8, 0);
-    for (int st = 0; st < h->bt_ksteps; ++st)
-      for (int tile = 0; tile < h->bt_tiles; ++tile)
-        for (int l = 0; l < 64; ++l) {
-          const int p = tile * 16 + (l & 15);
-          for (int i = 0; i < 8; ++i) {
-            const int d = st * 32 + (l >> 4) * 8 + i;
-            const int8_t v = p < P && d < h->dim ? h->planes_host[(size_t)p * h->dim + d] : 0;
-            bt[(((size_t)st * h->bt_tiles + tile) * 64 + l) * 8 + i] = v == 1 ? 0x3F80 : (v == -1 ? 0xBF80 : 0);
-          }
-        }
-    const int spn = (h->dim + 15) / 16;
-    std::vector<uint32_t> sp((size_t)P * spn, 0u);
-    for (int p = 0; p < P; ++p)
-      for (int d = 0; d < h->dim; ++d) {
-        const int8_t v = h->planes_host[(size_t)p * h->dim + d];
-        sp[(size_t)p * spn + d / 16] |= (v == 1 ? 1u : v == -1 ? 3u : 0u) << (2 * (d % 16));
+    for (int p = 0; p < P; ++p) {
+      const uint8_t* pl = planes + (size_t)p * h->dim;
+      for (int d0 = 0; d0 < h->dim; d0 += 8) {
+        uint16_t* e = bt.data() + (((size_t)(d0 / 32) * h->bt_tiles + p / 16) * 64 + (d0 / 8 % 4) * 16 + p % 16) * 8;
+        const int m = std::min(8, h->dim - d0);
+        for (int i = 0; i < m; ++i) e[i] = (uint16_t)((pl[d0 + i] & 1) * 0x3F80 | (pl[d0 + i] & 0x80) << 8);
       }
+    }
+    const int spn = (h->dim + 15) / 16;
+    std::vector<uint32_t> sp((size_t)P * spn);
+    for (int p = 0; p < P; ++p) {
+      const uint8_t* pl = planes + (size_t)p * h->dim;
+      for (int w = 0; w < spn; ++w) {
+        const int m = std::min(16, h->dim - w * 16);
+        uint32_t v = 0u;
+        for (int i = 0; i < m; ++i) v |= (uint32_t)(pl[w * 16 + i] & 3) << (2 * i);
+        sp[(size_t)p * spn + w] = v;
+      }
+    }
     h->bt_dev = static_cast<uint4*>(dev_alloc(sizeof(uint16_t) * bt.size()));
     h->sp_dev = static_cast<uint32_t*>(dev_alloc(sizeof(uint32_t) * sp.size()));
     if (!h->bt_dev || !h->sp_dev) {
@@ -1669,15 +1678,18 @@ static int family_finish(kh_hash_family* h, kh_hash_family** out) {
     h->sg_words = (h->sg_tpb * h->k + 15) / 16;
     h->sg_n4 = static_cast<int>(((int64_t)h->dim * h->sg_words + 3) / 4);
     std::vector<uint32_t> sg((size_t)h->sg_groups * h->sg_n4 * 4, 0u);
+    std::vector<uint32_t> col(h->dim);   // one word of every dimension
     for (int g = 0; g < h->sg_groups; ++g)
-      for (int q = 0; q < h->sg_tpb * h->k; ++q) {
-        const int p = g * h->sg_tpb * h->k + q;
-        if (p >= P) break;
-        const int8_t* pl = h->planes_host.data() + (size_t)p * h->dim;
-        for (int d = 0; d < h->dim; ++d) {
-          const uint32_t code = pl[d] == 1 ? 1u : (pl[d] == -1 ? 3u : 0u);
-          sg[(size_t)g * h->sg_n4 * 4 + (size_t)d * h->sg_words + q / 16] |= code << (2 * (q % 16));
+      for (int w = 0; w < h->sg_words; ++w) {
+        const int q0 = w * 16, q1 = std::min({q0 + 16, h->sg_tpb * h->k, P - g * h->sg_tpb * h->k});
+        if (q0 >= q1) break;
+        std::fill(col.begin(), col.end(), 0u);
+        for (int q = q0; q < q1; ++q) {
+          const uint8_t* pl = planes + (size_t)(g * h->sg_tpb * h->k + q) * h->dim;
+          for (int d = 0; d < h->dim; ++d) col[d] |= (uint32_t)(pl[d] & 3) << (2 * (q - q0));
         }
+        uint32_t* dst = sg.data() + (size_t)g * h->sg_n4 * 4 + w;
+        for (int d = 0; d < h->dim; ++d) dst[(size_t)d * h->sg_words] = col[d];
       }
     h->sg_dev = static_cast<uint4*>(dev_alloc(sizeof(uint32_t) * sg.size()));
     if (!h->sg_dev) {
@@ -1691,13 +1703,13 @@ static int family_finish(kh_hash_family* h, kh_hash_family** out) {
     }
   }
   h->nnz = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * std::max(P, 1)));
-  h->ent_t = static_cast<uint32_t*>(dev_alloc(sizeof(uint32_t) * ent.size()));
+  h->ent_t = static_cast<uint32_t*>(dev_alloc(sizeof(uint32_t) * ent_n));
   if (!h->nnz || !h->ent_t) {
     kh_hash_family_destroy(h);
     return KH_ERR_ALLOC;
   }
   if (hipMemcpy(h->nnz, nnz.data(), sizeof(int32_t) * P, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(h->ent_t, ent.data(), sizeof(uint32_t) * ent.size(), hipMemcpyHostToDevice) != hipSuccess) {
+      hipMemcpy(h->ent_t, ent.data(), sizeof(uint32_t) * ent_n, hipMemcpyHostToDevice) != hipSuccess) {
     set_error("plane upload failed");
     kh_hash_family_destroy(h);
     return KH_ERR_HIP;
