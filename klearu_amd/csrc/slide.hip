@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "gather.hpp"
+#include "entry_sum.hpp"
 #include "slide_internal.hpp"
 
 namespace kh {
@@ -345,15 +346,15 @@ __device__ __forceinline__ void csr_spill(const CsrOut& co, const CsrRow& r, int
 // values a thread at a time and its nonzeros placed by ballots and one barrier, and
 // the weights of kEntries nonzeros are in flight while those before them are summed
 // (the list is padded to 2 * kEntries entries, whose products are replaced by -0.0).
-// 128 rows of 784, 1024 neurons: 16.5 us, 20 with a block scan per 256 values of x and
-// loads where they are used.
+// 128 rows of 784, 1024 neurons: 14.2 us (16.5 with 64-bit offsets), 20 with a block
+// scan per 256 values of x and loads where they are used.
 constexpr int kRowLoads = 4;
-constexpr int kEntries = 16;
-__host__ __device__ constexpr int entries_padded(int nnz) { return (nnz + 2 * kEntries - 1) / (2 * kEntries) * (2 * kEntries); }
 
-// The nonzeros of xr[0..dim) in ascending order to nzi/nzv; returns their count.  wcnt:
-// kRowLoads words per wave.  A barrier follows before the lists are read.
-__device__ __forceinline__ int row_nonzeros(const float* __restrict__ xr, int dim, uint32_t* nzi, float* nzv, int* wcnt) {
+// The nonzeros of xr[0..dim) in ascending order, d * mul to nzi and values to nzv;
+// returns their count.  wcnt: kRowLoads words per wave.  A barrier follows before the
+// lists are read.
+__device__ __forceinline__ int row_nonzeros(const float* __restrict__ xr, int dim, uint32_t mul, uint32_t* nzi,
+                                            float* nzv, int* wcnt) {
   const int waves = blockDim.x >> 6, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   int base = 0;
   for (int c0 = 0; c0 < dim; c0 += kRowLoads * blockDim.x) {
@@ -378,39 +379,12 @@ __device__ __forceinline__ int row_nonzeros(const float* __restrict__ xr, int di
       }
       if ((m[u] >> lane) & 1ull) {
         pos += __popcll(m[u] & ((1ull << lane) - 1ull));
-        nzi[pos] = (uint32_t)(c0 + u * (int)blockDim.x + (int)threadIdx.x);
+        nzi[pos] = (uint32_t)(c0 + u * (int)blockDim.x + (int)threadIdx.x) * mul;
         nzv[pos] = v[u];
       }
     }
   }
   return base;
-}
-
-// sum_e weight(nzi[e]) * nzv[e] in order, from -0.0; nnz > 0, lists padded.
-template <typename W>
-__device__ __forceinline__ float sum_entries(const uint32_t* nzi, const float* nzv, int nnz, W&& weight) {
-  const int npad = entries_padded(nnz);
-  float s = -0.0f, w0[kEntries], w1[kEntries];
-  auto load = [&](float (&w)[kEntries], int e0) {
-#pragma unroll
-    for (int u = 0; u < kEntries; ++u) w[u] = weight(nzi[e0 + u]);
-  };
-  auto add = [&](const float (&w)[kEntries], int e0) {
-#pragma unroll
-    for (int u = 0; u < kEntries; ++u) {
-      const float p = __fmul_rn(w[u], nzv[e0 + u]);
-      s = __fadd_rn(s, e0 + u < nnz ? p : -0.0f);
-    }
-    asm volatile("" : "+v"(s));   // these sums stay ahead of the next loads
-  };
-  load(w0, 0);
-  for (int e0 = 0; e0 < npad; e0 += 2 * kEntries) {
-    load(w1, e0 + kEntries);
-    add(w0, e0);
-    load(w0, min(e0 + 2 * kEntries, npad - kEntries));
-    add(w1, e0 + kEntries);
-  }
-  return s;
 }
 
 template <bool SPARSE, bool TRANS>
@@ -431,6 +405,8 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
   bool all;
   const int n = vanilla_len(alen, row, fb_n, all);
   csr_part(co, alen, row, fb_n, part);
+  const bool fit = TRANS && offsets_fit(dim, nn);
+  const uint32_t mul = fit ? (uint32_t)nn : 1u;   // of the indices in LDS
   int nnz;
   int64_t xa = 0;
   if (SPARSE) {
@@ -438,11 +414,11 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     nnz = (int)(xoff[row + 1] - xa);
     if (nnz <= max_nz)
       for (int i = threadIdx.x; i < nnz; i += blockDim.x) {
-        nzi[i] = xidx[xa + i];
+        nzi[i] = xidx[xa + i] * mul;
         nzv[i] = xval[xa + i];
       }
   } else {
-    nnz = row_nonzeros(x + row * (int64_t)dim, dim, nzi, nzv, wcnt);
+    nnz = row_nonzeros(x + row * (int64_t)dim, dim, mul, nzi, nzv, wcnt);
   }
   const bool in_lds = !SPARSE || nnz <= max_nz;
   const int npad = entries_padded(nnz);
@@ -468,11 +444,10 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     const float bi = bias[id];
     const float* __restrict__ wl = TRANS ? W + id : W + (size_t)id * dim;   // this lane's weights
     float s = -0.0f;
-    if (in_lds && nnz) {
-      s = sum_entries(nzi, nzv, nnz, [&](uint32_t d) {
-        const size_t q = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
-        return wl[TRANS ? q * nn : q];
-      });
+    if (in_lds && nnz && fit) {
+      s = sum_entries(nzi, nzv, nnz, [&](uint32_t q) { return weight_at(W, id + q); });
+    } else if (in_lds && nnz) {
+      s = sum_entries(nzi, nzv, nnz, [&](uint32_t d) { return wl[TRANS ? (size_t)d * nn : d]; });
     } else {
       for (int e = 0; e < nnz; ++e) {
         const size_t d = xidx[xa + e];
@@ -549,7 +524,7 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
   const int waves = blockDim.x >> 6;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   csr_part(co, alen, row, fb_n, part);
-  const int nnz = row_nonzeros(x + row * (int64_t)dim, dim, nzi, nzv, wcnt);
+  const int nnz = row_nonzeros(x + row * (int64_t)dim, dim, 1u, nzi, nzv, wcnt);
   for (int i = nnz + threadIdx.x; i < entries_padded(nnz); i += blockDim.x) {
     nzi[i] = 0u;
     nzv[i] = 0.0f;
