@@ -387,6 +387,49 @@ __device__ __forceinline__ int row_nonzeros(const float* __restrict__ xr, int di
   return base;
 }
 
+// Softmax over a row's active set (layer.rs:286-308) from prow to orow, by a block of at
+// least kSlideThreads threads; lmax: the thread's largest value.  The sum keeps one
+// order: thread t < kSlideThreads adds entries t, t + kSlideThreads, ..., then waves,
+// then the block.  kSmLoads values are in flight, and the exponentials stay in LDS (eb,
+// room for ecap; free once every thread is here) between the passes, where each value
+// and pass was a round trip to the caches.
+constexpr int kSmLoads = 8;
+__device__ __forceinline__ void softmax_row(float lmax, const float* prow, float* orow, int n, float* red, float* eb,
+                                            int ecap) {
+  constexpr int kWaves = kSlideThreads / 64;
+  const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  lmax = wave_max(lmax);
+  if ((threadIdx.x & 63) == 0) red[wave] = lmax;
+  __syncthreads();
+  float mx = red[0];
+  for (int i = 1; i < waves; ++i) mx = fmaxf(mx, red[i]);
+  __syncthreads();
+  float* e_out = n <= ecap ? eb : orow;
+  if (wave < kWaves) {
+    float ls = 0.0f;
+    for (int a = threadIdx.x; a < n; a += kSlideThreads * kSmLoads) {
+      float z[kSmLoads];
+#pragma unroll
+      for (int u = 0; u < kSmLoads; ++u) z[u] = prow[min(a + u * kSlideThreads, n - 1)];
+#pragma unroll
+      for (int u = 0; u < kSmLoads; ++u) {
+        if (a + u * kSlideThreads < n) {
+          const float e = expf_glibc(z[u] - mx);
+          e_out[a + u * kSlideThreads] = e;
+          ls += e;
+        }
+      }
+    }
+    ls = wave_sum(ls);
+    if ((threadIdx.x & 63) == 0) red[wave] = ls;
+  }
+  __syncthreads();
+  float tot = 0.0f;
+  for (int i = 0; i < kWaves; ++i) tot += red[i];
+  const float uniform = 1.0f / (float)n;
+  for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = tot > 0.0f ? e_out[a] / tot : uniform;
+}
+
 template <bool SPARSE, bool TRANS>
 __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     const float* __restrict__ W, int nn, const float* __restrict__ bias, int dim,
@@ -463,53 +506,34 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
     else if (act != KH_ACT_SOFTMAX) orow[a] = z;
   }
   if (act != KH_ACT_SOFTMAX) return csr_spill(co, cr, n, a0, astep);
-  // softmax over the active set (layer.rs:286-308)
-  lmax = wave_max(lmax);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lmax;
-  __syncthreads();
-  float mx = red[0];
-  for (int i = 1; i < (int)(blockDim.x >> 6); ++i) mx = fmaxf(mx, red[i]);
-  __syncthreads();
-  float ls = 0.0f;
-  for (int a = threadIdx.x; a < n; a += blockDim.x) {
-    const float e = expf_glibc(prow[a] - mx);
-    orow[a] = e;
-    ls += e;
-  }
-  ls = wave_sum(ls);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ls;
-  __syncthreads();
-  float tot = 0.0f;
-  for (int i = 0; i < (int)(blockDim.x >> 6); ++i) tot += red[i];
-  if (tot > 0.0f) {
-    for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = orow[a] / tot;
-  } else {
-    const float u = 1.0f / (float)n;
-    for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = u;
-  }
+  softmax_row(lmax, prow, orow, n, red, reinterpret_cast<float*>(smem), 2 * max_nz);
   csr_spill(co, cr, n, threadIdx.x, blockDim.x);   // its own entries (one block per row)
 }
 
 // Row-major layers over dense inputs of at most kTileMaxDim features (cfg5's
-// output layer): each wave takes 64 active neurons at a time and loads their
+// output layer): each wave takes 32 active neurons at a time and loads their
 // weight rows cooperatively, 32 lanes per 512-byte row (two whole rows per load
 // instruction, instead of 64 scattered rows per instruction), into an LDS tile
 // whose odd row stride makes the per-lane column reads conflict-free; lane j
 // then runs neuron j's sequential sum over the input's nonzeros (ascending, as
 // neuron_kernel does).  The next tile's loads are in flight during the sums, which
 // have to be shorter than those loads take: sixteen LDS reads are in flight ahead of
-// them.  256 rows of 128, 6400 of 670091 neurons each: 146 us (5.7 TB/s), 158 with
-// each product read where it is added.
+// them.  Two waves per SIMD, so that loads also run while one of them fills its tile
+// (a tile of 64, which has a lane for every lane, leaves room for one).
+// 256 rows of 128, 6400 of 670091 neurons each: 135 us (6.2 TB/s); 147 us with tiles of
+// 64 and a round trip per value in the softmax, 158 with each product read where it is
+// added.
 // With several blocks per row (gridDim.y) the tiles are dealt over them and a
 // softmax layer's activations are left to another kernel; `dense`, when given,
 // also gets the activations at their ids.
-constexpr int kTileN = 64;
+constexpr int kTileN = 32;
 constexpr int kTileStride = 129;   // floats per LDS row
 constexpr int kTileMaxDim = 128;
-constexpr int kTileWaves = kSlideThreads / 64;   // waves per block at most (two at least)
+constexpr int kTileWaves = 8;      // waves per block at most (two at least)
+constexpr int kTileThreads = 64 * kTileWaves;
 constexpr size_t tile_lds(int waves) { return sizeof(float) * waves * kTileN * kTileStride; }
 
-__global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
+__global__ __launch_bounds__(kTileThreads) void neuron_tile_kernel(
     const float* __restrict__ W, const float* __restrict__ bias, int dim, const float* __restrict__ x,
     uint32_t* __restrict__ aids, int astride, const int32_t* __restrict__ alen, int act,
     float* __restrict__ pre, float* __restrict__ post, int fb_n, int32_t* __restrict__ alen_out,
@@ -540,13 +564,13 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     for (int a = threadIdx.x; a < n; a += blockDim.x) ids[a] = (uint32_t)a;
   float* buf = tl + (size_t)wave * kTileN * kTileStride;
   const int q4 = dim >> 2;              // float4 per weight row (<= 32)
-  const int c = lane & 31;              // this lane's float4 of a row
+  const int c = lane & 31;              // this lane's float4 of a row, and its neuron of a tile
   const int half = lane >> 5;           // which of the two rows of a load
   const int ntiles = (n + kTileN - 1) / kTileN;
   float4 v[kTileN / 2];
-  // neuron t*64 + lane of tile t (clamped to the last active id)
+  // neuron c of tile t (clamped to the last active id), the same in both halves
   auto id_of = [&](int t) {
-    const int ia = min(t * kTileN + lane, n - 1);
+    const int ia = min(t * kTileN + c, n - 1);
     return all ? (uint32_t)ia : ids[ia];
   };
   // the rows of the next tile, whose ids came with the one before it
@@ -584,10 +608,10 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
       }
     }
     if (t + tstep < ntiles) issue(t + 2 * tstep);
-    const int a = t * kTileN + lane;
-    const float* wr = buf + lane * kTileStride;
+    const int a = t * kTileN + c;
+    const float* wr = buf + c * kTileStride;
     const float s = nnz ? sum_entries(nzi, nzv, nnz, [&](uint32_t d) { return wr[d]; }) : -0.0f;
-    if (a < n) {
+    if (a < n && half == 0) {
       const float z = __fadd_rn(s, bi);
       prow[a] = z;
       if (co.off && cr.o + a < co.capacity) co.ids[cr.o + a] = id;
@@ -608,30 +632,7 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_tile_kernel(
     __syncthreads();   // the entries are other lanes'
     return csr_spill(co, cr, n, threadIdx.x, blockDim.x);   // (one block per row with a CsrOut)
   }
-  // softmax over the active set (layer.rs:286-308), as neuron_kernel
-  lmax = wave_max(lmax);
-  if (lane == 0) red[wave] = lmax;
-  __syncthreads();
-  float mx = red[0];
-  for (int i = 1; i < kTileWaves; ++i) mx = fmaxf(mx, red[i]);
-  __syncthreads();
-  float ls = 0.0f;
-  for (int a = threadIdx.x; a < n; a += blockDim.x) {
-    const float e = expf_glibc(prow[a] - mx);
-    orow[a] = e;
-    ls += e;
-  }
-  ls = wave_sum(ls);
-  if (lane == 0) red[wave] = ls;
-  __syncthreads();
-  float tot = 0.0f;
-  for (int i = 0; i < kTileWaves; ++i) tot += red[i];
-  if (tot > 0.0f) {
-    for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = orow[a] / tot;
-  } else {
-    const float u = 1.0f / (float)n;
-    for (int a = threadIdx.x; a < n; a += blockDim.x) orow[a] = u;
-  }
+  softmax_row(lmax, prow, orow, n, red, tl, waves * kTileN * kTileStride);
   csr_spill(co, cr, n, threadIdx.x, blockDim.x);
 }
 
@@ -886,7 +887,7 @@ static int slide_forward_common(const kh_slide_layer* lc, const float* x, const 
                        l->bias, l->dim, x, nullptr, nullptr, nullptr, aids, as, ilen, act,
                        max_nz, pre, post, fb_n, olen, co);
   else if (l->dim <= kTileMaxDim && l->dim % 4 == 0 && tile_kernel_ready() == KH_OK)
-    hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)batch), dim3(kSlideThreads), tile_lds(kTileWaves), st, l->w,
+    hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)batch), dim3(kTileThreads), tile_lds(kTileWaves), st, l->w,
                        l->bias, l->dim, x, aids, as, ilen, act, pre, post, fb_n, olen, nullptr, 0, co);
   else
     hipLaunchKernelGGL((neuron_kernel<false, false>), ng, dim3(kSlideThreads), lds, st, l->w, l->n,
