@@ -177,13 +177,16 @@ __global__ __launch_bounds__(kL1LdsThreads) void pred_l1_lds_kernel(
 //    once the consumer has released that slot, then publishes the stage index
 //    in ready[slot]; the consumer releases a slot by writing the stage index
 //    to freed[slot].  LDS flags, not barriers: no wave waits for another
-//    except on the data it needs.  One consumer and three producers, one wave
-//    per SIMD, so no producer takes issue slots from the chain.
+//    except on the data it needs.  One consumer and six producers, two on each
+//    of the other three SIMDs, so no producer takes issue slots from the chain; the
+//    wave that shares the consumer's SIMD only stages x.  A stage costs its producer
+//    two LDS round trips and the write's wait: three producers just kept pace and held
+//    the chain up (16 rows of 4096 x 256: the call took 1.7 us more).
 //  * Quad q of chain c sits at position c ^ (q & 14) of its ring row: the
 //    consumer's 16 lanes still read one contiguous row, and a producer's
 //    write instruction (8 quads x 8 chains) spreads evenly over the banks
 //    instead of hitting one bank group 8 times.  Eight slots of 64 steps give
-//    a producer six stages of slack to refill a slot: it takes about three
+//    a producer five stages of slack to refill a slot: it takes about three
 //    times as long to form a stage as the consumer takes to add one.
 //  * The consumer adds each chain's products in step order through a window
 //    of two stages of quads: while stage s is added, its registers are
@@ -193,8 +196,9 @@ __global__ __launch_bounds__(kL1LdsThreads) void pred_l1_lds_kernel(
 // Each chain is the same sequential sum as pred_l1_lds_kernel's.
 constexpr int kLbOut = 8, kLbRows = 2, kLbChains = kLbOut * kLbRows;
 static_assert(kLbChains == 16 || kLbChains == 32, "the ring swizzle c ^ (q & 14) stays inside a row");
-constexpr int kLbStage = 64, kLbSlots = 8, kLbProd = 3;
-constexpr int kLbThreads = 64 * (1 + kLbProd);
+constexpr int kLbStage = 64, kLbSlots = 8, kLbProd = 6;
+constexpr int kLbThreads = 64 * (2 + kLbProd);
+constexpr int kLbIdle = 4;  // the wave that shares the consumer's SIMD (wave w is on SIMD w % 4)
 constexpr int kLbStages = kL1LdsIn / kLbStage;
 constexpr int kLbSpp = (kLbStages + kLbProd - 1) / kLbProd;  // stages per producer (at most)
 constexpr int kLbQuads = kLbStage / 4;
@@ -250,10 +254,10 @@ __global__ __launch_bounds__(kLbThreads) void pred_l1_batch_kernel(
     ready[threadIdx.x] = -1;
     freed[threadIdx.x] = -1;
   }
-  // producer p = wave - 1: lane -> (8-step block jl of a stage, output o)
-  const int p = wave - 1, jl = lane >> 3, po = lane & 7;
+  // producer p (waves 1-3, 5-7): lane -> (8-step block jl of a stage, output o)
+  const int p = wave < kLbIdle ? wave - 1 : wave - 2, jl = lane >> 3, po = lane & 7;
   uint4 wr[kLbSpp];
-  if (wave > 0) {
+  if (wave > 0 && wave != kLbIdle) {
     const uint4* __restrict__ wv = reinterpret_cast<const uint4*>(Wb);
 #pragma unroll
     for (int i = 0; i < kLbSpp; ++i) {
@@ -265,6 +269,7 @@ __global__ __launch_bounds__(kLbThreads) void pred_l1_batch_kernel(
   for (int q = 0; q < kXq; ++q)
     reinterpret_cast<float4*>(xs)[min((int)threadIdx.x + q * kLbThreads, kLbRows * n4 - 1)] = xv[q];
   lds_barrier();
+  if (wave == kLbIdle) return;
   bool gave_up = false;
   if (wave > 0) {
 #pragma unroll
