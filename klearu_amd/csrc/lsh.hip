@@ -1131,6 +1131,51 @@ __device__ __forceinline__ uint32_t query_buckets(const uint32_t* __restrict__ q
   return bstart[L];
 }
 
+// put(id) for every entry of the query's buckets: 16 lanes to a bucket, which finds its
+// entries without a search (a binary search over bstart is a chain of LDS reads per
+// entry).  TU buckets x EU entries per lane are in flight.
+constexpr int kBucketLanes = 16;
+template <int TU, int EU, typename Put>
+__device__ __forceinline__ void bucket_entries(const uint32_t* __restrict__ data, const uint32_t* bstart,
+                                               const uint32_t* bslot, int L, int cap, Put put) {
+  const int grp = threadIdx.x / kBucketLanes, li = threadIdx.x % kBucketLanes, ng = blockDim.x / kBucketLanes;
+  for (int t0 = grp; t0 < L; t0 += ng * TU) {
+    uint32_t n[TU], most = 0;
+    const uint32_t* p[TU];
+#pragma unroll
+    for (int u = 0; u < TU; ++u) {
+      const int t = min(t0 + u * ng, L - 1);
+      n[u] = t0 + u * ng < L ? bstart[t + 1] - bstart[t] : 0u;
+      p[u] = data + (size_t)bslot[t] * cap;
+      most = max(most, n[u]);
+    }
+    for (uint32_t i0 = li; i0 < most; i0 += kBucketLanes * EU) {
+      uint32_t id[TU][EU];
+#pragma unroll
+      for (int u = 0; u < TU; ++u)
+#pragma unroll
+        for (int e = 0; e < EU; ++e)  // clamped (cap >= 1), unconditional
+          id[u][e] = p[u][min(i0 + e * kBucketLanes, max(n[u], 1u) - 1u)];
+#pragma unroll
+      for (int u = 0; u < TU; ++u)
+#pragma unroll
+        for (int e = 0; e < EU; ++e)
+          if (i0 + e * kBucketLanes < n[u]) put(id[u][e]);
+    }
+  }
+}
+
+// m: entries in all.  Full buckets want one bucket's entries in flight, short ones several
+// buckets.
+template <typename Put>
+__device__ __forceinline__ void for_bucket_entries(const uint32_t* __restrict__ data, const uint32_t* bstart,
+                                                   const uint32_t* bslot, int L, int cap, uint32_t m, Put put) {
+  if (m > (uint32_t)L * 2 * kBucketLanes)
+    bucket_entries<1, 8>(data, bstart, bslot, L, cap, put);
+  else
+    bucket_entries<4, 2>(data, bstart, bslot, L, cap, put);
+}
+
 // One block per query row: unique bucket ids in ascending order with counts.
 // Direct path (ids < kDirectIds): a count per id in LDS, then two passes over the
 // ids, each wave on its own run of them, 64 adjacent ids a step (a run per thread
@@ -1151,15 +1196,7 @@ __global__ __launch_bounds__(kQueryBigThreads) void query_direct_kernel(
   uint32_t* ocnt = out_cnt ? out_cnt + row * (int64_t)stride : nullptr;
   for (uint32_t i = threadIdx.x; i < id_bound; i += blockDim.x) sm[i] = 0u;
   const uint32_t m = query_buckets(qcodes, row, L, k, len, bstart, bslot, wsum, &s_total);
-  // every bucket entry of every table, kQueryBatch per thread in flight
-  for (uint32_t i0 = threadIdx.x; i0 < m; i0 += blockDim.x * kQueryBatch) {
-    uint32_t id[kQueryBatch];
-#pragma unroll
-    for (int q = 0; q < kQueryBatch; ++q) id[q] = data[bucket_entry(bstart, bslot, L, cap, min(i0 + q * blockDim.x, m - 1))];
-#pragma unroll
-    for (int q = 0; q < kQueryBatch; ++q)
-      if (i0 + q * blockDim.x < m) atomicAdd(&sm[id[q]], 1u);
-  }
+  for_bucket_entries(data, bstart, bslot, L, cap, m, [&](uint32_t id) { atomicAdd(&sm[id], 1u); });
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
   const uint32_t R = (id_bound + blockDim.x - 1) / blockDim.x * 64;   // ids per wave
@@ -1226,14 +1263,7 @@ __global__ __launch_bounds__(kQueryBigThreads) void query_bitmap_kernel(
   if (ocnt)
     for (int i = threadIdx.x; i < L * cap; i += blockDim.x) cnt[i] = 0u;
   const uint32_t m = query_buckets(qcodes, row, L, k, len, bstart, bslot, wsum, &s_total);
-  for (uint32_t i0 = threadIdx.x; i0 < m; i0 += blockDim.x * kQueryBatch) {
-    uint32_t id[kQueryBatch];
-#pragma unroll
-    for (int q = 0; q < kQueryBatch; ++q) id[q] = data[bucket_entry(bstart, bslot, L, cap, min(i0 + q * blockDim.x, m - 1))];
-#pragma unroll
-    for (int q = 0; q < kQueryBatch; ++q)
-      if (i0 + q * blockDim.x < m) atomicOr(&bm[id[q] >> 5], 1u << (id[q] & 31u));
-  }
+  for_bucket_entries(data, bstart, bslot, L, cap, m, [&](uint32_t id) { atomicOr(&bm[id >> 5], 1u << (id & 31u)); });
   __syncthreads();
   int base = 0;
   for (int g0 = 0; g0 < G; g0 += blockDim.x) {
