@@ -960,7 +960,12 @@ struct kh_slide_network {
   uint64_t step = 0;
   kh_rebuild_scheduler sched{};
   float* loss_total = nullptr;
-  float* x_dense = nullptr;  // [in_dim] the current sparse example, densified
+  // The current sparse example: its nonzeros, and the same densified [in_dim].  Apart from
+  // a dense example's list (b[0]), as the next one clears x_dense at these entries.
+  uint32_t* x_nzi = nullptr;
+  float* x_nzv = nullptr;
+  int64_t* x_off = nullptr;
+  float* x_dense = nullptr;
   uint32_t* labels = nullptr;
   size_t labels_cap = 0;
   kh::Scratch rows_ws;       // net_predict_rows' buffers
@@ -1033,8 +1038,11 @@ extern "C" int kh_slide_network_create(kh_slide_layer* const* layers, int n_laye
   }
   if (rc == KH_OK) {
     net->loss_total = net->alloc<float>(1, true);
+    net->x_nzi = net->alloc<uint32_t>(net->in_dim);
+    net->x_nzv = net->alloc<float>(net->in_dim);
+    net->x_off = net->alloc<int64_t>(2, true);
     net->x_dense = net->alloc<float>(net->in_dim, true);
-    if (!net->loss_total || !net->x_dense) rc = KH_ERR_ALLOC;
+    if (!net->loss_total || !net->x_nzi || !net->x_nzv || !net->x_off || !net->x_dense) rc = KH_ERR_ALLOC;
   }
   if (rc != KH_OK) {
     kh_slide_network_destroy(net);
@@ -1047,9 +1055,8 @@ extern "C" int kh_slide_network_create(kh_slide_layer* const* layers, int n_laye
 // Stage example e of a CSR batch as layer 0's input (to_dense semantics).
 static int net_stage_sparse(kh_slide_network* net, const int64_t* xoff, const uint32_t* xidx,
                             const float* xval, int64_t e, hipStream_t st) {
-  TrainBufs& t = net->b[0];
   hipLaunchKernelGGL(tr_stage_csr_kernel, dim3(1), dim3(1024), 0, st, xoff, xidx, xval, e,
-                     net->in_dim, (int64_t)0, t.nzi, t.nzv, t.xoff, net->x_dense);
+                     net->in_dim, (int64_t)0, net->x_nzi, net->x_nzv, net->x_off, net->x_dense);
   KH_LAUNCHED();
   return KH_OK;
 }
@@ -1080,13 +1087,16 @@ static int net_forward_one(kh_slide_network* net, const float* x, hipStream_t st
     // kernel read them as they are (128 -> 8191 neurons, 4470
     // active: hash 4.2 and sums 7.1 us, against 4.6 + 5.8 + 21 with the list)
     const bool tile = in && hash_dense_rows(l->index->h) && neuron_tile_ok(l);
+    const uint32_t* nzi = in ? t.nzi : net->x_nzi;
+    const float* nzv = in ? t.nzv : net->x_nzv;
+    const int64_t* xoff = in ? t.xoff : net->x_off;
     if (in && !tile) {
       hipLaunchKernelGGL(tr_stage_nz_kernel, dim3(1), dim3(1024), 0, st, in, l->dim, (int64_t)0, (int64_t)0,
                          t.nzi, t.nzv, t.xoff);
       KH_LAUNCHED();
     }
     int rc = tile ? hash_dense_launch(l->index->h, in, l->dim, 1, t.codes, st)
-                  : hash_sparse_launch(l->index->h, t.xoff, t.nzi, t.nzv, 1, t.codes, st);
+                  : hash_sparse_launch(l->index->h, xoff, nzi, nzv, 1, t.codes, st);
     if (rc != KH_OK) return rc;
     const int qs = query_stride(l->index);
     rc = query_launch(l->index, t.codes, 1, t.qids, t.qcnt, qs, t.qlen, st);
@@ -1101,8 +1111,8 @@ static int net_forward_one(kh_slide_network* net, const float* x, hipStream_t st
       if (rc != KH_OK) return rc;
     } else {
       const unsigned nb = static_cast<unsigned>(std::min(ceil_div(t.as, kTrThreads / 64), 4096));
-      hipLaunchKernelGGL(tr_neuron_wave_kernel, dim3(nb), dim3(kTrThreads), 0, st, l->w, l->bias, l->dim, t.nzi, t.nzv,
-                         t.xoff, t.aids, t.alen, t.as, l->act, t.pre, t.post, t.dense);
+      hipLaunchKernelGGL(tr_neuron_wave_kernel, dim3(nb), dim3(kTrThreads), 0, st, l->w, l->bias, l->dim, nzi, nzv,
+                         xoff, t.aids, t.alen, t.as, l->act, t.pre, t.post, t.dense);
       KH_LAUNCHED();
     }
     if (l->act == KH_ACT_SOFTMAX) {

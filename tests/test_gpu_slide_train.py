@@ -220,3 +220,24 @@ def test_sparse_examples_match_dense_training(kh, orc):
     p = net.predict_sparse(vecs[:4]).cpu().numpy()
     for i in range(4):
         np.testing.assert_array_equal(p[i], onet.predict(X[i]))
+
+
+@pytest.mark.parametrize("optimizer", ["Sgd", "Adam"])
+@pytest.mark.parametrize("dim", [130, 200])
+def test_dense_steps_between_sparse_steps(kh, orc, optimizer, dim):
+    """Sparse examples are densified into a buffer that the network keeps: a dense step in
+    between (layer 0 too wide for the tile kernel, so its nonzeros are listed) leaves nothing
+    of the example before it for the next sparse one."""
+    from klearu_amd.lsh import SparseVector
+    rng = np.random.default_rng(dim)
+    specs = [spec(rng, dim, 40, "Relu", sampling="Vanilla", k=4, L=6, cap=32, seed=41),
+             spec(rng, 40, 20, "Softmax", sampling="Vanilla", k=4, L=6, cap=32, seed=42)]
+    net, layers, onet = build(orc, specs, optimizer)
+    X, labels = data(rng, 12, dim, 20)
+    for s in range(4):
+        lo = 3 * s
+        xb, lb = X[lo:lo + 3], labels[lo:lo + 3]
+        got = (net.train_step(xb, lb, 0.05) if s % 2
+               else net.train_step_sparse([SparseVector.from_dense(x) for x in xb], lb, 0.05))
+        assert got == pytest.approx(onet.train_step(xb, lb, 0.05), rel=1e-5, abs=1e-6)
+        check_same(layers, onet, f"after step {s}")
