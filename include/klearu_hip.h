@@ -378,7 +378,8 @@ int kh_slide_network_train_step_sparse(kh_slide_network* n, const int64_t* xoff_
                                        void* stream);
 /* Network::predict (net.rs:151-154) for each row of x_dev[batch][input_dim]:
  * out_dev[batch][num_neurons of the last layer], the last layer's dense
- * activations. */
+ * activations.  Does not mutate; keeps up to 256 MB of scratch (at least one
+ * row's) for each stream it is called on. */
 int kh_slide_network_predict(kh_slide_network* n, const float* x_dev, int64_t batch,
                              float* out_dev, void* stream);
 /* Same for CSR rows (as kh_slide_network_train_step_sparse reads them). */

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "chain_add.hpp"
@@ -968,7 +969,8 @@ struct kh_slide_network {
   float* x_dense = nullptr;
   uint32_t* labels = nullptr;
   size_t labels_cap = 0;
-  kh::Scratch rows_ws;       // net_predict_rows' buffers
+  kh::StreamWs rows_ws;      // net_predict_rows' buffers, a slot of each stream
+  std::mutex rows_mu;        // one prediction is enqueued at a time: host threads may share a stream
   int in_dim = 0, out_dim = 0;
   template <typename T>
   T* alloc(size_t n, bool zero = false) {
@@ -1247,16 +1249,22 @@ extern "C" int kh_slide_network_train_step_sparse(kh_slide_network* net, const i
                         labels_host, lr, loss_out, stream);
 }
 
+// While it lives, this thread may allocate beside a capture (allocations are not captured).
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Network::forward for a batch, a row per example: the kernels of
 // net_forward_one over `rows` examples at a time, so a batch costs one chain of
-// launches instead of one per example (784 -> 1024 -> 32, batch 128: 0.118 ms,
+// launches instead of one per example (784 -> 1024 -> 32, batch 128: 71 us,
 // against 17.1 ms for 128 chains, each bound by its launches' latency).  Ternary families whose
 // signs fit the per-row LDS kernel hash the dense rows; the others hash the
 // staged lists, as net_forward_one does (the codes are the same).  The rows
-// taken at a time keep the scratch within kRowsWs bytes (at least one row).
-// KH_ERR_UNSUPPORTED, before anything is launched, when the scratch would have
-// to grow under stream capture or cannot be allocated: the caller then runs
-// the examples one by one in the network's own buffers.
+// taken at a time keep the scratch within kRowsWs bytes (at least one row).  The
+// scratch is the stream's own, as a prediction writes nothing else and may run
+// beside others; it grows under stream capture too.
 constexpr size_t kRowsWs = (size_t)256 << 20;
 static int net_predict_rows(kh_slide_network* net, const float* x_dev, const int64_t* xoff,
                             const uint32_t* xidx, const float* xval, int64_t batch, float* out_dev,
@@ -1278,22 +1286,21 @@ static int net_predict_rows(kh_slide_network* net, const float* x_dev, const int
     if (i + 1 < nl) mdense = std::max(mdense, (size_t)l->n);
   }
   const size_t per_row = sizeof(int64_t) * 2 + 4 * (mL + 2 * mqs + 3 * mas + 2 * mnz + 2 * mdense + 2);
-  const int64_t rows = std::min<int64_t>({batch, std::max<int64_t>(1, (int64_t)(kRowsWs / per_row)), 65535});
-  const size_t R = (size_t)rows;
-  const size_t sizes[] = {pad(R * 16), pad(4 * R * mL), pad(4 * R * mqs), pad(4 * R * mqs), pad(4 * R),
-                          pad(4 * R * mas), pad(4 * R), pad(4 * R * mas), pad(4 * R * mas), pad(4 * R * mnz),
-                          pad(4 * R * mnz), pad(4 * R * mdense), pad(4 * R * mdense)};
-  constexpr int kBufs = sizeof(sizes) / sizeof(sizes[0]);
-  size_t total = 0;
-  for (size_t s : sizes) total += s;
-  if (total > net->rows_ws.cap) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return KH_ERR_UNSUPPORTED;
-  }
-  char* base = static_cast<char*>(net->rows_ws.get(total));
-  if (!base) {
+  constexpr int kBufs = 13;
+  size_t sizes[kBufs];
+  int64_t rows = std::min<int64_t>({batch, std::max<int64_t>(1, (int64_t)(kRowsWs / per_row)), 65535});
+  char* base = nullptr;
+  for (;; rows /= 2) {   // fewer rows at a time where memory is short
+    const size_t R = (size_t)rows;
+    const size_t need[kBufs] = {R * 16, 4 * R * mL, 4 * R * mqs, 4 * R * mqs, 4 * R, 4 * R * mas, 4 * R, 4 * R * mas,
+                                4 * R * mas, 4 * R * mnz, 4 * R * mnz, 4 * R * mdense, 4 * R * mdense};
+    size_t total = 0;
+    for (int i = 0; i < kBufs; ++i) total += sizes[i] = pad(need[i]);
+    RelaxedCapture relaxed;
+    base = static_cast<char*>(net->rows_ws.get(st)->get(0, total));
+    if (base) break;
+    if (rows == 1) return KH_ERR_ALLOC;
     (void)hipGetLastError();
-    return KH_ERR_UNSUPPORTED;
   }
   char* buf[kBufs];
   for (int i = 0; i < kBufs; ++i) {
@@ -1377,19 +1384,8 @@ static int net_predict(kh_slide_network* net, const float* x_dev, const int64_t*
     rc = net_check_csr(xoff, batch, st);
     if (rc != KH_OK) return rc;
   }
-  rc = net_predict_rows(net, x_dev, xoff, xidx, xval, batch, out_dev, st);
-  if (rc != KH_ERR_UNSUPPORTED) return rc;
-  for (int64_t e = 0; e < batch; ++e) {
-    if (xoff) {
-      rc = net_stage_sparse(net, xoff, xidx, xval, e, st);
-      if (rc != KH_OK) return rc;
-    }
-    rc = net_forward_one(net, xoff ? nullptr : x_dev + e * static_cast<int64_t>(net->in_dim), st);
-    if (rc != KH_OK) return rc;
-    KH_HIP(hipMemcpyAsync(out_dev + e * static_cast<int64_t>(net->out_dim), net->b.back().dense,
-                          sizeof(float) * net->out_dim, hipMemcpyDeviceToDevice, st));
-  }
-  return KH_OK;
+  std::lock_guard<std::mutex> g(net->rows_mu);
+  return net_predict_rows(net, x_dev, xoff, xidx, xval, batch, out_dev, st);
 }
 
 extern "C" int kh_slide_network_predict(kh_slide_network* net, const float* x_dev, int64_t batch,

@@ -73,8 +73,8 @@ def test_predict_rank_families_hash_the_lists(kh, family):
 
 
 def test_predict_captured_before_its_rows_fit(kh, orc):
-    """Under capture the scratch cannot grow: a larger batch than any before is captured all the
-    same (example by example), and its replays are the eager results."""
+    """A larger batch than any before is captured all the same, and its replays are the eager
+    results."""
     rng = np.random.default_rng(12)
     specs = [spec(rng, 40, 50, "Relu", top_k=20, k=4, L=5, cap=16, seed=7),
              spec(rng, 50, 30, "Softmax", top_k=10, k=4, L=5, cap=16, seed=8)]
@@ -93,3 +93,45 @@ def test_predict_captured_before_its_rows_fit(kh, orc):
         for i, x in enumerate(X.cpu().numpy()):
             np.testing.assert_array_equal(got[i], onet.predict(x))
         np.testing.assert_array_equal(net.predict_batch(X).cpu().numpy(), got)
+
+
+@pytest.mark.parametrize("streams,threads", [(2, 1), (3, 3), (1, 3)])
+def test_predictions_of_one_network_side_by_side(kh, orc, streams, threads):
+    """Predictions do not mutate: several streams, and host threads sharing one, each get the
+    outputs of their own inputs."""
+    import threading
+    from klearu_amd.lsh import SparseVector
+    rng = np.random.default_rng(31)
+    specs = [spec(rng, 300, 400, "Relu", top_k=100, k=5, L=8, cap=24, seed=9),
+             spec(rng, 400, 200, "Softmax", top_k=60, k=5, L=8, cap=24, seed=10)]
+    net, layers, onet = build(orc, specs)
+    n = max(streams, threads)
+    Xs = [inputs(rng, 40 + 30 * j, 300) for j in range(n)]
+    want = [net.predict_batch(X).cpu().numpy() for X in Xs]
+    for j in range(n):
+        np.testing.assert_array_equal(want[j][0], onet.predict(Xs[j][0]))
+    dev = [torch.from_numpy(X).cuda() for X in Xs]
+    sv = [[SparseVector.from_dense(x) for x in X[:20]] for X in Xs]
+    st = [torch.cuda.Stream() for _ in range(streams)]
+    outs = [[] for _ in range(n)]
+    torch.cuda.synchronize()
+
+    def work(j, reps):
+        for _ in range(reps):
+            outs[j].append(net.predict_batch(dev[j], stream=st[j % streams]))
+    if threads == 1:
+        for _ in range(12):
+            for j in range(n):
+                work(j, 1)
+                outs[j].append(net.predict_sparse(sv[j], stream=st[j % streams]))
+    else:
+        ts = [threading.Thread(target=work, args=(j, 12)) for j in range(n)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    torch.cuda.synchronize()
+    for j in range(n):
+        assert len(outs[j]) >= 12
+        for o in outs[j]:
+            np.testing.assert_array_equal(o.cpu().numpy(), want[j][:o.shape[0]])
