@@ -1131,16 +1131,20 @@ __device__ __forceinline__ uint32_t query_buckets(const uint32_t* __restrict__ q
   return bstart[L];
 }
 
-// put(id) for every entry of the query's buckets: 16 lanes to a bucket, which finds its
+// put(id) for every entry of the query's buckets: some lanes to a bucket, which finds its
 // entries without a search (a binary search over bstart is a chain of LDS reads per
-// entry).  TU buckets x EU entries per lane are in flight.  One row of 6400 entries in
-// query_direct_kernel: 4.8 us, 9.0 with the search; 256 rows in query_bitmap_kernel 16.4
-// against 19.3.
+// entry).  Sixteen of them, and for few tables all the block has: with sixteen, one bucket
+// of 8192 ids leaves all but a few lanes idle (a query of one row over 100000 ids, with
+// counts: 193 us; 21.6 with 1024 lanes, 22.2 with the search).  TU buckets x EU entries
+// per lane are in flight.  One row of 6400 entries in 50 buckets, query_direct_kernel: 4.8
+// us, 9.0 with the search; 256 rows in query_bitmap_kernel 16.4 against 19.3.
 constexpr int kBucketLanes = 16;
-template <int TU, int EU, typename Put>
+template <int TU, int EU, bool WIDE, typename Put>
 __device__ __forceinline__ void bucket_entries(const uint32_t* __restrict__ data, const uint32_t* bstart,
                                                const uint32_t* bslot, int L, int cap, Put put) {
-  const int grp = threadIdx.x / kBucketLanes, li = threadIdx.x % kBucketLanes, ng = blockDim.x / kBucketLanes;
+  // WIDE: the block's lanes over L, rounded up to a power of two
+  const int lanes = WIDE ? (int)blockDim.x >> (L > 1 ? 32 - __clz(L - 1) : 0) : kBucketLanes;
+  const int grp = threadIdx.x / lanes, li = threadIdx.x % lanes, ng = blockDim.x / lanes;
   for (int t0 = grp; t0 < L; t0 += ng * TU) {
     uint32_t n[TU], most = 0;
     const uint32_t* p[TU];
@@ -1151,31 +1155,34 @@ __device__ __forceinline__ void bucket_entries(const uint32_t* __restrict__ data
       p[u] = data + (size_t)bslot[t] * cap;
       most = max(most, n[u]);
     }
-    for (uint32_t i0 = li; i0 < most; i0 += kBucketLanes * EU) {
+    for (uint32_t i0 = li; i0 < most; i0 += lanes * EU) {
       uint32_t id[TU][EU];
 #pragma unroll
       for (int u = 0; u < TU; ++u)
 #pragma unroll
         for (int e = 0; e < EU; ++e)  // clamped (cap >= 1), unconditional
-          id[u][e] = p[u][min(i0 + e * kBucketLanes, max(n[u], 1u) - 1u)];
+          id[u][e] = p[u][min(i0 + e * lanes, max(n[u], 1u) - 1u)];
 #pragma unroll
       for (int u = 0; u < TU; ++u)
 #pragma unroll
         for (int e = 0; e < EU; ++e)
-          if (i0 + e * kBucketLanes < n[u]) put(id[u][e]);
+          if (i0 + e * lanes < n[u]) put(id[u][e]);
     }
   }
 }
 
-// m: entries in all.  Full buckets want one bucket's entries in flight, short ones several
-// buckets.
+// m: entries in all.  Where the block has lanes for two buckets' worth each, all of it
+// works on the L buckets at once; otherwise full buckets want one bucket's entries in
+// flight, short ones several buckets.
 template <typename Put>
 __device__ __forceinline__ void for_bucket_entries(const uint32_t* __restrict__ data, const uint32_t* bstart,
                                                    const uint32_t* bslot, int L, int cap, uint32_t m, Put put) {
-  if (m > (uint32_t)L * 2 * kBucketLanes)
-    bucket_entries<1, 8>(data, bstart, bslot, L, cap, put);
+  if (L * 2 * kBucketLanes <= (int)blockDim.x)
+    bucket_entries<1, 8, true>(data, bstart, bslot, L, cap, put);
+  else if (m > (uint32_t)L * 2 * kBucketLanes)
+    bucket_entries<1, 8, false>(data, bstart, bslot, L, cap, put);
   else
-    bucket_entries<4, 2>(data, bstart, bslot, L, cap, put);
+    bucket_entries<4, 2, false>(data, bstart, bslot, L, cap, put);
 }
 
 // One block per query row: unique bucket ids in ascending order with counts.
