@@ -90,3 +90,19 @@ def test_bf16_dot_rows(kh, orc, rows, n):
     xb = orc.bf16_from_f32(x)
     got = F(float(bf16_full_dot(at_offset(w[0].view(np.int16), 0), at_offset(xb.view(np.int16), 1))))
     assert got.tobytes() == orc.bf16_full_dot(w[0], xb).tobytes()
+
+
+@pytest.mark.parametrize("rows,n,ldw", [(1, 16, 16), (1, 17, 17), (65, 0, 4), (64, 1, 3), (2, 16, 20), (2549, 17, 17),
+                                        (2550, 17, 21), (3900, 26, 26), (3899, 26, 28)])
+def test_bf16_dot_short_rows(kh, orc, rows, n, ldw):
+    """Short rows take a thread each: one row to many, on both sides of the rule."""
+    from klearu_amd import _lib
+    from klearu_amd._dev import ptr, stream_ptr
+    rng = np.random.default_rng(rows + n)
+    w = orc.bf16_from_f32(rng.standard_normal(rows * ldw).astype(F)).reshape(rows, ldw)
+    x = rng.standard_normal(max(n, 1)).astype(F)[:n]
+    wd, xd = at_offset(w.view(np.int16), 1), at_offset(np.append(x, F(0)), 1)
+    out = torch.full((rows,), 7.0, dtype=torch.float32, device="cuda")
+    _lib.call("kh_bf16_dot_f32", ptr(wd), rows, ldw, ptr(xd), n, ptr(out), stream_ptr())
+    want = [orc.bf16_dot_f32(np.ascontiguousarray(r[:n]), x) if n else F(-0.0) for r in w]
+    np.testing.assert_array_equal(bits(out.cpu().numpy()), bits(want))
