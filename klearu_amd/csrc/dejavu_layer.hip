@@ -216,36 +216,45 @@ __global__ __launch_bounds__(kDcThreads) void dl_chain_down_kernel(
   if (b < batch && j < hidden) y[b * hidden + j] = __fadd_rn(s, bd[j]);
 }
 
-// Many outputs (kDlWide of them or more): one thread per output row and TB
-// tokens.  A group of kDlAhead coalesced loads of the transposed weights is in
-// flight while the group before is added; the tokens' inputs are the same for
-// every lane (scalar loads).  No LDS traffic is spent on products, and the TB
-// chains of a thread hide each other's adds.
+// Many outputs (wide_rows_form and the like): one thread per output row and TB tokens.  A group of
+// kDlAhead coalesced loads of the transposed weights is in flight while the group
+// before is added; the tokens' inputs are the same for every lane (scalar loads).
+// No LDS traffic is spent on products, and the TB chains of a thread hide each
+// other's adds.  GATEUP: a thread has a neuron's gate and up rows.
 constexpr int kDlAhead = 16;
-template <int TB>
+template <bool GATEUP, int TB>
 __global__ __launch_bounds__(64) void dl_wide_rows_kernel(const DcRows a, int out_f) {
+  constexpr int M = GATEUP ? 2 : 1;
   const int64_t at = min((int64_t)blockIdx.x * 64 + threadIdx.x, a.nrows - 1);
   const int64_t r = dc_row(a, at);
   const int64_t b0 = (int64_t)blockIdx.y * TB;
-  const DcMat& mat = a.m[blockIdx.z];
-  const float* __restrict__ wt = mat.w + r;
+  const DcMat* mat = &a.m[GATEUP ? 0 : blockIdx.z];
+  const float* __restrict__ wt[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) wt[m] = mat[m].w + r;
   const float* __restrict__ xr[TB];
 #pragma unroll
   for (int t = 0; t < TB; ++t) xr[t] = a.x + min(b0 + t, a.batch - 1) * a.ldx;
-  float s[TB];
+  float s[M][TB];
 #pragma unroll
-  for (int t = 0; t < TB; ++t) s[t] = -0.0f;
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int t = 0; t < TB; ++t) s[m][t] = -0.0f;
   const int n = a.in_f, full = n / kDlAhead * kDlAhead;
-  float w0[kDlAhead], w1[kDlAhead];
-  auto load = [&](float (&w)[kDlAhead], int j) {
+  float w0[M][kDlAhead], w1[M][kDlAhead];
+  auto load = [&](float (&w)[M][kDlAhead], int j) {
 #pragma unroll
-    for (int u = 0; u < kDlAhead; ++u) w[u] = wt[(int64_t)min(j + u, n - 1) * out_f];
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int u = 0; u < kDlAhead; ++u) w[m][u] = wt[m][(int64_t)min(j + u, n - 1) * out_f];
   };
-  auto add = [&](const float (&w)[kDlAhead], int j) {
+  auto add = [&](const float (&w)[M][kDlAhead], int j) {
 #pragma unroll
     for (int u = 0; u < kDlAhead; ++u)
 #pragma unroll
-      for (int t = 0; t < TB; ++t) s[t] = __fadd_rn(s[t], __fmul_rn(w[u], xr[t][j + u]));
+      for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int m = 0; m < M; ++m) s[m][t] = __fadd_rn(s[m][t], __fmul_rn(w[m][u], xr[t][j + u]));
   };
   load(w0, 0);
   int j = 0;
@@ -261,16 +270,97 @@ __global__ __launch_bounds__(64) void dl_wide_rows_kernel(const DcRows a, int ou
     add(w0, j);
     j += kDlAhead;
   }
-  for (; j < n; ++j) {
-    const float w = wt[(int64_t)j * out_f];
+  for (; j < n; ++j)
 #pragma unroll
-    for (int t = 0; t < TB; ++t) s[t] = __fadd_rn(s[t], __fmul_rn(w, xr[t][j]));
-  }
+    for (int m = 0; m < M; ++m) {
+      const float w = wt[m][(int64_t)j * out_f];
+#pragma unroll
+      for (int t = 0; t < TB; ++t) s[m][t] = __fadd_rn(s[m][t], __fmul_rn(w, xr[t][j]));
+    }
   if ((int64_t)blockIdx.x * 64 + threadIdx.x >= a.nrows) return;
-  const float bi = mat.bias[r];
+  float bi[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) bi[m] = mat[m].bias[r];
 #pragma unroll
   for (int t = 0; t < TB; ++t)
-    if (b0 + t < a.batch) mat.y[(b0 + t) * a.ldy + (a.scatter ? r : at)] = __fadd_rn(s[t], bi);
+    if (b0 + t < a.batch) {
+      const float z = __fadd_rn(s[0][t], bi[0]);
+      mat->y[(b0 + t) * a.ldy + (a.scatter ? r : at)] =
+          GATEUP ? __fmul_rn(silu_ref(z), __fadd_rn(s[M - 1][t], bi[M - 1])) : z;
+    }
+}
+
+// The down projection's: one thread per output column and TB tokens, the selected
+// neurons' columns read as rows of the transposed weights.
+template <int TB>
+__global__ __launch_bounds__(64) void dl_wide_down_kernel(
+    const float* __restrict__ wdt, const float* __restrict__ bd, int hidden,
+    const float* __restrict__ h, int64_t batch, const int64_t* __restrict__ sel, int n,
+    float* __restrict__ y) {
+  const int j = min((int)blockIdx.x * 64 + (int)threadIdx.x, hidden - 1);
+  const int64_t b0 = (int64_t)blockIdx.y * TB;
+  const float* __restrict__ hr[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) hr[t] = h + min(b0 + t, batch - 1) * n;
+  float s[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) s[t] = 0.0f;
+  const int full = n / kDlAhead * kDlAhead;
+  int id[kDlAhead];                              // neurons of the group to load next
+  float w0[kDlAhead], w1[kDlAhead];
+  auto ids = [&](int a0) {
+#pragma unroll
+    for (int u = 0; u < kDlAhead; ++u) id[u] = (int)sel[min(a0 + u, n - 1)];
+  };
+  auto load = [&](float (&w)[kDlAhead]) {
+#pragma unroll
+    for (int u = 0; u < kDlAhead; ++u) w[u] = wdt[(size_t)id[u] * hidden + j];
+  };
+  // a zero activation adds nothing, whatever the weight
+  auto add = [&](const float (&w)[kDlAhead], int a0) {
+#pragma unroll
+    for (int u = 0; u < kDlAhead; ++u)
+#pragma unroll
+      for (int t = 0; t < TB; ++t) {
+        const float v = hr[t][a0 + u];
+        s[t] = __fadd_rn(s[t], v != 0.0f ? __fmul_rn(w[u], v) : -0.0f);
+      }
+  };
+  auto add_some = [&](const float (&w)[kDlAhead], int a0) {
+#pragma unroll
+    for (int u = 0; u < kDlAhead; ++u)
+#pragma unroll
+      for (int t = 0; t < TB; ++t) {
+        const float v = hr[t][min(a0 + u, n - 1)];
+        s[t] = __fadd_rn(s[t], a0 + u < n && v != 0.0f ? __fmul_rn(w[u], v) : -0.0f);
+      }
+  };
+  if (n > 0) {
+    ids(0);
+    load(w0);
+    ids(kDlAhead);
+    int a0 = 0;
+    for (; a0 + 2 * kDlAhead <= full; a0 += 2 * kDlAhead) {
+      load(w1);
+      ids(a0 + 2 * kDlAhead);
+      __builtin_amdgcn_sched_barrier(0);
+      add(w0, a0);
+      load(w0);
+      ids(a0 + 3 * kDlAhead);
+      __builtin_amdgcn_sched_barrier(0);
+      add(w1, a0 + kDlAhead);
+    }
+    if (a0 < n) {
+      if (a0 + kDlAhead < n) load(w1);
+      add_some(w0, a0);
+      if (a0 + kDlAhead < n) add_some(w1, a0 + kDlAhead);
+    }
+  }
+  if ((int)blockIdx.x * 64 + (int)threadIdx.x >= hidden) return;
+  const float bi = bd[j];
+#pragma unroll
+  for (int t = 0; t < TB; ++t)
+    if (b0 + t < batch) y[(b0 + t) * hidden + j] = __fadd_rn(s[t], bi);
 }
 
 // One wave per (head, token): the score's products in LDS, added by one lane in
@@ -348,10 +438,31 @@ static int upload_indices(WsSet* w, const int64_t* idx_host, int64_t n, int64_t 
   return KH_OK;
 }
 
-// Outputs from which the thread-per-output form is taken.  A square Linear of
-// 1024 (chain kernel, wide form; us per call): 64 tokens 28.2, 30.1; 128 tokens
-// 54.9, 30.3; of 2048: 32 tokens 45, 57; 64 tokens 89, 57.
-constexpr int64_t kDlWide = 3 << 15;
+// Which form a call takes.  A chain block costs 3.5 to 4 us and 6 ns a term, whatever part of
+// it is used, and kDcRound outputs' blocks run at once; the wide forms cost a term more but
+// take many times as many outputs in that time.  `outputs`: in whole chain blocks.
+constexpr int64_t kDcRound = 1 << 15;
+// Rows of a Linear, us on the device, chains / wide.  32 inputs: 16384 outputs 5.9 / 3.3, 262144
+// 69 / 4.1; 96: 1024 outputs 4.2 / 4.2, 16384 5.9 / 4.8; 128: 4096 of one token 4.4 / 4.9; 256: 16384
+// 5.9 / 8.9, 65536 18.9 / 9.4; 512: 65536 20.5 / 16.6; 1024: 65536 28.0 / 30.4, 131072 55 / 30, 262144
+// 107 / 36; 2048: 65536 43 / 58, 262144 168 / 68.
+static bool wide_rows_form(int64_t outputs, int64_t terms) {
+  return terms <= 96 || outputs > (terms <= 512 ? 1 : 3) * kDcRound;
+}
+// Gate and up rows of n of `of` neurons (two outputs a neuron).  Few of many leave a lane alone on its
+// line of the transposed rows, which counts the more the longer they are.  64 inputs: wide is the
+// faster at any size; 128 inputs, 30 of 2752: 64 tokens 2 us slower, 1024 5 faster; 256 inputs, 200 of
+// 2752: 256 tokens 3 us faster, 4096 322 faster, 30 of 2752: 4096 7 slower; 512 inputs, 800 of 2752: 64
+// tokens 2 us faster, 256 58 faster, 200 of 2752: 1024 60 slower; 1024 inputs, 800 of 2752: 64 tokens
+// 15 us slower, 256 38 faster.
+static bool wide_gateup_form(int64_t outputs, int64_t terms, int64_t n, int64_t of) {
+  return terms <= 96 ||
+         (outputs > kDcRound && 160 * outputs > terms * kDcRound && (terms <= 128 || n * 4096 >= of * terms));
+}
+// The down projection over n neurons, whose columns it gathers: 90 ns a term.  8 neurons: 16384 outputs
+// the same, 32768 4 us faster; 30: 16384 4 us slower, 65536 6 faster; 200: 65536 5 us slower, 131072 8
+// faster; 800: 131072 25 us slower, 262144 16 faster.
+static bool wide_down_form(int64_t outputs, int64_t n) { return 160 * outputs > (128 + n) * kDcRound; }
 // Waves of one token each below which a thread takes two tokens rather than four
 // (1024: 256 tokens 35.4 with two, 38.2 with four; 1024 tokens 96.9, 69.5).
 constexpr int64_t kDlWideSplit = 6144;
@@ -386,6 +497,7 @@ static int chain_rows(DcRows a, int mats, hipStream_t st) {
   return KH_OK;
 }
 
+template <bool GATEUP>
 static int wide_rows(DcRows a, int out_f, int mats, hipStream_t st) {
   constexpr int64_t kMaxTokens = 65535 * 4;
   const float* x = a.x;
@@ -397,12 +509,12 @@ static int wide_rows(DcRows a, int out_f, int mats, hipStream_t st) {
     for (int i = 0; i < 3; ++i) a.m[i].y = y[i] ? y[i] + b0 * a.ldy : nullptr;
     const unsigned gx = (unsigned)ceil_div(a.nrows, 64);
     if (a.batch == 1)
-      hipLaunchKernelGGL(dl_wide_rows_kernel<1>, dim3(gx, 1, (unsigned)mats), dim3(64), 0, st, a, out_f);
+      hipLaunchKernelGGL((dl_wide_rows_kernel<GATEUP, 1>), dim3(gx, 1, (unsigned)mats), dim3(64), 0, st, a, out_f);
     else if (a.batch < 4 || (int64_t)gx * a.batch * mats < kDlWideSplit)
-      hipLaunchKernelGGL(dl_wide_rows_kernel<2>, dim3(gx, (unsigned)ceil_div(a.batch, 2), (unsigned)mats), dim3(64), 0,
+      hipLaunchKernelGGL((dl_wide_rows_kernel<GATEUP, 2>), dim3(gx, (unsigned)ceil_div(a.batch, 2), (unsigned)mats), dim3(64), 0,
                          st, a, out_f);
     else
-      hipLaunchKernelGGL(dl_wide_rows_kernel<4>, dim3(gx, (unsigned)ceil_div(a.batch, 4), (unsigned)mats), dim3(64), 0,
+      hipLaunchKernelGGL((dl_wide_rows_kernel<GATEUP, 4>), dim3(gx, (unsigned)ceil_div(a.batch, 4), (unsigned)mats), dim3(64), 0,
                          st, a, out_f);
     KH_LAUNCHED();
   }
@@ -414,7 +526,7 @@ static int rows_launch(const kh_dejavu_linear* const* l, int mats, const float* 
                        int64_t batch, const int64_t* rows, int64_t nrows, float* const* y,
                        int64_t ldy, int scatter, int head_dim, hipStream_t st) {
   if (batch * nrows == 0) return KH_OK;
-  const bool wide = batch * nrows >= kDlWide;
+  const bool wide = wide_rows_form(mats * batch * ceil_div(nrows, kDcRows) * kDcRows, l[0]->in_f);
   DcRows a{};
   for (int i = 0; i < mats; ++i) a.m[i] = {wide ? l[i]->wt : l[i]->w, l[i]->bias, y[i]};
   a.in_f = l[0]->in_f;
@@ -426,16 +538,18 @@ static int rows_launch(const kh_dejavu_linear* const* l, int mats, const float* 
   a.ldy = ldy;
   a.scatter = scatter;
   a.head_dim = head_dim;
-  if (wide) return wide_rows(a, l[0]->out_f, mats, st);
+  if (wide) return wide_rows<false>(a, l[0]->out_f, mats, st);
   return chain_rows<false>(a, mats, st);
 }
 
 template <int TB>
-static void chain_down_go(const kh_dejavu_linear* d, const float* h, int64_t batch, const int64_t* sel,
-                          int n, float* y, hipStream_t st) {
+static void down_go(const kh_dejavu_linear* d, bool wide, const float* h, int64_t batch, const int64_t* sel,
+                    int n, float* y, hipStream_t st) {
   const int H = d->out_f;
-  const dim3 g((unsigned)ceil_div(H, kDcRows), (unsigned)ceil_div(batch, TB));
-  if (H % 4 == 0)
+  const dim3 g((unsigned)ceil_div(H, wide ? 64 : kDcRows), (unsigned)ceil_div(batch, TB));
+  if (wide)
+    hipLaunchKernelGGL(dl_wide_down_kernel<TB>, g, dim3(64), 0, st, d->wt, d->bias, H, h, batch, sel, n, y);
+  else if (H % 4 == 0)
     hipLaunchKernelGGL((dl_chain_down_kernel<TB, true>), g, dim3(kDcThreads), 0, st, d->wt, d->bias, H, h, batch,
                        sel, n, y);
   else
@@ -548,8 +662,9 @@ extern "C" int kh_dejavu_sparse_mlp_forward(const kh_dejavu_sparse_mlp* m, const
   if (!h) return KH_ERR_ALLOC;
   if (batch * n_sel > 0) {
     DcRows g{};
-    g.m[0] = {gate->w, gate->bias, h};
-    g.m[1] = {up->w, up->bias, nullptr};
+    const bool wide = wide_gateup_form(batch * ceil_div(n_sel, kDcRows / 2) * kDcRows, H, n_sel, I);
+    g.m[0] = {wide ? gate->wt : gate->w, gate->bias, h};
+    g.m[1] = {wide ? up->wt : up->w, up->bias, nullptr};
     g.in_f = H;
     g.x = x_dev;
     g.ldx = H;
@@ -557,16 +672,17 @@ extern "C" int kh_dejavu_sparse_mlp_forward(const kh_dejavu_sparse_mlp* m, const
     g.rows = sel;
     g.nrows = n_sel;
     g.ldy = n_sel;
-    rc = chain_rows<true>(g, 1, st);
+    rc = wide ? wide_rows<true>(g, I, 1, st) : chain_rows<true>(g, 1, st);
     if (rc != KH_OK) return rc;
   }
   for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
     const int64_t nb = std::min<int64_t>(batch - b0, 65535);
     const float* hb = h + b0 * n_sel;
     float* yb = y_dev + b0 * H;
-    if (nb == 1) chain_down_go<1>(down, hb, nb, sel, (int)n_sel, yb, st);
-    else if (nb == 2) chain_down_go<2>(down, hb, nb, sel, (int)n_sel, yb, st);
-    else chain_down_go<4>(down, hb, nb, sel, (int)n_sel, yb, st);
+    const bool wide = wide_down_form(nb * ceil_div(H, kDcRows) * kDcRows, n_sel);
+    if (nb == 1) down_go<1>(down, wide, hb, nb, sel, (int)n_sel, yb, st);
+    else if (nb == 2) down_go<2>(down, wide, hb, nb, sel, (int)n_sel, yb, st);
+    else down_go<4>(down, wide, hb, nb, sel, (int)n_sel, yb, st);
     KH_LAUNCHED();
   }
   return KH_OK;
