@@ -317,37 +317,77 @@ __device__ __forceinline__ void hm_load8(const float* __restrict__ xr, int d0, i
   }
 }
 
-// The reference's sequential sum for one (row, plane): its sign bit.  `spw` are the
-// plane's 2-bit signs (kh_hash_family::sp_dev); a dimension without a coefficient
-// adds a zero of either sign, which leaves every later sum and the sign test alone,
-// and its x is masked off, so inf and NaN add nothing there.  Both are read in
-// whole pieces, NB words (16 dimensions each) in flight.
+// A plane's terms for the replays below: its 2-bit signs (kh_hash_family::sp_dev) and its
+// entries (ent_t).
+struct HmPlanes {
+  const uint32_t* sp;
+  int spn;        // words of signs per plane
+  const int32_t* nnz;
+  const uint32_t* ent_t;
+  int P;
+  bool quads;     // dim and the row stride multiples of 4, rows 16-byte aligned
+};
+
+// s plus term i of a sign word (bit 2i: a term, 2i + 1: negative).  Without a term it adds a
+// zero of either sign, which leaves every later sum and the sign test alone; x is masked off
+// then, so inf and NaN add nothing.
+__device__ __forceinline__ float hm_term(float s, float x, uint32_t w, int i) {
+  const uint32_t c = w >> (2 * i);
+  const uint32_t on = 0u - (c & 1u);
+  return __fadd_rn(s, __uint_as_float((__float_as_uint(x) & on) ^ ((c & 2u) << 30)));
+}
+
+// The reference's sequential sum for one (row, plane): its sign bit.  Rows are read four
+// values a load where they allow it, NB sign words (16 dimensions each) in flight; others
+// value by value, and past 512 dimensions by the plane's entries, whose indices the lanes of
+// a wave share.  5000 rows of zeros and ones (many ties), 300 planes: of 784 dimensions 487 us (915
+// value by value), of 65 153 (217 by entries), of 785 782 (893 value by value).
 template <bool VEC, int NB>
-__device__ __forceinline__ bool hm_replay(const float* __restrict__ xr, const uint32_t* __restrict__ spw, int dim) {
+__device__ __forceinline__ bool hm_replay(const HmPlanes& p, int pl, const float* __restrict__ xr, int dim) {
+  const uint32_t* __restrict__ spw = p.sp + (int64_t)pl * p.spn;
   float s = 0.0f;
-  const int nw = (dim + 15) / 16;
-  for (int w0 = 0; w0 < nw; w0 += NB) {
-    uint32_t w[NB];
-    float4 x[NB][4];
+  if (VEC || p.quads) {
+    for (int w0 = 0; w0 < p.spn; w0 += NB) {
+      uint32_t w[NB];
+      float4 x[NB][4];
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      w[j] = w0 + j < nw ? spw[w0 + j] : 0u;
-      const int d = 16 * min(w0 + j, nw - 1);
-      hm_load8<VEC>(xr, d, dim, x[j][0], x[j][1]);
-      hm_load8<VEC>(xr, VEC ? min(d + 8, dim - 8) : d + 8, dim, x[j][2], x[j][3]);
-    }
+      for (int j = 0; j < NB; ++j) {
+        w[j] = w0 + j < p.spn ? spw[w0 + j] : 0u;
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float v[4] = {x[j][q].x, x[j][q].y, x[j][q].z, x[j][q].w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t c = w[j] >> (2 * (4 * q + i));   // bit 0: a term, bit 1: negative
-          const uint32_t on = 0u - (c & 1u);
-          s = __fadd_rn(s, __uint_as_float((__float_as_uint(v[i]) & on) ^ ((c & 2u) << 30)));
-        }
+        for (int q = 0; q < 4; ++q) x[j][q] = *reinterpret_cast<const float4*>(xr + min(16 * (w0 + j) + 4 * q, dim - 4));
       }
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          s = hm_term(s, x[j][q].x, w[j], 4 * q);
+          s = hm_term(s, x[j][q].y, w[j], 4 * q + 1);
+          s = hm_term(s, x[j][q].z, w[j], 4 * q + 2);
+          s = hm_term(s, x[j][q].w, w[j], 4 * q + 3);
+        }
+    }
+  } else if (p.spn <= 32) {
+    for (int w0 = 0; w0 < p.spn; ++w0) {
+      const uint32_t w = spw[w0];
+      float x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = xr[min(16 * w0 + i, dim - 1)];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s = hm_term(s, x[i], w, i);
+    }
+  } else {
+    constexpr int E = 8;
+    const int e1 = p.nnz[pl];
+    for (int e0 = 0; e0 < e1; e0 += E) {
+      uint32_t v[E];
+      float xd[E];
+#pragma unroll
+      for (int j = 0; j < E; ++j) v[j] = p.ent_t[(size_t)min(e0 + j, e1 - 1) * p.P + pl];
+#pragma unroll
+      for (int j = 0; j < E; ++j) xd[j] = xr[v[j] >> 1];
+#pragma unroll
+      for (int j = 0; j < E; ++j)
+        if (e0 + j < e1) s = (v[j] & 1u) ? __fsub_rn(s, xd[j]) : __fadd_rn(s, xd[j]);
     }
   }
   return s >= 0.0f;
@@ -388,8 +428,8 @@ __device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmc
 
 template <int KS, bool VEC>
 __global__ __launch_bounds__(64 * kHrWaves) void hash_dense_resident_kernel(
-    const uint4* __restrict__ bt, int ksteps, int ntiles, const uint32_t* __restrict__ sp, int spn, int k, int L,
-    int dim, const float* __restrict__ x, int64_t ldx, int64_t batch, uint32_t* __restrict__ codes, int64_t row_stride,
+    const uint4* __restrict__ bt, int ksteps, int ntiles, HmPlanes planes, int k, int L, int dim,
+    const float* __restrict__ x, int64_t ldx, int64_t batch, uint32_t* __restrict__ codes, int64_t row_stride,
     int64_t table_stride) {
   extern __shared__ uint4 hr_lds_buf[];
   __shared__ int nq[kHrWaves];
@@ -516,7 +556,7 @@ __global__ __launch_bounds__(64 * kHrWaves) void hash_dense_resident_kernel(
         const uint32_t e = queue[i];
         const int rr = (int)(e >> 10), pl = (int)(e & 1023u);
         const uint32_t bit = 1u << (pl & 31);
-        if (hm_replay<VEC, kHrBatch>(x + (r0 + rr) * ldx, sp + (int64_t)pl * spn, dim)) atomicOr(&pm[rr * words + (pl >> 5)], bit);
+        if (hm_replay<VEC, kHrBatch>(planes, pl, x + (r0 + rr) * ldx, dim)) atomicOr(&pm[rr * words + (pl >> 5)], bit);
         else atomicAnd(&pm[rr * words + (pl >> 5)], ~bit);
       }
       wave_lds_fence();
@@ -543,8 +583,8 @@ __global__ __launch_bounds__(64 * kHrWaves) void hash_dense_resident_kernel(
 // wait (200000 rows of 256 dimensions, 450 planes: 345 us against 290).
 template <bool VEC>
 __global__ __launch_bounds__(256, 3) void hash_dense_mfma_kernel(
-    const uint4* __restrict__ bt, int ksteps, int ntiles, const uint32_t* __restrict__ sp, int spn, int k, int L,
-    int dim, const float* __restrict__ x, int64_t ldx, int64_t batch, uint32_t* __restrict__ codes,
+    const uint4* __restrict__ bt, int ksteps, int ntiles, HmPlanes planes, int k, int L, int dim,
+    const float* __restrict__ x, int64_t ldx, int64_t batch, uint32_t* __restrict__ codes,
     int64_t row_stride, int64_t table_stride) {
   constexpr int kW = kHmMaxPlanes / 32 + 1;  // 32-plane words per row (one spare for the code window)
   __shared__ uint32_t pm[kHmRows][kW];
@@ -624,7 +664,7 @@ __global__ __launch_bounds__(256, 3) void hash_dense_mfma_kernel(
             queue[slot] = ((uint32_t)rr << 16) | (uint32_t)pl;
             bit = false;   // set by the replay below
           } else {
-            bit = hm_replay<VEC, kHmBatch>(x + (rb + rr) * ldx, sp + (int64_t)pl * spn, dim);
+            bit = hm_replay<VEC, kHmBatch>(planes, pl, x + (rb + rr) * ldx, dim);
           }
         }
         const uint64_t m = __ballot(bit && pl < P);
@@ -638,7 +678,7 @@ __global__ __launch_bounds__(256, 3) void hash_dense_mfma_kernel(
   for (int i = threadIdx.x; i < nrep; i += blockDim.x) {
     const uint32_t e = queue[i];
     const int rr = (int)(e >> 16), pl = (int)(e & 0xffffu);
-    if (hm_replay<VEC, kHmBatch>(x + (rb + rr) * ldx, sp + (int64_t)pl * spn, dim)) atomicOr(&pm[rr][pl >> 5], 1u << (pl & 31));
+    if (hm_replay<VEC, kHmBatch>(planes, pl, x + (rb + rr) * ldx, dim)) atomicOr(&pm[rr][pl >> 5], 1u << (pl & 31));
   }
   __syncthreads();
   // codes: table t takes planes t*k .. t*k+k-1 of its row
@@ -1448,7 +1488,8 @@ static bool hash_by_matrix(const kh_hash_family* h, int64_t batch) {
 static int hash_matrix_launch(const kh_hash_family* h, const float* x, int64_t ldx, int64_t batch, uint32_t* codes,
                               int64_t row_stride, int64_t table_stride, hipStream_t st) {
   const bool vec = h->dim % 32 == 0 && ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-  const int spn = (h->dim + 15) / 16;
+  const bool quads = h->dim % 4 == 0 && ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const HmPlanes planes{h->sp_dev, (h->dim + 15) / 16, h->nnz, h->ent_t, h->L * h->k, quads};
   const size_t lds = hr_lds(h->bt_ksteps, h->bt_tiles);
   if (h->bt_ksteps <= (vec ? kHrMaxSteps : kHrMaxSteps / 2) && lds <= (size_t)kMaxDynLds) {
     using Fn = decltype(&hash_dense_resident_kernel<1, true>);
@@ -1468,8 +1509,8 @@ static int hash_matrix_launch(const kh_hash_family* h, const float* x, int64_t l
     const int ks = h->bt_ksteps;
     const Fn fn = fns[ks <= 1 ? 0 : ks <= 2 ? 1 : 2][vec ? 1 : 0];
     const int blocks = (int)std::min<int64_t>(256, (batch + 16 * kHrWaves - 1) / (16 * kHrWaves));
-    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * kHrWaves), lds, st, h->bt_dev, ks, h->bt_tiles, h->sp_dev,
-                       spn, h->k, h->L, h->dim, x, ldx, batch, codes, row_stride, table_stride);
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * kHrWaves), lds, st, h->bt_dev, ks, h->bt_tiles, planes,
+                       h->k, h->L, h->dim, x, ldx, batch, codes, row_stride, table_stride);
     KH_LAUNCHED();
     return KH_OK;
   }
@@ -1477,7 +1518,7 @@ static int hash_matrix_launch(const kh_hash_family* h, const float* x, int64_t l
     const int64_t nb = std::min<int64_t>(batch - b0, (int64_t)65535 * kHmRows);
     hipLaunchKernelGGL(vec ? hash_dense_mfma_kernel<true> : hash_dense_mfma_kernel<false>,
                        dim3((unsigned)ceil_div(nb, kHmRows)), dim3(256), 0, st, h->bt_dev, h->bt_ksteps,
-                       h->bt_tiles, h->sp_dev, spn, h->k, h->L, h->dim, x + b0 * ldx, ldx, nb,
+                       h->bt_tiles, planes, h->k, h->L, h->dim, x + b0 * ldx, ldx, nb,
                        codes + b0 * row_stride, row_stride, table_stride);
     KH_LAUNCHED();
   }

@@ -1,7 +1,8 @@
 """GPU parity: hashing of large dense batches with the planes resident in LDS (up to 128
 dimensions, planes that fit), at the edges of its tiles: k steps of 32 dimensions, 16-plane
 tiles, 16-row tiles, more rows than one pass of the grid, rows of inf / NaN, a queue of
-undecided signs that overflows.  Bar: bit-exact codes."""
+undecided signs that overflows; and of wider batches, whose planes are read again, with rows
+that allow whole pieces, none, and too many values for either.  Bar: bit-exact codes."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +12,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dim,k,L,batch", [
     (1, 1, 1, 1024), (31, 3, 7, 1025), (32, 24, 3, 1030), (33, 9, 50, 1040), (64, 5, 13, 1999), (96, 6, 50, 1500),
-    (100, 7, 37, 1100), (127, 9, 50, 1031), (128, 9, 50, 70001), (128, 1, 17, 1024)])
+    (100, 7, 37, 1100), (127, 9, 50, 1031), (128, 9, 50, 70001), (128, 1, 17, 1024),
+    (4, 9, 50, 1025), (36, 9, 50, 1300), (65, 9, 50, 1100), (130, 5, 20, 1040), (204, 5, 20, 1040), (512, 4, 11, 1030),
+    (511, 4, 11, 1030), (513, 4, 11, 1030), (2001, 2, 9, 1025)])
 def test_resident_codes(kh, orc, dim, k, L, batch):
     from klearu_amd.lsh import HashFamily
     rng = np.random.default_rng(dim * 100 + k)
