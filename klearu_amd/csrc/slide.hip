@@ -451,7 +451,6 @@ __global__ __launch_bounds__(kSlideThreads) void neuron_kernel(
   const int64_t row = blockIdx.x;
   bool all;
   const int n = vanilla_len(alen, row, fb_n, all);
-  if (blockIdx.y && (int)(blockIdx.y * blockDim.x) >= n) return;   // no neurons: block 0 has the row's offset
   csr_part(co, alen, row, fb_n, part);
   const bool fit = TRANS && offsets_fit(dim, nn);
   const uint32_t mul = fit ? (uint32_t)nn : 1u;   // of the indices in LDS
