@@ -410,12 +410,14 @@ __device__ __forceinline__ float hm_bound(float sum_abs, int ksteps, int dim) {
 // instructions per sum: a sign costs a compare into a lane mask and its share of one
 // margin test for kHrGroup plane tiles; the undecided ones (about 7 in 10000) queue
 // per wave and are replayed in its lanes, which set or clear their bit.
-// 200003 rows: 113 us, 224 before.
+// 200003 rows: 113 us, 224 before.  Tiles go to the blocks in turn, so that a short batch does
+// not fill a few CUs and leave the rest: 1024 rows of 33 dimensions, 300 planes 10.8 us, 17.8 in
+// four blocks (rows of zeros and ones, which replay the most, 58 and 236).
 constexpr int kHrWaves = 16;
 constexpr int kHrGroup = 4;      // plane tiles in flight per wave
 constexpr int kHrQueue = 512;    // queued replays per wave; emptied when over kHrFull
 constexpr int kHrFull = kHrQueue - 256;   // a plane tile adds at most 256
-constexpr int kHrMaxSteps = 4;   // k steps whose A operands fit 128 registers (unaligned rows: half)
+constexpr int kHrMaxSteps = 4;   // k steps: the kernel then takes 127 of the 128 registers a thread of 1024 has (unaligned: 2)
 constexpr int kHrBatch = 2;      // sign words in flight per replay
 // Words of plane bits per row: 32 planes each, and one to read past the last.
 __host__ __device__ constexpr int hr_words(int ntiles) { return (ntiles + 1) / 2 + 1; }
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(64 * kHrWaves) void hash_dense_resident_kernel(
   const int P = L * k;
   const int kq = (lane >> 4) * 8;
   const int64_t tiles = (batch + 15) / 16, step = (int64_t)gridDim.x * kHrWaves;
-  for (int64_t tile = (int64_t)blockIdx.x * kHrWaves + wave; tile < tiles; tile += step) {
+  for (int64_t tile = (int64_t)wave * gridDim.x + blockIdx.x; tile < tiles; tile += step) {   // few tiles: all CUs
     const int64_t r0 = tile * 16;
     uint4 hi[KS], lo[KS];
     float ax = 0.0f;
@@ -1508,7 +1510,7 @@ static int hash_matrix_launch(const kh_hash_family* h, const float* x, int64_t l
     KH_HIP(attr_rc);
     const int ks = h->bt_ksteps;
     const Fn fn = fns[ks <= 1 ? 0 : ks <= 2 ? 1 : 2][vec ? 1 : 0];
-    const int blocks = (int)std::min<int64_t>(256, (batch + 16 * kHrWaves - 1) / (16 * kHrWaves));
+    const int blocks = (int)std::min<int64_t>(256, (batch + 15) / 16);
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * kHrWaves), lds, st, h->bt_dev, ks, h->bt_tiles, planes,
                        h->k, h->L, h->dim, x, ldx, batch, codes, row_stride, table_stride);
     KH_LAUNCHED();

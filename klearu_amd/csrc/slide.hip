@@ -896,19 +896,19 @@ static int slide_forward_common(const kh_slide_layer* lc, const float* x, const 
                        pre, post, fb_n, olen, co);
   else if (l->wtn)
     hipLaunchKernelGGL((wide ? neuron_kernel<false, true, kRowLoads> : neuron_kernel<false, true, 1>), ng,
-                       dim3(kSlideThreads), lds, st, l->wtn, l->n, l->bias, l->dim, x, nullptr, nullptr, nullptr, aids, as, ilen, act,
-                       max_nz, pre, post, fb_n, olen, co);
+                       dim3(kSlideThreads), lds, st, l->wtn, l->n, l->bias, l->dim, x, nullptr, nullptr, nullptr, aids,
+                       as, ilen, act, max_nz, pre, post, fb_n, olen, co);
   else if (l->dim <= kTileMaxDim && l->dim % 4 == 0 && tile_kernel_ready() == KH_OK) {
     // Eight waves are a block per CU. Rows without a tile for each take the four that the
-    // softmax needs, two blocks to a CU: 5000 rows of 20 neurons 163 -> 103 us, of 160 171 -> 111.
+    // softmax needs, two blocks to a CU: 5000 rows of 20 neurons 94 us, 163 with eight.
     const int waves = ceil_div(as, kTileN) < kTileWaves ? kSlideThreads / 64 : kTileWaves;
     hipLaunchKernelGGL(neuron_tile_kernel, dim3((unsigned)batch), dim3(64 * waves), tile_lds(waves), st, l->w, l->bias,
                        l->dim, x, aids, as, ilen, act, pre, post, fb_n, olen, nullptr, 0, co);
   }
   else
     hipLaunchKernelGGL((wide ? neuron_kernel<false, false, kRowLoads> : neuron_kernel<false, false, 1>), ng,
-                       dim3(kSlideThreads), lds, st, l->w, l->n, l->bias, l->dim, x, nullptr, nullptr, nullptr, aids, as, ilen, act,
-                       max_nz, pre, post, fb_n, olen, co);
+                       dim3(kSlideThreads), lds, st, l->w, l->n, l->bias, l->dim, x, nullptr, nullptr, nullptr, aids,
+                       as, ilen, act, max_nz, pre, post, fb_n, olen, co);
   KH_LAUNCHED();
   if (packed) return csr_check(off, batch, as, capacity, st);
   return csr_finish(aids, nullptr, pre, post, as, alen, batch, off, act_ids, nullptr, pre_out,
