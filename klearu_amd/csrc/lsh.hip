@@ -981,7 +981,8 @@ __global__ __launch_bounds__(kBpThreads) void bucket_count_kernel(const uint32_t
 // Reservoir: base = the length before, before = the insertion count before.
 __global__ void bucket_scan_kernel(uint32_t* __restrict__ hist, int chunks, int buckets, int cap, int reservoir,
                                    uint32_t* __restrict__ len, uint64_t* __restrict__ count,
-                                   int32_t* __restrict__ base, uint64_t* __restrict__ before) {
+                                   uint32_t* __restrict__ old_len, int32_t* __restrict__ base,
+                                   uint64_t* __restrict__ before) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= buckets) return;
   uint32_t m = 0;
@@ -1004,6 +1005,7 @@ __global__ void bucket_scan_kernel(uint32_t* __restrict__ hist, int chunks, int 
     len[q] = min((uint32_t)cap, l + m);
   } else {
     const uint32_t total = l + m, keep = min(total, (uint32_t)cap);
+    old_len[q] = l;
     base[q] = (int32_t)l - (int32_t)(total - keep);
     len[q] = keep;
   }
@@ -1989,10 +1991,13 @@ int max_id_begin(kh_lsh_index* idx, const uint32_t* ids_dev, int64_t n, hipStrea
   const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, 256), 256);
   uint32_t* part = cb.get<uint32_t>(blocks);
   if (!part) return KH_ERR_ALLOC;
-  hipLaunchKernelGGL(max_id_kernel, dim3(blocks), dim3(256), 0, st, ids_dev, n, part);
+  // one block's result is the call's (a second launch costs a short call 20 us of its 60)
+  hipLaunchKernelGGL(max_id_kernel, dim3(blocks), dim3(256), 0, st, ids_dev, n, blocks > 1 ? part : idx->mx_host);
   KH_LAUNCHED();
-  hipLaunchKernelGGL(max_id_kernel, dim3(1), dim3(256), 0, st, part, (int64_t)blocks, idx->mx_host);
-  KH_LAUNCHED();
+  if (blocks > 1) {
+    hipLaunchKernelGGL(max_id_kernel, dim3(1), dim3(256), 0, st, part, (int64_t)blocks, idx->mx_host);
+    KH_LAUNCHED();
+  }
   KH_HIP(hipEventRecord(idx->mx_done, st));
   return KH_OK;
 }
@@ -2078,12 +2083,22 @@ static int insert_sorted(kh_lsh_index* idx, const uint32_t* ids_dev, const uint3
   return KH_OK;
 }
 
+// Few vectors into many buckets: placing by rank passes over every bucket, sorting over the
+// vectors. FIFO, us, sorted / placed: 524288 buckets, 1 vector 67 / 165, 128 103 / 169, 500 170 /
+// 200; 204800 buckets, 64 vectors 79 / 95, 256 100 / 98; 102400, 4 69 / 71, 64 76 / 71; 65536, 1 69 / 63.
+// A reservoir's passes over its slots stay: 524288, 1 117 / 137, 64 143 / 142; 204800, 4 86 / 88, 16
+// 96 / 88.
+static bool insert_few(const kh_lsh_index* idx, int64_t n) {
+  const int64_t buckets = (int64_t)idx->L * idx->nb;
+  return idx->type == KH_BUCKET_RESERVOIR ? n <= (buckets - 131072) / 30000 : n <= (buckets - 65536) / 900;
+}
+
 // Applies n inserts with codes[i * rs + t * ts], after max_id_begin; synchronises.
 static int insert_finish(kh_lsh_index* idx, const uint32_t* ids_dev, const uint32_t* codes, int64_t rs, int64_t ts,
                          int64_t n, hipStream_t st, CallBufs& cb) {
   uint32_t mx = 0;
   int rc;
-  if (idx->k > kBpMaxBits) {
+  if (idx->k > kBpMaxBits || (rs == idx->L && insert_few(idx, n))) {
     rc = max_id_end(idx, &mx);  // before anything is inserted
     if (rc == KH_OK) rc = insert_sorted(idx, ids_dev, codes, n, st, cb);
     if (rc != KH_OK) return rc;
@@ -2113,11 +2128,10 @@ static int insert_finish(kh_lsh_index* idx, const uint32_t* ids_dev, const uint3
                        per_wave, idx->k, hist);
     KH_LAUNCHED();
     if (reservoir) KH_HIP(hipMemsetAsync(last, 0, sizeof(*last) * nslots, st));
-    if (held) KH_HIP(hipMemcpyAsync(old_len, idx->len, sizeof(uint32_t) * nbk, hipMemcpyDeviceToDevice, st));
     rc = max_id_end(idx, &mx);  // before anything is inserted
     if (rc != KH_OK) return rc;
     hipLaunchKernelGGL(bucket_scan_kernel, dim3(ceil_div(nbk, 256)), dim3(256), 0, st, hist, chunks, nbk, idx->cap,
-                       reservoir, idx->len, idx->count, base, before);
+                       reservoir, idx->len, idx->count, old_len, base, before);
     KH_LAUNCHED();
     if (held) {
       hipLaunchKernelGGL(fifo_shift_kernel, dim3((unsigned)nbk), dim3(64), 0, st, idx->cap, old_len, base, idx->data);

@@ -1,6 +1,6 @@
 """Inserts by rank against the oracle's replay of each bucket, bit for bit: sizes around
 a wave (64), a block's chunk (4096), the transposing of row-major codes (512) and the
-tables too large to count (12 bits, sorted); skewed codes, so that buckets overflow
+tables too large to count (12 bits, sorted) and few inserts into many buckets (sorted); skewed codes, so that buckets overflow
 within one chunk; a second call into buckets that hold entries, with fewer and with more
 inserts than they keep."""
 import numpy as np
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("bt", [FIFO, RESERVOIR])
 @pytest.mark.parametrize("k,L,cap,n1,n2", [(1, 1, 1, 1, 1), (3, 2, 6, 64, 65), (6, 33, 128, 511, 513),
                                            (9, 5, 7, 4095, 4097), (11, 3, 16, 12345, 700), (11, 70, 4, 1, 4096),
-                                           (12, 2, 8, 5000, 900)])
+                                           (12, 2, 8, 5000, 900), (6, 10, 16, 256, 257), (11, 256, 4, 509, 510)])
 def test_inserts_by_rank_match_the_replay(kh, orc, bt, k, L, cap, n1, n2):
     from klearu_amd.lsh import LshIndex, SimHash
     rng = np.random.default_rng(k * 100 + n1)
