@@ -585,7 +585,7 @@ extern "C" int kh_dejavu_linear_create(int in_features, int out_features, const 
     hipLaunchKernelGGL(transpose_kernel<float>, dim3(ceil_div(in_features, 32), ceil_div(out_features, 32)),
                        dim3(256), 0, 0, l->w, out_features, in_features, l->wt);
     e = hipGetLastError();
-    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // other streams go on
   }
   if (e != hipSuccess) {
     set_error("linear upload failed: %s", hipGetErrorString(e));

@@ -78,3 +78,21 @@ def test_index_list_in_the_launch_and_copied(kh, orc, n):
     idx = rng.integers(0, 500, n)
     y = Linear(w, b).forward_sparse(x, idx).cpu().numpy()
     np.testing.assert_array_equal(bits(y), bits(orc.dejavu_linear_forward(w, b, x)[idx]))
+
+
+def test_creating_a_linear_leaves_other_streams_running(kh):
+    """The upload is waited for on its own stream; work queued on another goes on meanwhile."""
+    from klearu_amd.dejavu_transformer import Linear
+    side = torch.cuda.Stream()
+    a = torch.randn(4096, 4096, device="cuda")
+    Linear(np.ones((64, 64), np.float32))
+    torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    with torch.cuda.stream(side):
+        for _ in range(200):
+            a = torch.tanh(a @ a)
+        done.record()
+    lin = Linear(np.ones((64, 64), np.float32))
+    assert not done.query()
+    torch.cuda.synchronize()
+    assert float(lin.forward(np.ones(64, np.float32))[3]) == 64.0
