@@ -81,8 +81,6 @@ __device__ __forceinline__ void widen16(const uint4& v, float* f, float) {
   f[0] = __uint_as_float(v.x); f[1] = __uint_as_float(v.y);
   f[2] = __uint_as_float(v.z); f[3] = __uint_as_float(v.w);
 }
-__device__ __forceinline__ void store_kv(uint16_t* p, float v) { *p = f32_to_bf16(v); }
-__device__ __forceinline__ void store_kv(float* p, float v) { *p = v; }
 
 // The union of selected heads in ascending order -> rows h*D + r of WoT
 // (qrows, their count in *nqrows) and each head's union rank (urank, -1 for

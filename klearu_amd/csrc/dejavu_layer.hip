@@ -399,10 +399,6 @@ __global__ __launch_bounds__(64) void dl_head_score_kernel(
   for (int d = lane; d < head_dim; d += 64) att[st + d] = __fmul_rn(v[st + d], sc);
 }
 
-static unsigned grid_for(int64_t threads) {
-  return (unsigned)((threads + kDlThreads - 1) / kDlThreads);
-}
-
 // Lists of up to kDlArgList indices travel in the launch itself: the caller's
 // list may be freed on return and nothing waits, where a copy from pageable host
 // memory made every call wait for its stream (SparseMlp with 822 neurons, then

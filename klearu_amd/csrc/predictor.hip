@@ -181,7 +181,8 @@ __global__ __launch_bounds__(kL1LdsThreads) void pred_l1_lds_kernel(
 //    of the other three SIMDs, so no producer takes issue slots from the chain; the
 //    wave that shares the consumer's SIMD only stages x.  A stage costs its producer
 //    two LDS round trips and the write's wait: three producers just kept pace and held
-//    the chain up (16 rows of 4096 x 256: the call took 1.7 us more).
+//    the chain up (layers 1 and 2, 512 to 4096 inputs, 160 to 256 outputs, 9 to 16 rows: 0.5 to
+//    0.8 us of 11 to 24 more; 16 rows of 4096 x 256 24.2 us, 23.4 with six).
 //  * Quad q of chain c sits at position c ^ (q & 14) of its ring row: the
 //    consumer's 16 lanes still read one contiguous row, and a producer's
 //    write instruction (8 quads x 8 chains) spreads evenly over the banks

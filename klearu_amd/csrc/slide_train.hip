@@ -1158,8 +1158,7 @@ static int net_train_step(kh_slide_network* net, const float* x_dev, const int64
                  (long long)e, kTrMaxLabels);
   const int64_t n_labels = label_off_host[batch];
   KH_CHECK_ARG(n_labels == 0 || labels_host, "null labels");
-  int rc = net_setup_attrs();
-  if (rc != KH_OK) return rc;
+  int rc = KH_OK;
   hipStream_t st = as_stream(stream);
   if (xoff) {
     rc = net_check_csr(xoff, batch, st);
