@@ -140,6 +140,26 @@ def test_hash_sparse_matches_dense(kh, orc):
     assert fam.hash_sparse(SparseVector([], [], 2000), 0) == (1 << 9) - 1
 
 
+@pytest.mark.parametrize("nnz,at", [(1, 0), (40, 7), (512, 511), (513, 512), (1200, 3), (1200, 1100)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_hash_sparse_values_that_are_not_finite(kh, orc, nnz, at, bad):
+    """An entry without a coefficient adds nothing, whatever its value; entries past the last
+    dimension are passed over; chunks are of 512 entries."""
+    from klearu_amd.lsh import HashFamily, SparseVector
+    rng = np.random.default_rng(nnz + at)
+    planes = rng.choice(np.array([-1, 0, 0, 1], np.int8), (7, 9, 1500))
+    fam = HashFamily.from_planes(planes)
+    idx = np.sort(rng.choice(1500, nnz, replace=False)).astype(np.uint32)
+    val = rng.standard_normal(nnz).astype(np.float32)
+    val[at] = bad
+    want = [orc.hash_sparse(planes, idx, val, t) for t in range(7)]
+    past_i, past_v = np.insert(idx, [0, at + 1], [1500, 2**32 - 1]), np.insert(val, [0, at + 1], [5.0, np.nan])
+    got = fam.hash_sparse_batch([SparseVector(idx, val, 1500), SparseVector(past_i, past_v, 2**32)])
+    got = got.cpu().numpy().view(np.uint32)
+    np.testing.assert_array_equal(got[0], want)
+    np.testing.assert_array_equal(got[1], want)
+
+
 def test_family_from_planes_and_errors(kh, orc):
     from klearu_amd._lib import KlearuError
     from klearu_amd.lsh import HashFamily, SimHash

@@ -1,6 +1,6 @@
 """Training steps through a wave per neuron, bit for bit against the oracle: rows with 1,
 63..65, 255..257 and all nonzeros, layers of 130 to 2000 inputs (row-major, not the
-64-neuron tiles), one to seventy neurons."""
+32-neuron tiles), one to seventy neurons."""
 import numpy as np
 import pytest
 

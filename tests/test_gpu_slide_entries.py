@@ -1,7 +1,7 @@
 """SLIDE forward, bit for bit against the oracle, at the edges of its entry lists: rows
 with 0, 1 and around 16, 32 and all dimensions nonzero; dimensions around a load of a
-block (256) and of four (1024), the 64-neuron tiles (dimensions up to 128, a multiple
-of 4) and the largest dense input; row-major and transposed weights (act); sparse
+block (256) and of four (1024), the 32-neuron tiles (dimensions up to 128, a multiple
+of 4; fewer than one, of four waves and of eight) and the largest dense input; row-major and transposed weights (act); sparse
 inputs longer than the list kept on chip (4096)."""
 import numpy as np
 import pytest
@@ -19,7 +19,8 @@ def rows_of(rng, dim):
     return X
 
 
-@pytest.mark.parametrize("dim,n", [(1, 70), (4, 64), (5, 300), (100, 65), (127, 129), (128, 1000), (255, 63), (256, 64),
+@pytest.mark.parametrize("dim,n", [(4, 1), (128, 31), (100, 32), (64, 33), (128, 129), (128, 224), (60, 225), (128, 257),
+                                   (1, 70), (4, 64), (5, 300), (100, 65), (127, 129), (128, 1000), (255, 63), (256, 64),
                                    (257, 600), (1023, 300), (1024, 257), (1025, 100), (8191, 40), (8192, 40)])
 @pytest.mark.parametrize("act", ["Relu", "Softmax"])
 def test_forward_over_entry_counts(kh, orc, dim, n, act):
