@@ -1988,10 +1988,11 @@ int max_id_begin(kh_lsh_index* idx, const uint32_t* ids_dev, int64_t n, hipStrea
     idx->mx_host = static_cast<uint32_t*>(p);
   }
   if (!idx->mx_done) KH_HIP(hipEventCreateWithFlags(&idx->mx_done, hipEventDisableTiming));
-  const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, 256), 256);
+  // up to 2048 ids: one block, whose result is the call's (a second launch costs a short call
+  // 20 us of its 60; eight ids a thread about 2)
+  const unsigned blocks = n <= 2048 ? 1u : (unsigned)std::min<int64_t>(ceil_div(n, 256), 256);
   uint32_t* part = cb.get<uint32_t>(blocks);
   if (!part) return KH_ERR_ALLOC;
-  // one block's result is the call's (a second launch costs a short call 20 us of its 60)
   hipLaunchKernelGGL(max_id_kernel, dim3(blocks), dim3(256), 0, st, ids_dev, n, blocks > 1 ? part : idx->mx_host);
   KH_LAUNCHED();
   if (blocks > 1) {

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("bt", [FIFO, RESERVOIR])
 @pytest.mark.parametrize("k,L,cap,n1,n2", [(1, 1, 1, 1, 1), (3, 2, 6, 64, 65), (6, 33, 128, 511, 513),
                                            (9, 5, 7, 4095, 4097), (11, 3, 16, 12345, 700), (11, 70, 4, 1, 4096),
-                                           (12, 2, 8, 5000, 900), (6, 10, 16, 256, 257), (11, 256, 4, 509, 510)])
+                                           (12, 2, 8, 5000, 900), (6, 10, 16, 256, 257), (5, 4, 16, 2048, 2049), (11, 256, 4, 509, 510)])
 def test_inserts_by_rank_match_the_replay(kh, orc, bt, k, L, cap, n1, n2):
     from klearu_amd.lsh import LshIndex, SimHash
     rng = np.random.default_rng(k * 100 + n1)
