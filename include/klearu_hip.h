@@ -538,7 +538,8 @@ int kh_dejavu_mlp_block_batch(const kh_predictor* p, const kh_sparse_ffn* f, flo
 
 typedef struct kh_dejavu_linear kh_dejavu_linear;
 
-/* Linear{weight [out][in], bias [out]} (transformer/mod.rs:79-111) from host arrays. */
+/* Linear{weight [out][in], bias [out]} (transformer/mod.rs:79-111) from host arrays.
+ * Keeps the weights twice on the device, row-major and transposed. */
 int kh_dejavu_linear_create(int in_features, int out_features, const float* w_host,
                             const float* b_host, kh_dejavu_linear** out);
 int kh_dejavu_linear_destroy(kh_dejavu_linear* l);

@@ -27,8 +27,8 @@
 // (count, id), gives each insert a slot and each slot its last insert.  So the
 // build counts the buckets of every chunk of vectors, sums the counts over the
 // chunks, and places each vector by its rank, with no sort.  (Tables of more than
-// 2^11 buckets, and removals, sort the (bucket, position) pairs with a stable radix
-// sort and apply each bucket's run.)  Buckets are dense
+// 2^11 buckets, few vectors into many buckets, and removals sort the (bucket,
+// position) pairs with a stable radix sort and apply each bucket's run.)  Buckets are dense
 // [L][2^k][cap] u32 with len[L][2^k] and the reservoir insertion count[L][2^k].
 //
 // Query.  One block per input gathers its L buckets.  When ids are below
@@ -2057,7 +2057,8 @@ int group_by_bucket(const kh_lsh_index* idx, const uint32_t* codes_dev, int64_t 
 
 }  // namespace
 
-// Inserts by sorted runs, for tables of more buckets than bucket_place_kernel counts.
+// Inserts by sorted runs, for tables of more buckets than bucket_place_kernel counts and
+// for the calls of insert_few.
 static int insert_sorted(kh_lsh_index* idx, const uint32_t* ids_dev, const uint32_t* codes_dev, int64_t n,
                          hipStream_t st, CallBufs& cb) {
   Groups g;
